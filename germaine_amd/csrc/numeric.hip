@@ -1461,8 +1461,24 @@ __global__ void __launch_bounds__(256) k_diag_inv(cx<T> *__restrict__ arena, int
 // ---------------------------------------------------------------------------
 namespace {
 size_t g_panel_lds_cap = 0;   // 0: the hardware limit
-int g_persistent = 1;         // small subtrees in one persistent launch
-int g_deep_min_m = 0;         // blocked levels with a front of order >= this take the two-panel schedule
+// Until a caller selects otherwise (g_deep_min_m < 0): the small fronts level by
+// level, and two panels per step only where the trailing update is bound by
+// its passes over memory.  The persistent subtree launch is a serial chain of
+// fronts per workgroup: 61x41, one FP64 frequency, 0.91 ms per factorisation
+// against 0.52 level by level; 1601x401, four frequencies, 43.0 against 42.3.
+// Two panels per step trade a pass over the trailing block for three more
+// launches and a 64-row triangular solve: 270x145 2.46 ms against 2.30, 1601x401
+// (four frequencies) 42.3 against 38.6 in FP64 and 24.7 against 24.4 in FP32;
+// they pay in FP32 from fronts of order 384 once the level's tiles fill the
+// device several times over (1601x401, eight frequencies: 43.2 against 43.9).
+int g_persistent = 0;    // small subtrees in one persistent launch
+int g_deep_min_m = -1;   // blocked levels with a front of order >= this take the two-panel schedule
+constexpr int kDeepFp32M = 384, kDeepFp32Tiles = 6 * 256;
+template <typename T>
+bool deep_level(const LevelPlan &L, const DevPlan::DeepStep &first, int nf) {
+    if (g_deep_min_m >= 0) return L.large_mmax >= g_deep_min_m;
+    return sizeof(T) == 4 && L.large_mmax >= kDeepFp32M && (int64_t)first.deep_cnt * nf >= kDeepFp32Tiles;
+}
 }
 void set_factor_tuning(int panel_lds_cap, int persistent, int deep_min_m) {
     g_panel_lds_cap = panel_lds_cap > 0 ? (size_t)panel_lds_cap : 0;
@@ -1586,7 +1602,7 @@ void factor_numeric(const DevPlan &dp, Factors<T> &F, const cx<double> *vals, in
                     hipLaunchKernelGGL((k_gemm_update<T, false>), dim3(cnt, nf), dim3(256), 0, st, F.arena,
                                        F.fstride, dp.fronts, dp.lv_large[l], dp.tiles + off, k0, depth, ccap);
             };
-            if (L.large_mmax >= g_deep_min_m) {
+            if (deep_level<T>(L, dp.deep_steps[l][0], nf)) {
                 // two panels per block: panel 1; its U rows and update on panel 2's
                 // columns only; panel 2; the U rows of both panels (one 64-row
                 // solve) and one depth-64 trailing update, so the trailing block

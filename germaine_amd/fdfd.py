@@ -106,7 +106,8 @@ def factor_tuning(panel_lds_cap=0, persistent=1, deep_min_m=0):
     hardware limit); persistent selects the one-launch factorisation of the
     small subtrees (else level by level); levels whose largest blocked front
     has order >= deep_min_m take the two-panel schedule (trailing update once
-    per 64 pivots), the others one panel at a time (NO_DEEP: none)."""
+    per 64 pivots), the others one panel at a time (NO_DEEP: none).  Until the
+    first call: level by level, and a schedule by the level's size and precision."""
     check(lib().gfdfd_factor_tuning(int(panel_lds_cap), int(persistent), int(deep_min_m)), "gfdfd_factor_tuning")
 
 

@@ -184,12 +184,14 @@ int gfdfd_solve_tuning(int rw_cap, int fused_mmax, int refine_layout);
  * panel_lds_cap bytes of LDS is factored by the global-memory panel kernel
  * instead of in LDS (0: the hardware limit, 159 KB -- separators above 318
  * rows in FP64, 637 in FP32), which lets small systems exercise that path;
- * persistent != 0 (the default) factors the small subtrees -- fronts of order
+ * persistent != 0 factors the small subtrees -- fronts of order
  * <= 64 whose descendants are all that small -- in one persistent launch in
  * which a workgroup factors one whole subtree of one frequency per task, 0
  * level by level; levels whose largest blocked front has order >= deep_min_m
- * (default 0: every level) factor two 32-column panels per step and update
- * the trailing block once per 64 pivots, the others once per panel.        */
+ * factor two 32-column panels per step and update the trailing block once
+ * per 64 pivots (0: every level), the others once per panel.  Until the first
+ * call the small fronts go level by level and the schedule follows the
+ * level's size and precision.                                               */
 int gfdfd_factor_tuning(int panel_lds_cap, int persistent, int deep_min_m);
 
 /* ---- shot kernels --------------------------------------------------------------
