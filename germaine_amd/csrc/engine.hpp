@@ -23,7 +23,6 @@ struct DevPlan {
     std::shared_ptr<const Plan> host;
     FrontDev *fronts = nullptr;
     int *children = nullptr, *idx = nullptr, *inv = nullptr, *perm = nullptr, *iperm = nullptr;
-    int64_t *orig_q = nullptr, *orig_dst = nullptr;
     int *colptr = nullptr, *rowind = nullptr;
     int64_t *tq = nullptr;                 // CSR-of-M position -> CSC index (symmetric pattern)
     std::vector<int *> lv_small, lv_large, lv_all;
@@ -73,27 +72,31 @@ struct DevPlan {
     std::vector<FrontDev *> lv_fr;                  // per level: the level's fronts, contiguous
     std::vector<int> lv_children;                   // per level: 1 if any front has children
 
-    // Small subtrees (fronts whose whole subtree has m <= small_max), factored
-    // by one persistent launch: a task is one maximal such subtree (a
+    // Small fronts (order <= small_max), each assembled and factored by one
+    // workgroup: a slot per front with its original entries.
+    int *slot_of = nullptr;                         // [nfronts] small-front slot, -1 for blocked fronts
+    int64_t *small_optr = nullptr;                  // [slots + 1] ranges of the slots' original entries
+    int64_t *small_oq = nullptr;                    // CSC index of each such entry
+    int *small_ooff = nullptr;                      // its local offset r + c m in the front
+    // the blocked fronts' original entries, by level
+    int64_t *orig_q_large = nullptr, *orig_dst_large = nullptr;
+    std::vector<std::pair<int64_t, int64_t>> orig_large_range;   // per level [begin, end)
+    std::vector<double> asm_elems_large;            // per level: entries of the blocked fronts
+
+    // Small subtrees (fronts whose whole subtree has m <= small_max), which one
+    // persistent launch can factor: a task is one maximal such subtree (a
     // contiguous postorder range of fronts) for one frequency, taken from a
     // global counter by a workgroup that factors its fronts leaves to root.
-    // The level path takes the remaining fronts.
-    int nsub = 0, nroots = 0, sub_mmax = 0;
+    // The level path then takes the remaining small fronts.
+    int nroots = 0, sub_mmax = 0;
     int *root_first = nullptr, *root_last = nullptr;   // [nroots] front range of each subtree
-    int *slot_of = nullptr;                         // [nfronts] subtree-front slot, -1 outside the subtrees
-    int64_t *sub_optr = nullptr;                    // [nsub + 1] ranges of the slots' original entries
-    int64_t *sub_oq = nullptr;                      // CSC index of each such entry
-    int *sub_ooff = nullptr;                        // its local offset r + c m in the front
     double sub_flops = 0, sub_elems = 0;            // algorithmic counts of the launch (per frequency)
-    std::vector<int *> lv_asm_rest, lv_small_rest;  // per level: fronts outside the subtrees
-    std::vector<int> n_asm_rest, n_small_rest, mmax_asm_rest, small_mmax_rest;
-    int64_t *orig_q_rest = nullptr, *orig_dst_rest = nullptr;
-    std::vector<std::pair<int64_t, int64_t>> orig_rest_range;   // per level [begin, end)
-    std::vector<double> asm_rest_elems;             // per level: entries the level path assembles
-    std::vector<double> small_rest_flops, small_rest_elems;   // per level: the level path's small fronts
+    std::vector<int *> lv_small_rest;               // per level: small fronts outside the subtrees
+    std::vector<int> n_small_rest, small_mmax_rest;
+    std::vector<double> small_rest_flops, small_rest_elems;   // per level: those fronts
 
     explicit DevPlan(std::shared_ptr<const Plan> p);
-    void build_subtrees(const Plan &pl);
+    void build_small(const Plan &pl);
     ~DevPlan();
     DevPlan(const DevPlan &) = delete;
     DevPlan &operator=(const DevPlan &) = delete;

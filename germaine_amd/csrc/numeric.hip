@@ -16,6 +16,7 @@
 // Factors stay in place in the front arena (L11\U11 and L21 in the first p
 // columns, U12 in the first p rows); the pivot swaps go to piv[pos0 + j].
 #include <algorithm>
+#include <utility>
 
 #include "engine.hpp"
 #include "mfma.hpp"
@@ -27,42 +28,52 @@ namespace gfdfd {
 // ---------------------------------------------------------------------------
 // DevPlan
 // ---------------------------------------------------------------------------
-// Small subtrees: a front belongs when its order is at most the plan's
-// small_max and all its children belong (leaves included), so a whole subtree
-// is factored by the persistent launch and the level path never waits on it.
+// Small fronts (order <= the plan's small_max) are assembled and factored in
+// one kernel each, so every small front gets a slot with its own list of
+// original entries; the blocked fronts' entries are listed by level.
+// Small subtrees: a front belongs when its order is at most small_max and all
+// its children belong (leaves included), so a whole subtree can be factored
+// by the persistent launch and the level path never waits on it.
 // Fronts are in postorder, so each maximal subtree is a contiguous range
 // ending at its root.
-void DevPlan::build_subtrees(const Plan &pl) {
+void DevPlan::build_small(const Plan &pl) {
     const int nfr = (int)pl.fronts.size();
-    std::vector<char> in(nfr, 0);
+    std::vector<char> in(nfr, 0), small(nfr, 0);
+    for (const LevelPlan &L : pl.levels)
+        for (int f : L.small) small[f] = 1;
     for (int f = 0; f < nfr; f++) {   // postorder: children first
         const Front &F = pl.fronts[f];
-        bool ok = pl.grid && F.m <= pl.small_max && F.m <= kSubMaxM && F.nchild <= kAsmMaxChildren;
+        bool ok = pl.grid && small[f] && F.m <= kSubMaxM && F.nchild <= kAsmMaxChildren;
         for (int c = 0; c < F.nchild && ok; c++) ok = in[pl.children[F.child_off + c]] != 0;
         in[f] = ok;
     }
-    std::vector<int> list, slot(nfr, -1), first, last, lo(nfr);
-    for (int f = 0; f < nfr; f++) {   // first (lowest) front of f's subtree
+    std::vector<int> slot(nfr, -1), first, last, lo(nfr);
+    int nslot = 0;
+    for (int f = 0; f < nfr; f++) {   // lowest front of f's subtree
         const Front &F = pl.fronts[f];
         lo[f] = f;
         for (int c = 0; c < F.nchild; c++) lo[f] = std::min(lo[f], lo[pl.children[F.child_off + c]]);
+        if (small[f]) slot[f] = nslot++;
     }
     for (int f = 0; f < nfr; f++)
         if (in[f]) {
-            slot[f] = (int)list.size();
-            list.push_back(f);
-            const int par = pl.fronts[f].parent;
-            if (par < 0 || !in[par]) {
+            const Front &F = pl.fronts[f];
+            sub_mmax = std::max(sub_mmax, F.m);
+            for (int k = 0; k < F.p; k++) {
+                const double t = F.m - k - 1;
+                sub_flops += 4.0 * (2.0 * t * t + t);
+            }
+            sub_elems += (double)F.m * F.m;
+            if (F.parent < 0 || !in[F.parent]) {
                 for (int g = lo[f]; g <= f; g++)
                     if (!in[g]) throw std::logic_error("small subtree is not a contiguous postorder range");
                 first.push_back(lo[f]);
                 last.push_back(f);
             }
         }
-    nsub = (int)list.size();
     nroots = (int)first.size();
-    // original entries: the subtrees' by slot (local offsets), the rest by level
-    std::vector<std::vector<std::pair<int64_t, int>>> per_slot(nsub);
+    // original entries: the small fronts' by slot (local offsets), the rest by level
+    std::vector<std::vector<std::pair<int64_t, int>>> per_slot(nslot);
     std::vector<std::vector<std::pair<int64_t, int64_t>>> rest(pl.nlevels);
     std::vector<std::pair<int64_t, int>> starts;   // buf_off -> front
     for (int f = 0; f < nfr; f++) starts.push_back({pl.fronts[f].buf_off, f});
@@ -77,9 +88,9 @@ void DevPlan::build_subtrees(const Plan &pl) {
         if (slot[f] >= 0) per_slot[slot[f]].push_back({pl.orig_q[e], (int)(d - F.buf_off)});
         else rest[F.level].push_back({pl.orig_q[e], d});
     }
-    std::vector<int64_t> optr(nsub + 1, 0), oq;
+    std::vector<int64_t> optr(nslot + 1, 0), oq;
     std::vector<int> ooff;
-    for (int k = 0; k < nsub; k++) {
+    for (int k = 0; k < nslot; k++) {
         for (auto &e : per_slot[k]) { oq.push_back(e.first); ooff.push_back(e.second); }
         optr[k + 1] = (int64_t)oq.size();
     }
@@ -87,58 +98,39 @@ void DevPlan::build_subtrees(const Plan &pl) {
     for (int l = 0; l < pl.nlevels; l++) {
         const int64_t b = (int64_t)rq.size();
         for (auto &e : rest[l]) { rq.push_back(e.first); rd.push_back(e.second); }
-        orig_rest_range.push_back({b, (int64_t)rq.size()});
+        orig_large_range.push_back({b, (int64_t)rq.size()});
     }
     root_first = dev_upload(first);
     root_last = dev_upload(last);
     slot_of = dev_upload(slot);
-    sub_optr = dev_upload(optr);
-    sub_oq = dev_upload(oq);
-    sub_ooff = dev_upload(ooff);
-    orig_q_rest = dev_upload(rq);
-    orig_dst_rest = dev_upload(rd);
+    small_optr = dev_upload(optr);
+    small_oq = dev_upload(oq);
+    small_ooff = dev_upload(ooff);
+    orig_q_large = dev_upload(rq);
+    orig_dst_large = dev_upload(rd);
     bytes += (2 * first.size() + slot.size() + ooff.size()) * 4 + (optr.size() + oq.size() + rq.size() + rd.size()) * 8;
-    for (int f : list) {
-        const Front &F = pl.fronts[f];
-        sub_mmax = std::max(sub_mmax, F.m);
-        for (int k = 0; k < F.p; k++) {
-            const double t = F.m - k - 1;
-            sub_flops += 4.0 * (2.0 * t * t + t);
-        }
-        sub_elems += (double)F.m * F.m;
-    }
-    // the level path's lists of the remaining fronts
     for (int l = 0; l < pl.nlevels; l++) {
         const LevelPlan &L = pl.levels[l];
-        std::vector<int> a, sm;
-        int mm = 0, smm = 0;
+        // the level's small fronts outside the subtrees
+        std::vector<int> sm;
+        int smm = 0;
         double el = 0, sfl = 0, sel = 0;
         for (int f : L.small)
-            if (slot[f] < 0) {
+            if (!in[f]) {
                 const Front &F = pl.fronts[f];
-                a.push_back(f);
                 sm.push_back(f);
-                mm = std::max(mm, F.m);
                 smm = std::max(smm, F.m);
-                el += (double)F.m * F.m;
                 sel += 2.0 * F.m * F.m;
                 for (int k = 0; k < F.p; k++) {
                     const double t = F.m - k - 1;
                     sfl += 4.0 * (2.0 * t * t + t);
                 }
             }
-        for (int f : L.large) {
-            a.push_back(f);
-            mm = std::max(mm, pl.fronts[f].m);
-            el += (double)pl.fronts[f].m * pl.fronts[f].m;
-        }
-        lv_asm_rest.push_back(dev_upload(a));
+        for (int f : L.large) el += (double)pl.fronts[f].m * pl.fronts[f].m;
         lv_small_rest.push_back(dev_upload(sm));
-        n_asm_rest.push_back((int)a.size());
         n_small_rest.push_back((int)sm.size());
-        mmax_asm_rest.push_back(mm);
         small_mmax_rest.push_back(smm);
-        asm_rest_elems.push_back(el);
+        asm_elems_large.push_back(el);
         small_rest_flops.push_back(sfl);
         small_rest_elems.push_back(sel);
     }
@@ -157,13 +149,10 @@ DevPlan::DevPlan(std::shared_ptr<const Plan> p) : host(std::move(p)) {
     inv = dev_upload(pl.inv);
     perm = dev_upload(pl.perm);
     iperm = dev_upload(pl.iperm);
-    orig_q = dev_upload(pl.orig_q);
-    orig_dst = dev_upload(pl.orig_dst);
     colptr = dev_upload(pl.colptr);
     rowind = dev_upload(pl.rowind);
     bytes += fd.size() * sizeof(FrontDev) + (pl.children.size() + pl.idx.size() + pl.inv.size() +
-                                            2 * pl.perm.size() + pl.colptr.size() + pl.rowind.size()) * 4 +
-             (pl.orig_q.size() + pl.orig_dst.size()) * 8;
+                                            2 * pl.perm.size() + pl.colptr.size() + pl.rowind.size()) * 4;
     // gather sources of every front row before pivoting, at the front's work rows:
     // [X position or -1, W row of a child's contribution or -1, a second one or -1]
     {
@@ -312,7 +301,7 @@ DevPlan::DevPlan(std::shared_ptr<const Plan> p) : host(std::move(p)) {
         vinv_list_off = dev_upload(loff);
         bytes += lst.size() * 12;
     }
-    build_subtrees(pl);
+    build_small(pl);
     counts.resize(pl.levels.size());
     for (size_t l = 0; l < pl.levels.size(); l++) {
         const LevelPlan &L = pl.levels[l];
@@ -372,15 +361,14 @@ DevPlan::DevPlan(std::shared_ptr<const Plan> p) : host(std::move(p)) {
 
 DevPlan::~DevPlan() {
     dev_free(fronts); dev_free(children); dev_free(idx); dev_free(inv); dev_free(perm); dev_free(iperm);
-    dev_free(orig_q); dev_free(orig_dst); dev_free(colptr); dev_free(rowind); dev_free(tq); dev_free(tiles);
+    dev_free(colptr); dev_free(rowind); dev_free(tq); dev_free(tiles);
     dev_free(lv_single);
     dev_free(gsrc_id);
     for (auto p : vinv_off) dev_free(p);
     dev_free(vinv_list);
     dev_free(vinv_list_off);
-    dev_free(root_first); dev_free(root_last); dev_free(slot_of); dev_free(sub_optr); dev_free(sub_oq);
-    dev_free(sub_ooff); dev_free(orig_q_rest); dev_free(orig_dst_rest);
-    for (auto p : lv_asm_rest) dev_free(p);
+    dev_free(root_first); dev_free(root_last); dev_free(slot_of); dev_free(small_optr);
+    dev_free(small_oq); dev_free(small_ooff); dev_free(orig_q_large); dev_free(orig_dst_large);
     for (auto p : lv_small_rest) dev_free(p);
     for (auto p : lv_fr) dev_free(p);
     for (auto p : lv_small) dev_free(p);
@@ -524,80 +512,218 @@ __device__ int block_argmax(T best, int bi, T *sb, int *si) {
 // ---------------------------------------------------------------------------
 // 3a: small fronts, one workgroup, front in LDS
 // ---------------------------------------------------------------------------
+// fn(0), fn(1), .. fn(N - 1) with constant indices, so that arrays indexed by
+// them stay in registers (a loop whose guard is monotone in its index can be
+// rolled again after unrolling, which puts them in scratch)
+template <typename Fn, int... I>
+__device__ __forceinline__ void static_for_seq(Fn &&fn, std::integer_sequence<int, I...>) {
+    (fn(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename Fn>
+__device__ __forceinline__ void static_for(Fn &&fn) {
+    static_for_seq(fn, std::make_integer_sequence<int, N>{});
+}
+// wave-wide maximum and minimum by DPP (row shifts, then row broadcasts): six
+// register steps where xor-shuffles take six LDS-crossbar round trips
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_i(int v) {
+    return __builtin_amdgcn_update_dpp(v, v, CTRL, ROWS, 0xF, false);
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_f(float v) {
+    return __int_as_float(dpp_i<CTRL, ROWS>(__float_as_int(v)));
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_f(double v) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    const unsigned lo = (unsigned)dpp_i<CTRL, ROWS>((int)(unsigned)b);
+    const unsigned hi = (unsigned)dpp_i<CTRL, ROWS>((int)(unsigned)(b >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+__device__ __forceinline__ float readlane_t(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ __forceinline__ double readlane_t(double d, int l) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(d);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, l);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), l);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+template <typename T>
+__device__ __forceinline__ cx<T> readlane_t(cx<T> v, int l) {
+    return {readlane_t(v.x, l), readlane_t(v.y, l)};
+}
+template <typename T>
+__device__ __forceinline__ T wave_max(T v) {
+    v = fmax(v, dpp_f<0x111, 0xF>(v));   // row_shr 1, 2, 4, 8
+    v = fmax(v, dpp_f<0x112, 0xF>(v));
+    v = fmax(v, dpp_f<0x114, 0xF>(v));
+    v = fmax(v, dpp_f<0x118, 0xF>(v));
+    v = fmax(v, dpp_f<0x142, 0xA>(v));   // row_bcast 15 into rows 1 and 3
+    v = fmax(v, dpp_f<0x143, 0xC>(v));   // row_bcast 31 into rows 2 and 3
+    return readlane_t(v, 63);
+}
+__device__ __forceinline__ int wave_min(int v) {
+    v = min(v, dpp_i<0x111, 0xF>(v));
+    v = min(v, dpp_i<0x112, 0xF>(v));
+    v = min(v, dpp_i<0x114, 0xF>(v));
+    v = min(v, dpp_i<0x118, 0xF>(v));
+    v = min(v, dpp_i<0x142, 0xA>(v));
+    v = min(v, dpp_i<0x143, 0xC>(v));
+    return __builtin_amdgcn_readlane(v, 63);
+}
+
 // Partial LU of an m x m front held column-major in LDS (p pivots, row
 // pivoting within the p fully-summed rows); the swap of step j goes to piv[j].
-// All threads of the workgroup call it (at least one wave); sp holds kLuNb
-// ints of LDS.  Blocked by kLuNb pivots: wave 0 alone factors a panel of kLuNb
-// columns -- pivot search, row swap within the panel, scaling and the rank-1
-// update of the panel's columns, lanes over rows, with no barrier (a wave's
-// LDS operations complete in order) -- then the workgroup applies the panel's
-// swaps to the other columns, forms the panel's rows of U12 by forward
-// substitution with the panel's unit lower block, and makes one trailing update
-// A22 -= L21 U12 of depth kLuNb with 2 x 2 output tiles per thread, so the
-// trailing block passes through LDS once per panel instead of once per pivot.
+// All 256 threads of the workgroup call it.  Blocked by kLuNb pivots, three
+// barriers per panel:
+//   - wave 0 factors the panel's kLuNb columns with its rows in registers (lane
+//     l holds rows l and, for NR = 2, l + 64).  Rows do not move: each lane
+//     carries the position its row has reached, so a swap is two label
+//     changes.  The pivot is found by a DPP maximum and a ballot (ties by the
+//     lowest position), its row reaches the wave by readlane, and every lane's
+//     reciprocal of its own candidate runs beside the search, so the two
+//     divisions are off the chain;
+//   - the workgroup reads each other column's panel rows and displaced rows
+//     through the panel's permutation, forms the U12 rows by forward
+//     substitution in registers and writes both back;
+//   - one trailing update A22 -= L21 U12 of depth kLuNb with 2 x 2 output tiles
+//     per thread.
 // Complex products use the explicit fused multiply-adds (cmul_f, cmsub_f): the
 // persistent subtree kernel and the level path inline this function and must
 // round alike.
 constexpr int kLuNb = 8;
-template <typename T>
-__device__ void small_lu_lds(cx<T> *S, int m, int p, int *__restrict__ piv, int *__restrict__ sing, int *sp) {
-    const int tid = threadIdx.x, bs = blockDim.x, lane = tid & 63;
+struct LuPerm {
+    int top[kLuNb];             // row (before the panel) that ends at each panel position
+    int q[kLuNb], r[kLuNb];     // positions below the panel that change, and the rows they take
+    int nd;
+};
+template <typename T, int NR>
+__device__ __forceinline__ void small_lu_lds(cx<T> *S, int m, int p, int *__restrict__ piv, int *__restrict__ sing,
+                                             LuPerm *pm) {
+    const int tid = threadIdx.x, bs = 256, lane = tid & 63;
     for (int jb = 0; jb < p; jb += kLuNb) {
-        const int je = min(p, jb + kLuNb);   // panel columns [jb, je)
+        const int je = min(p, jb + kLuNb), nb = je - jb;   // panel columns [jb, je)
         if (tid < 64) {
-            for (int j = jb; j < je; j++) {
-                // pivot: largest |.|_1 over rows [j, p), ties to the lower row
-                T best = T(-1);
-                int bi = j;
-                for (int r = j + lane; r < p; r += 64) better(best, bi, cabs1(S[r + j * m]), r);
-                for (int off = 32; off > 0; off >>= 1) {
-                    const T ob = __shfl_xor(best, off);
-                    const int oi = __shfl_xor(bi, off);
-                    better(best, bi, ob, oi);
+            cx<T> a[NR][kLuNb];
+            int pos[NR];   // position of the lane's row
+#pragma unroll
+            for (int k = 0; k < NR; k++) {
+                const int r = lane + 64 * k;
+                pos[k] = r;
+#pragma unroll
+                for (int c = 0; c < kLuNb; c++)
+                    a[k][c] = r < m && c < nb ? S[r + (jb + c) * m] : cx<T>{T(0), T(0)};
+            }
+            bool zero = false;
+#pragma unroll
+            for (int jj = 0; jj < kLuNb; jj++) if (jj < nb) {
+                const int j = jb + jj;
+                // the lane's candidate: rows at positions [j, p); a NaN counts as -1
+                T best = T(-2);
+                int bp = m;
+                cx<T> ca = a[0][jj];
+#pragma unroll
+                for (int k = 0; k < NR; k++)
+                    if (pos[k] >= j && pos[k] < p) {
+                        const T v = cabs1(a[k][jj]), w = v >= T(0) ? v : T(-1);
+                        if (w > best || (w == best && pos[k] < bp)) {
+                            best = w;
+                            bp = pos[k];
+                            ca = a[k][jj];
+                        }
+                    }
+                const cx<T> rc = crecip(ca);
+                const T mx = wave_max(best);
+                const unsigned long long tie = __ballot(best == mx);
+                int L = __ffsll((unsigned long long)tie) - 1;
+                if (tie & (tie - 1)) {
+                    const int lowest = wave_min(best == mx ? bp : m);
+                    L = __ffsll((unsigned long long)__ballot(best == mx && bp == lowest)) - 1;
                 }
-                if (lane == 0) {
-                    sp[j - jb] = bi;
-                    piv[j] = bi;
-                    if (best == T(0)) atomicOr(sing, 1);
+                const int pr = __builtin_amdgcn_readlane(bp, L);
+                zero |= mx == T(0);
+                if (lane == 0) piv[j] = pr;
+                const cx<T> d = readlane_t(rc, L);
+                cx<T> u[kLuNb];
+#pragma unroll
+                for (int c = jj + 1; c < kLuNb; c++) {
+                    if constexpr (NR == 1) {
+                        u[c] = readlane_t(a[0][c], L);
+                    } else {
+                        const bool k1 = pos[1] == bp;   // which of the lane's rows is its candidate
+                        const cx<T> w = {k1 ? a[1][c].x : a[0][c].x, k1 ? a[1][c].y : a[0][c].y};
+                        u[c] = readlane_t(w, L);
+                    }
                 }
-                // swap rows j and bi in the panel's columns
-                if (bi != j && jb + lane < je) {
-                    const int c = jb + lane;
-                    const cx<T> t = S[j + c * m];
-                    S[j + c * m] = S[bi + c * m];
-                    S[bi + c * m] = t;
-                }
-                const cx<T> d = crecip(S[j + j * m]);
-                for (int r = j + 1 + lane; r < m; r += 64) {
-                    const cx<T> l = cmul_f(S[r + j * m], d);
-                    S[r + j * m] = l;
-                    for (int c = j + 1; c < je; c++) S[r + c * m] = cmsub_f(S[r + c * m], l, S[j + c * m]);
+#pragma unroll
+                for (int k = 0; k < NR; k++) {
+                    pos[k] = pos[k] == pr ? j : pos[k] == j ? pr : pos[k];
+                    if (pos[k] > j) {
+                        const cx<T> l = cmul_f(a[k][jj], d);
+                        a[k][jj] = l;
+#pragma unroll
+                        for (int c = jj + 1; c < kLuNb; c++) a[k][c] = cmsub_f(a[k][c], l, u[c]);
+                    }
                 }
             }
+            if (zero && lane == 0) atomicOr(sing, 1);
+            int base = 0;
+#pragma unroll
+            for (int k = 0; k < NR; k++) {
+                const int r = lane + 64 * k;
+                const bool in = r >= jb && r < m;
+                if (in) {
+#pragma unroll
+                    for (int c = 0; c < kLuNb; c++)
+                        if (c < nb) S[pos[k] + (jb + c) * m] = a[k][c];
+                    if (pos[k] < je) pm->top[pos[k] - jb] = r;
+                }
+                const bool moved = in && pos[k] >= je && pos[k] != r;
+                const unsigned long long mv = __ballot(moved);
+                if (moved) {
+                    const int at = base + __popcll(mv & ((1ull << lane) - 1));
+                    pm->q[at] = pos[k];
+                    pm->r[at] = r;
+                }
+                base += __popcll(mv);
+            }
+            if (lane == 0) pm->nd = base;
         }
         __syncthreads();
-        // the panel's swaps, in order, on the columns outside it
-        for (int c = tid; c < m; c += bs) {
-            if (c >= jb && c < je) continue;
-            for (int j = jb; j < je; j++) {
-                const int r = sp[j - jb];
-                if (r != j) {
-                    const cx<T> t = S[j + c * m];
-                    S[j + c * m] = S[r + c * m];
-                    S[r + c * m] = t;
+        // the other columns: rows of the panel and the rows it displaced, through
+        // the permutation; beyond the panel the U12 rows by forward substitution
+        {
+            const int nd = pm->nd;
+            for (int c = tid; c < m; c += bs) {
+                if (c >= jb && c < je) continue;
+                cx<T> *col = S + c * m;
+                cx<T> u[kLuNb];
+#pragma unroll
+                for (int i = 0; i < kLuNb; i++) u[i] = col[i < nb ? pm->top[i] : jb];
+                if (nd > 0) {
+                    T wr[kLuNb], wi[kLuNb];
+                    static_for<kLuNb>([&](auto k) {
+                        const cx<T> w = col[k < nd ? pm->r[k] : jb];
+                        wr[k] = w.x;
+                        wi[k] = w.y;
+                    });
+                    static_for<kLuNb>([&](auto k) {
+                        if (k < nd) col[pm->q[k]] = {wr[k], wi[k]};
+                    });
                 }
+                if (c >= je)
+                    static_for<kLuNb>([&](auto i) {
+                        if (i < nb)
+                            static_for<i>([&](auto t) { u[i] = cmsub_f(u[i], S[jb + i + (jb + t) * m], u[t]); });
+                    });
+                static_for<kLuNb>([&](auto i) {
+                    if (i < nb) col[jb + i] = u[i];
+                });
             }
         }
         __syncthreads();
         if (je >= m) break;
-        // U12 rows [jb, je) of columns [je, m): one thread per column, rows in order
-        for (int c = je + tid; c < m; c += bs)
-            for (int i = jb + 1; i < je; i++) {
-                cx<T> a = S[i + c * m];
-                for (int t = jb; t < i; t++) a = cmsub_f(a, S[i + t * m], S[t + c * m]);
-                S[i + c * m] = a;
-            }
-        __syncthreads();
         // trailing update of rows and columns [je, m): 2 x 2 tiles, the tile's
         // rows fastest across threads
         const int q = m - je, qt = (q + 1) >> 1;
@@ -625,42 +751,114 @@ __device__ void small_lu_lds(cx<T> *S, int m, int p, int *__restrict__ piv, int 
     }
 }
 
+// what a small front's assembly and LU read of the plan and write beside the arena
+struct SmallDev {
+    const FrontDev *fronts;
+    const int *slot_of, *children, *inv;
+    const int64_t *optr, *oq;
+    const int *ooff;
+    const cx<double> *vals;
+    int64_t vstride;
+    int *piv;
+    int n;
+    int *sing;
+};
+struct SmallShared {
+    LuPerm pm;
+    int64_t cbase[kAsmMaxChildren];
+    int cstride[kAsmMaxChildren];
+};
+// LDS of a small front: the front, then its children's row maps
 template <typename T>
-__global__ void __launch_bounds__(256) k_small_lu(cx<T> *__restrict__ arena, int64_t fstride,
-                                                  const FrontDev *__restrict__ fronts, const int *__restrict__ list,
-                                                  int *__restrict__ piv, int n, int *__restrict__ sing) {
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    cx<T> *S = reinterpret_cast<cx<T> *>(smem_raw);
-    __shared__ int sp[kLuNb];   // the current panel's pivot rows
-    const FrontDev F = fronts[list[blockIdx.x]];
-    const int fq = blockIdx.y;
-    cx<T> *G = arena + fq * fstride + F.buf_off;
-    const int m = F.m, mm = m * m, tid = threadIdx.x, bs = blockDim.x;
-    // FP32: the front staged with all of a thread's loads in flight (m <= 64: at
-    // most 16 entries per thread at 256 threads; entries past the front read its
-    // first).  FP64 keeps one round per 4 entries, measured faster at its
-    // register budget.
-    if constexpr (sizeof(T) == 8) {
-#pragma unroll 4
-        for (int e = tid; e < mm; e += bs) S[e] = G[e];
-    } else {
-        for (int e0 = 0; e0 < mm; e0 += 16 * bs) {
-            cx<T> v[16];
+constexpr size_t small_front_lds(int mmax, int max_children) {
+    return sizeof(cx<T>) * (size_t)mmax * mmax + sizeof(int) * (size_t)mmax * max_children;
+}
+constexpr size_t kSmallLdsMax = 160 * 1024 - 512, kSubLdsMax = 68 * 1024;
+
+// One small front of one frequency, by 256 threads: pull-assembly in LDS from
+// the children's contribution blocks, the original entries added, the partial
+// LU, the front written to the arena -- one pass over the front in memory,
+// where separate assembly, scatter and LU launches wrote it, updated it, read
+// it and wrote it again.  A wave assembles whole columns (lane = row), so the
+// row's child entry is found once per lane and the column's once per wave, and
+// four columns' loads per child are in flight before the first add; an entry
+// no child covers reads the child's block origin and is dropped.  Bound by the
+// LU's chain of panels at four workgroups per CU (LDS).  1601x401, four
+// frequencies: small fronts 4.7 ms in FP64 and 2.3 in FP32, the factorisation
+// 38.6 to 34.6 ms and 24.4 to 22.1.
+template <typename T, int NR>
+__device__ __forceinline__ void small_front(cx<T> *__restrict__ A, const SmallDev &d, int f, int fq, cx<T> *S,
+                                            SmallShared &sh) {
+    const FrontDev F = d.fronts[f];
+    const int m = F.m, mm = m * m, nc = F.nchild, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    int *cmap = reinterpret_cast<int *>(S + mm);   // [nchild][m]: child row of each front row, or -1
+    const int slot = d.slot_of[f];
+    const int64_t o0 = d.optr[slot], o1 = d.optr[slot + 1];
+    if (nc > 0) {
+        if (tid < nc) {
+            const FrontDev C = d.fronts[d.children[F.child_off + tid]];
+            sh.cbase[tid] = C.buf_off + C.p + (int64_t)C.p * C.m;   // contribution block origin
+            sh.cstride[tid] = C.m;
+        }
+        for (int c = 0; c < nc; c++) {
+            const int io = d.fronts[d.children[F.child_off + c]].inv_off;
+            for (int r = tid; r < m; r += 256) cmap[c * m + r] = d.inv[io + r];
+        }
+        __syncthreads();
 #pragma unroll
-            for (int u = 0; u < 16; u++) {
-                const int e = e0 + tid + u * bs;
-                v[u] = G[e < mm ? e : 0];
-            }
+        for (int k = 0; k < NR; k++) {
+            const int r = lane + 64 * k;
+            if (r >= m) break;
+            constexpr int U = 4;
+            for (int s0 = wave * U; s0 < m; s0 += 4 * U) {
+                cx<T> v[U];
 #pragma unroll
-            for (int u = 0; u < 16; u++) {
-                const int e = e0 + tid + u * bs;
-                if (e < mm) S[e] = v[u];
+                for (int u = 0; u < U; u++) v[u] = {T(0), T(0)};
+                for (int c = 0; c < nc; c++) {
+                    const int a = cmap[c * m + r], st = sh.cstride[c];
+                    const cx<T> *B = A + sh.cbase[c];
+                    cx<T> w[U];
+                    bool ok[U];
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        const int b = s0 + u < m ? cmap[c * m + s0 + u] : -1;
+                        ok[u] = a >= 0 && b >= 0;
+                        w[u] = B[ok[u] ? a + b * st : 0];
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; u++)
+                        if (ok[u]) v[u] = cadd(v[u], w[u]);
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++)
+                    if (s0 + u < m) S[r + (s0 + u) * m] = v[u];
             }
         }
+    } else {
+        for (int e = tid; e < mm; e += 256) S[e] = {T(0), T(0)};
     }
     __syncthreads();
-    small_lu_lds<T>(S, m, F.p, piv + (int64_t)fq * n + F.pos0, sing + fq, sp);
-    for (int e = tid; e < mm; e += bs) G[e] = S[e];
+    const cx<double> *V = d.vals + (int64_t)fq * d.vstride;
+    for (int64_t e = o0 + tid; e < o1; e += 256) {
+        const cx<double> v = V[d.oq[e]];
+        cx<T> &t = S[d.ooff[e]];
+        t.x += (T)v.x;
+        t.y += (T)v.y;
+    }
+    __syncthreads();
+    small_lu_lds<T, NR>(S, m, F.p, d.piv + (int64_t)fq * d.n + F.pos0, d.sing + fq, &sh.pm);
+    cx<T> *G = A + F.buf_off;
+    for (int e = tid; e < mm; e += 256) G[e] = S[e];
+}
+
+// grid (the level's small fronts, nfreq)
+template <typename T, int NR>
+__global__ void __launch_bounds__(256) k_small_front(cx<T> *__restrict__ arena, int64_t fstride, SmallDev d,
+                                                     const int *__restrict__ list) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    __shared__ SmallShared sh;
+    const int fq = blockIdx.y;
+    small_front<T, NR>(arena + fq * fstride, d, list[blockIdx.x], fq, reinterpret_cast<cx<T> *>(smem_raw), sh);
 }
 
 // ---------------------------------------------------------------------------
@@ -672,28 +870,16 @@ __global__ void __launch_bounds__(256) k_small_lu(cx<T> *__restrict__ arena, int
 // workgroup earlier in the task, so a workgroup barrier is all the
 // synchronisation there is -- and its original entries, factored there and
 // written to the arena.  No workgroup ever waits for another.  Same
-// arithmetic, in the same order, as k_front_assemble + k_scatter_orig +
-// k_small_lu.
+// arithmetic, in the same order, as k_small_front.
 // ---------------------------------------------------------------------------
 template <typename T>
-__global__ void __launch_bounds__(256) k_subtree_factor(cx<T> *__restrict__ arena, int64_t fstride,
-                                                        const FrontDev *__restrict__ fronts,
+__global__ void __launch_bounds__(256) k_subtree_factor(cx<T> *arena, int64_t fstride, SmallDev d,
                                                         const int *__restrict__ root_first,
-                                                        const int *__restrict__ root_last,
-                                                        const int *__restrict__ slot_of,
-                                                        const int *__restrict__ children, const int *__restrict__ inv,
-                                                        const int64_t *__restrict__ optr,
-                                                        const int64_t *__restrict__ oq, const int *__restrict__ ooff,
-                                                        const cx<double> *__restrict__ vals, int64_t vstride,
-                                                        int nroots, int nf, int *__restrict__ piv, int n,
-                                                        int *__restrict__ sing, int *__restrict__ counter) {
+                                                        const int *__restrict__ root_last, int nroots, int nf,
+                                                        int *__restrict__ counter) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    cx<T> *S = reinterpret_cast<cx<T> *>(smem_raw);
-    __shared__ int cmap[kAsmMaxChildren][kSubMaxM];
-    __shared__ int64_t cbase[kAsmMaxChildren];
-    __shared__ int cstride[kAsmMaxChildren];
+    __shared__ SmallShared sh;
     __shared__ int task;
-    __shared__ int sp[kLuNb];   // the current panel's pivot rows
     const int tid = threadIdx.x, ntask = nroots * nf;
     for (;;) {
         if (tid == 0) task = atomicAdd(counter, 1);
@@ -701,43 +887,9 @@ __global__ void __launch_bounds__(256) k_subtree_factor(cx<T> *__restrict__ aren
         const int t = task;
         if (t >= ntask) return;
         const int r = t / nf, fq = t - r * nf;
-        cx<T> *A = arena + (int64_t)fq * fstride;
-        const cx<double> *V = vals + (int64_t)fq * vstride;
         const int f0 = root_first[r], f1 = root_last[r];
         for (int f = f0; f <= f1; f++) {
-            const FrontDev F = fronts[f];
-            const int m = F.m, nc = F.nchild, mm = m * m, slot = slot_of[f];
-            if (tid < nc) {
-                const FrontDev C = fronts[children[F.child_off + tid]];
-                cbase[tid] = C.buf_off + C.p + (int64_t)C.p * C.m;   // contribution block origin
-                cstride[tid] = C.m;
-            }
-            for (int c = 0; c < nc; c++) {
-                const int io = fronts[children[F.child_off + c]].inv_off;
-                for (int i = tid; i < m; i += blockDim.x) cmap[c][i] = inv[io + i];
-            }
-            __syncthreads();
-#pragma unroll 4
-            for (int e = tid; e < mm; e += blockDim.x) {
-                const int c2 = e / m, i = e - c2 * m;
-                cx<T> v = {T(0), T(0)};
-                for (int c = 0; c < nc; c++) {
-                    const int a = cmap[c][i], b = cmap[c][c2];
-                    if (a >= 0 && b >= 0) v = cadd(v, A[cbase[c] + a + (int64_t)b * cstride[c]]);
-                }
-                S[e] = v;
-            }
-            __syncthreads();
-            for (int64_t e = optr[slot] + tid; e < optr[slot + 1]; e += blockDim.x) {
-                const cx<double> v = V[oq[e]];
-                cx<T> &d = S[ooff[e]];
-                d.x += (T)v.x;
-                d.y += (T)v.y;
-            }
-            __syncthreads();
-            small_lu_lds<T>(S, m, F.p, piv + (int64_t)fq * n + F.pos0, sing + fq, sp);
-            cx<T> *G = A + F.buf_off;
-            for (int e = tid; e < mm; e += blockDim.x) G[e] = S[e];
+            small_front<T, 1>(arena + (int64_t)fq * fstride, d, f, fq, reinterpret_cast<cx<T> *>(smem_raw), sh);
             __syncthreads();   // the parent, later in this loop, reads this block
         }
     }
@@ -1492,25 +1644,25 @@ void factor_numeric(const DevPlan &dp, Factors<T> &F, const cx<double> *vals, in
     const int nf = F.nfreq;
     F.vinv_ready = false;   // the single-vector path's inverse squares follow the new factors
     hipLaunchKernelGGL(k_clear_flags, dim3((nf + 63) / 64), dim3(64), 0, st, F.sing, nf);
-    const size_t lds_small_max = 160 * 1024 - 256;
     const size_t panel_lds_hw = 160 * 1024 - 1024;    // panels of up to 640 c64 / 320 c128 candidate rows
     // panels above the cap take the global-memory panel kernel
     const size_t panel_lds_max = g_panel_lds_cap ? std::min(g_panel_lds_cap, panel_lds_hw) : panel_lds_hw;
     static bool attr_set = false;
     if (!attr_set) {
         // fronts of up to 90x90 complex doubles live in LDS (gfx950: 160 KB per CU)
-        GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_small_lu<double>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_small_max));
-        GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_small_lu<float>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_small_max));
+        for (const void *k : {reinterpret_cast<const void *>(&k_small_front<double, 1>),
+                              reinterpret_cast<const void *>(&k_small_front<double, 2>),
+                              reinterpret_cast<const void *>(&k_small_front<float, 1>),
+                              reinterpret_cast<const void *>(&k_small_front<float, 2>)})
+            GFDFD_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSmallLdsMax));
         GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_panel_lu<double>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)panel_lds_hw));
         GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_panel_lu<float>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)panel_lds_hw));
         GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_subtree_factor<double>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024));
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSubLdsMax));
         GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_subtree_factor<float>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024));
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSubLdsMax));
         GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_trsm_u<double, 64>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)trsm_lds<double, 64>()));
         GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_trsm_u<float, 64>),
@@ -1518,55 +1670,56 @@ void factor_numeric(const DevPlan &dp, Factors<T> &F, const cx<double> *vals, in
         attr_set = true;
     }
     const bool sub = g_persistent && dp.nroots > 0 && F.sched;
+    const SmallDev sd{dp.fronts, dp.slot_of, dp.children, dp.inv, dp.small_optr, dp.small_oq, dp.small_ooff,
+                      vals,      vstride,    F.piv,       pl.n,   F.sing};
+    if (dp.max_children > kAsmMaxChildren) throw std::logic_error("front assembly: too many children");
     if (sub) {
         const int ntask = dp.nroots * nf;
-        const size_t lds = (size_t)dp.sub_mmax * dp.sub_mmax * sizeof(cx<T>);
-        if (lds > 64 * 1024) throw std::logic_error("subtree front exceeds its LDS");
+        const size_t lds = small_front_lds<T>(dp.sub_mmax, dp.max_children);
+        if (lds > kSubLdsMax) throw std::logic_error("subtree front exceeds its LDS");
         hipLaunchKernelGGL(k_clear_flags, dim3(1), dim3(64), 0, st, F.sched, 1);
         ProfScope ps(K_SUBTREE, st, dp.sub_flops * nf, 3.0 * dp.sub_elems * sizeof(cx<T>) * nf);
         // every workgroup takes tasks until none is left; a few per CU keep the CUs busy
         const int grid = std::min(ntask, 256 * 8);
-        hipLaunchKernelGGL(k_subtree_factor<T>, dim3(grid), dim3(256), lds, st, F.arena, F.fstride, dp.fronts,
-                           dp.root_first, dp.root_last, dp.slot_of, dp.children, dp.inv, dp.sub_optr, dp.sub_oq,
-                           dp.sub_ooff, vals, vstride, dp.nroots, nf, F.piv, pl.n, F.sing, F.sched);
+        hipLaunchKernelGGL(k_subtree_factor<T>, dim3(grid), dim3(256), lds, st, F.arena, F.fstride, sd, dp.root_first,
+                           dp.root_last, dp.nroots, nf, F.sched);
     }
     for (int l = 0; l < pl.nlevels; l++) {
         const LevelPlan &L = pl.levels[l];
         const DevPlan::LevelCounts &cnt = dp.counts[l];
         const double es = sizeof(cx<T>) * (double)nf;
-        // the level path: every front of the level, or those outside the small subtrees
-        const int n_asm = sub ? dp.n_asm_rest[l] : dp.n_all[l];
-        const int mmax_asm = sub ? dp.mmax_asm_rest[l] : dp.mmax_all[l];
-        const int *lv_asm = sub ? dp.lv_asm_rest[l] : dp.lv_all[l];
-        if (n_asm > 0) {
-            ProfScope ps(K_FRONT_ASSEMBLE, st, 0.0, (sub ? dp.asm_rest_elems[l] : cnt.asm_elems) * es);
-            int64_t mm = (int64_t)mmax_asm * mmax_asm;
+        // the small fronts: every one of the level, or those outside the subtrees
+        const int n_small = sub ? dp.n_small_rest[l] : dp.n_small[l];
+        if (n_small > 0) {
+            const int smm = sub ? dp.small_mmax_rest[l] : L.small_mmax;
+            const size_t lds = small_front_lds<T>(smm, dp.max_children);
+            if (lds > kSmallLdsMax) throw std::logic_error("small front exceeds LDS");
+            ProfScope ps(K_SMALL_LU, st, (sub ? dp.small_rest_flops[l] : cnt.small_flops) * nf,
+                         (sub ? dp.small_rest_elems[l] : cnt.small_elems) * es);
+            const int *list = sub ? dp.lv_small_rest[l] : dp.lv_small[l];
+            if (smm <= 64)
+                hipLaunchKernelGGL((k_small_front<T, 1>), dim3(n_small, nf), dim3(256), lds, st, F.arena, F.fstride,
+                                   sd, list);
+            else
+                hipLaunchKernelGGL((k_small_front<T, 2>), dim3(n_small, nf), dim3(256), lds, st, F.arena, F.fstride,
+                                   sd, list);
+        }
+        if (dp.n_large[l] > 0) {
+            ProfScope ps(K_FRONT_ASSEMBLE, st, 0.0, dp.asm_elems_large[l] * es);
+            int64_t mm = (int64_t)L.large_mmax * L.large_mmax;
             // about 16 entries per thread (measured faster than 4 or 8)
             int chunks = (int)std::min<int64_t>(std::max<int64_t>(1, mm / (256 * 16)), 256);
-            const size_t lds = sizeof(int) * (size_t)dp.max_children * mmax_asm;
-            if (dp.max_children > kAsmMaxChildren || lds > 64 * 1024)
-                throw std::logic_error("front assembly: too many children or too large a front for the row maps");
-            hipLaunchKernelGGL(k_front_assemble<T>, dim3(n_asm, chunks, nf), dim3(256), lds, st, F.arena,
-                               F.fstride, dp.fronts, lv_asm, dp.children, dp.inv);
+            const size_t lds = sizeof(int) * (size_t)dp.max_children * L.large_mmax;
+            if (lds > 64 * 1024) throw std::logic_error("front assembly: too large a front for the row maps");
+            hipLaunchKernelGGL(k_front_assemble<T>, dim3(dp.n_large[l], chunks, nf), dim3(256), lds, st, F.arena,
+                               F.fstride, dp.fronts, dp.lv_large[l], dp.children, dp.inv);
         }
-        const int64_t obeg = sub ? dp.orig_rest_range[l].first : L.orig_begin;
-        const int64_t ocnt = sub ? dp.orig_rest_range[l].second - obeg : L.orig_end - L.orig_begin;
+        const int64_t obeg = dp.orig_large_range[l].first, ocnt = dp.orig_large_range[l].second - obeg;
         if (ocnt > 0) {
             ProfScope ps(K_SCATTER, st, 0.0, (double)ocnt * (16.0 + 16.0 + 2 * sizeof(cx<T>)) * nf);
             int blocks = (int)std::min<int64_t>((ocnt + 255) / 256, 4096);
             hipLaunchKernelGGL(k_scatter_orig<T>, dim3(blocks, nf), dim3(256), 0, st, F.arena, F.fstride, vals,
-                               vstride, (sub ? dp.orig_q_rest : dp.orig_q) + obeg,
-                               (sub ? dp.orig_dst_rest : dp.orig_dst) + obeg, ocnt);
-        }
-        const int n_small = sub ? dp.n_small_rest[l] : dp.n_small[l];
-        if (n_small > 0) {
-            const int smm = sub ? dp.small_mmax_rest[l] : L.small_mmax;
-            size_t lds = (size_t)smm * smm * sizeof(cx<T>);
-            if (lds > lds_small_max) throw std::logic_error("small front exceeds LDS");
-            ProfScope ps(K_SMALL_LU, st, (sub ? dp.small_rest_flops[l] : cnt.small_flops) * nf,
-                         (sub ? dp.small_rest_elems[l] : cnt.small_elems) * es);
-            hipLaunchKernelGGL(k_small_lu<T>, dim3(n_small, nf), dim3(256), lds, st, F.arena, F.fstride,
-                               dp.fronts, sub ? dp.lv_small_rest[l] : dp.lv_small[l], F.piv, pl.n, F.sing);
+                               vstride, dp.orig_q_large + obeg, dp.orig_dst_large + obeg, ocnt);
         }
         if (dp.n_large[l] > 0) {
             const size_t lds32 = trsm_lds<T, 32>(), lds64 = trsm_lds<T, 64>();

@@ -1,0 +1,48 @@
+"""The factorisation's kernels at the sizes where their code changes: orders
+around one and two rows per lane, panels shorter than a block, pivoting that
+moves rows, against the banded oracle."""
+import numpy as np
+import pytest
+
+import germaine_amd as G
+from germaine_amd import fdfd
+from oracle import oracle as O
+from tests._grids import smooth_model
+from tests.test_gpu_parity import dev, oracle_system, random_grid_csc, rel, say
+
+pytestmark = pytest.mark.gpu
+
+
+def solve_and_check(pl, nx, ny, mats, precision, tol64, sys=0):
+    F = pl.factor(dev(np.stack([c[2] + 1j * c[3] for c in mats])), precision)
+    assert np.all(F.singular() == 0)
+    rng = np.random.default_rng(nx * ny)
+    nf = len(mats)
+    B = rng.standard_normal((nf, 5, nx * ny)) + 1j * rng.standard_normal((nf, 5, nx * ny))
+    if precision == G.FP64:
+        X = F.solve_batch(list(range(nf)), dev(B), sys=sys).cpu().numpy()
+    else:
+        X = F.solve_refine_batch(list(range(nf)), dev(B), sys=sys, tol=1e-12, max_iter=30)[0].cpu().numpy()
+    for z, c in enumerate(mats):
+        Xr, _ = O.band_solve(*c, B[z].T, sys=sys, perm=O.grid_transpose_perm(nx, ny))
+        assert rel(X[z], Xr.T) <= (tol64 if precision == G.FP64 else 1e-8), z
+
+
+# small fronts of one and of two rows per lane (small_max up to 64, and above), leaves from 2 x 2 on
+@pytest.mark.parametrize("precision", [G.FP64, G.FP32])
+@pytest.mark.parametrize("leaf_area,small_max", [(4, 13), (9, 30), (32, 64), (32, 66), (50, 90)])
+def test_small_fronts_match_oracle(leaf_area, small_max, precision):
+    nx, ny = 53, 47
+    say("small fronts", leaf_area, small_max, precision)
+    pl = fdfd.Plan(nx, ny, leaf_area=leaf_area, small_max=small_max)
+    m = pl.fronts()["m"]
+    assert m[m <= small_max].max() > 0.7 * small_max
+    m1, m2 = smooth_model(nx, ny, seed=3)
+    helm = [oracle_system(G.AC, nx, ny, 6, 10.0, f, m1, m2)[1] for f in (4.0, 9.0)]
+    fdfd.factor_tuning(0, 0, fdfd.NO_DEEP)
+    try:
+        solve_and_check(pl, nx, ny, helm, precision, 1e-10)
+        # random values: rows move in every panel
+        solve_and_check(pl, nx, ny, [random_grid_csc(nx, ny, s) for s in (7, 8)], precision, 1e-8)
+    finally:
+        fdfd.factor_tuning()
