@@ -148,13 +148,11 @@ void cast_c64_to_c128(int64_t count, const cx<float> *a, cx<double> *b, hipStrea
 // (negative: no limit beyond LDS), and the layout of the panel refinement
 // (0: elimination order, 1: user layout with a transpose per correction)
 void set_solve_tuning(int rw_cap, int fused_mmax, int refine_layout);
-// factorisation kernel selection: panels needing more LDS than panel_lds_cap
-// bytes (0: the hardware limit) take the global-memory panel kernel; the small
-// subtrees take the persistent launch when persistent != 0, else the level path
-// panel_lds_cap: panels needing more LDS take the global-memory panel kernel
-// (0: the hardware limit); persistent: the small subtrees in one launch;
-// deep_min_m: levels whose largest blocked front has order >= deep_min_m take
-// the two-panel (depth-64) schedule, the others one panel at a time
+// factorisation kernel selection: panels of more than panel_lds_cap bytes
+// (0: no cap) take the global-memory panel kernel, as those too tall for
+// registers always do; persistent: the small subtrees in one launch, else level
+// by level; deep_min_m: levels whose largest blocked front has order >=
+// deep_min_m take the two-panel (depth-64) schedule, the others one panel at a time
 void set_factor_tuning(int panel_lds_cap, int persistent, int deep_min_m);
 // frees the calling thread's cached solve work buffers
 void release_solve_workspaces();

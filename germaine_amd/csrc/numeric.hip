@@ -938,155 +938,275 @@ __global__ void __launch_bounds__(256) k_panel(cx<T> *__restrict__ arena, int64_
 }
 
 // ---------------------------------------------------------------------------
-// 3c: blocked path, panel held in LDS.  The pivot candidates of a 32-column
-// panel are the front's remaining fully-summed rows [k0, p); their panel
-// columns are factored entirely in LDS (column-major, np rows), with the row
-// swaps kept inside the panel.  k_panel_apply then applies the swap sequence to
-// the front's other columns and finishes the panel columns of the
-// contribution rows [p, m), which need no pivoting: row a of them becomes the
-// solution of x U_kk = a.  Same result as k_panel, with the per-column steps in
-// LDS instead of global memory.
+// 3c: blocked path, panel held in registers.  The pivot candidates of a
+// 32-column panel are the front's remaining fully-summed rows [k0, p), one row
+// per thread, all its panel columns in that thread's registers.  Rows do not
+// move while the panel is factored: each thread carries the position its row
+// has reached.  Per column every wave finds its best candidate (DPP maximum
+// and a ballot) and that lane publishes value, position, reciprocal and row in
+// the wave's slot; one barrier later every thread picks the winning wave and
+// updates its own row from that slot (slots alternate, so a step has one
+// barrier).  Eight columns are unrolled, then the row is rotated by eight
+// registers, so the code stays short enough for the instruction cache.
+// k_panel_finish then applies the panel's permutation to the front's other
+// columns.  Bound by the 32-step chain: a panel in LDS with three barriers per
+// column took 48 us (270x145, one FP64 frequency, event-timed), this 32; the 69
+// panels of 1601x401, four frequencies, 8.5 ms (those above 318 rows in global
+// memory) and 3.5.
 // ---------------------------------------------------------------------------
 template <typename T>
-__global__ void __launch_bounds__(256) k_panel_lu(cx<T> *__restrict__ arena, int64_t fstride,
-                                                  const FrontDev *__restrict__ fronts, const int *__restrict__ list,
-                                                  int *__restrict__ piv, int n, int k0, int nb, int *__restrict__ sing) {
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    cx<T> *P = reinterpret_cast<cx<T> *>(smem_raw);
-    __shared__ int si[1];
+struct PanelSlot {
+    T best;
+    int pos;
+    cx<T> rc;
+    cx<T> row[32];
+};
+template <typename T, int NW>
+__global__ void __launch_bounds__(64 * NW) k_panel_reg(cx<T> *__restrict__ arena, int64_t fstride,
+                                                       const FrontDev *__restrict__ fronts,
+                                                       const int *__restrict__ list, int *__restrict__ piv, int n,
+                                                       int k0, int nb, int *__restrict__ sing) {
+    __shared__ PanelSlot<T> slot[2][NW];
     const FrontDev F = fronts[list[blockIdx.x]];
     if (F.p <= k0) return;
     const int fq = blockIdx.y;
     cx<T> *G = arena + fq * fstride + F.buf_off;
-    const int m = F.m, p = F.p, kb = min(nb, p - k0), np = p - k0, tid = threadIdx.x;
-    // the panel staged eight entries per thread at a time, all eight loads in
-    // flight before the stores (entries past the panel read its first)
-    for (int e0 = 0; e0 < np * kb; e0 += 8 * 256) {
-        cx<T> v[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const int e = e0 + tid + 256 * u, ec = e < np * kb ? e : 0, r = ec % np, c = ec / np;
-            v[u] = G[(k0 + r) + (int64_t)(k0 + c) * m];
-        }
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const int e = e0 + tid + 256 * u;
-            if (e < np * kb) P[(e / np) * np + e % np] = v[u];
-        }
-    }
-    __syncthreads();
-    __shared__ cx<T> pv[2];   // pivot entry and the entry it swaps with, published with the pivot row
-    for (int j = 0; j < kb; j++) {
-        // pivot search by wave 0 alone (a few candidates per lane)
-        if (tid < 64) {
-            T best = T(-1);
-            int bi = j;
-            for (int r = j + tid; r < np; r += 64) better(best, bi, cabs1(P[j * np + r]), r);
-            for (int off = 32; off > 0; off >>= 1) {
-                const T ob = __shfl_xor(best, off);
-                const int oi = __shfl_xor(bi, off);
-                better(best, bi, ob, oi);
+    const int m = F.m, p = F.p, kb = min(nb, p - k0), np = p - k0;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const bool in = tid < np;
+    // (rows past the panel and columns past kb read a valid entry and become zero)
+    T ar[32], ai[32];
+    static_for<32>([&](auto c) {
+        const cx<T> v = G[(k0 + (in ? tid : 0)) + (int64_t)(k0 + (c < kb ? c : 0)) * m];
+        ar[c] = in && c < kb ? v.x : T(0);
+        ai[c] = in && c < kb ? v.y : T(0);
+    });
+    int pos = tid;
+    bool zero = false;
+    const int n8 = (kb + 7) >> 3;
+#pragma unroll 1
+    for (int b = 0; b < 4; b++) {
+        static_for<8>([&](auto jj) {
+            const int j = 8 * b + jj;
+            if (j < kb) {
+                // the thread's candidate (a NaN counts as -1, rows done or outside as -2)
+                const T v = fabs(ar[jj]) + fabs(ai[jj]);
+                const T best = in && pos >= j ? (v >= T(0) ? v : T(-1)) : T(-2);
+                const cx<T> rc = crecip(cx<T>{ar[jj], ai[jj]});
+                const T mx = wave_max(best);
+                const unsigned long long tie = __ballot(best == mx);
+                int L = __ffsll((unsigned long long)tie) - 1;
+                if (tie & (tie - 1)) {
+                    const int lowest = wave_min(best == mx ? pos : 64 * NW);
+                    L = __ffsll((unsigned long long)__ballot(best == mx && pos == lowest)) - 1;
+                }
+                PanelSlot<T> *sl = slot[jj & 1];
+                if (lane == L) {
+                    PanelSlot<T> &s = sl[wave];
+                    s.best = best;
+                    s.pos = pos;
+                    s.rc = rc;
+                    static_for<8>([&](auto c) {
+                        if (c >= jj) s.row[c] = {ar[c], ai[c]};
+                    });
+                    static_for<3>([&](auto g) {
+                        if (b + g + 1 < n8) static_for<8>([&](auto c) {
+                            s.row[8 * g + 8 + c] = {ar[8 * g + 8 + c], ai[8 * g + 8 + c]};
+                        });
+                    });
+                }
+                __syncthreads();
+                T wb = sl[0].best;
+                int pr = sl[0].pos, ww = 0;
+                static_for<NW>([&](auto w) {
+                    if (w > 0) {
+                        const T ob = sl[w].best;
+                        const int op = sl[w].pos;
+                        if (ob > wb || (ob == wb && op < pr)) {
+                            wb = ob;
+                            pr = op;
+                            ww = w;
+                        }
+                    }
+                });
+                const PanelSlot<T> &s = sl[ww];
+                if (tid == 0) piv[(int64_t)fq * n + F.pos0 + k0 + j] = k0 + pr;
+                zero |= wb == T(0);
+                pos = pos == pr ? j : pos == j ? pr : pos;
+                if (in && pos > j) {
+                    const cx<T> l = cmul_f(cx<T>{ar[jj], ai[jj]}, s.rc);
+                    ar[jj] = l.x;
+                    ai[jj] = l.y;
+                    static_for<8>([&](auto c) {
+                        if (c > jj) {
+                            const cx<T> a = cmsub_f(cx<T>{ar[c], ai[c]}, l, s.row[c]);
+                            ar[c] = a.x;
+                            ai[c] = a.y;
+                        }
+                    });
+                    static_for<3>([&](auto g) {
+                        if (b + g + 1 < n8) static_for<8>([&](auto cc) {
+                            constexpr int c = 8 * g + 8 + cc;
+                            const cx<T> a = cmsub_f(cx<T>{ar[c], ai[c]}, l, s.row[c]);
+                            ar[c] = a.x;
+                            ai[c] = a.y;
+                        });
+                    });
+                }
             }
-            if (tid == 0) {
-                si[0] = bi;
-                pv[0] = P[j * np + bi];
-                pv[1] = P[j * np + j];
-                piv[(int64_t)fq * n + F.pos0 + k0 + j] = k0 + bi;
-                if (best == T(0)) atomicOr(sing + fq, 1);
-            }
-        }
-        __syncthreads();
-        // row swap in the panel's other columns and the scaled column j, in one
-        // pass: column j's swapped pair comes from pv, read before anyone wrote
-        const int pr = si[0];
-        const cx<T> d = crecip(pv[0]);
-        if (pr != j && tid < kb && tid != j) {
-            const cx<T> t = P[tid * np + j];
-            P[tid * np + j] = P[tid * np + pr];
-            P[tid * np + pr] = t;
-        }
-        for (int r = j + 1 + tid; r < np; r += 256) P[j * np + r] = cmul(r == pr ? pv[1] : P[j * np + r], d);
-        if (tid == 0) P[j * np + j] = pv[0];
-        __syncthreads();
-        const int rows = np - j - 1, ncol = kb - j - 1;
-        for (int e = tid; e < rows * ncol; e += 256) {
-            const int c = j + 1 + e / rows, r = j + 1 + e % rows;
-            P[c * np + r] = cmsub(P[c * np + r], P[j * np + r], P[c * np + j]);
-        }
-        __syncthreads();
+        });
+        // the next eight columns to the front; after four rotations the order is the first one
+        T tr[8], ti[8];
+        static_for<8>([&](auto c) {
+            tr[c] = ar[c];
+            ti[c] = ai[c];
+        });
+        static_for<24>([&](auto c) {
+            ar[c] = ar[c + 8];
+            ai[c] = ai[c + 8];
+        });
+        static_for<8>([&](auto c) {
+            ar[c + 24] = tr[c];
+            ai[c + 24] = ti[c];
+        });
     }
-    for (int e = tid; e < np * kb; e += 256) {
-        const int r = e % np, c = e / np;
-        G[(k0 + r) + (int64_t)(k0 + c) * m] = P[c * np + r];
-    }
+    if (zero && tid == 0) atomicOr(sing + fq, 1);
+    if (in)
+        static_for<32>([&](auto c) {
+            if (c < kb) G[(k0 + pos) + (int64_t)(k0 + c) * m] = {ar[c], ai[c]};
+        });
 }
-
-// grid (column or row chunks of 64, fronts, nfreq): chunk x < ccols handles 64
-// columns outside the panel (swap sequence), the rest 64 contribution rows
+// most candidate rows of a panel in registers: one per thread, 512 threads in
+// FP64 (128 registers a row, two waves per SIMD) and 1024 in FP32
 template <typename T>
-__global__ void __launch_bounds__(64) k_panel_apply(cx<T> *__restrict__ arena, int64_t fstride,
-                                                    const FrontDev *__restrict__ fronts, const int *__restrict__ list,
-                                                    const int *__restrict__ piv, int n, int k0, int nb, int ccols) {
+constexpr int kPanelRows = sizeof(T) == 8 ? 512 : 1024;
+
+// After a panel's LU: grid (column or row chunks of 64, fronts, nfreq), one
+// wave per chunk.  Chunk x < ccols: 64 columns outside the panel, one per lane
+// -- the panel's row permutation and, with TRSM, the U12 rows of the columns
+// beyond it by forward substitution, the column's 32 rows in registers.  The
+// permutation follows from the swap sequence: lane t tracks where row k0 + t
+// (t < 32), or the row that step t - 32 pulled in, ends.  A row outside the
+// panel only ever receives one of the panel's first rows, so those are moved
+// once every lane holds its sources.  The other chunks: 64 contribution rows,
+// x U_kk = a.  Replaces 32 dependent swaps in memory and a triangular
+// solve with a shuffle reduction per row in a launch of its own: 345 + 325 us
+// against 511 per factorisation of 270x145 (FP64, 22 panels), 1.48 + 1.70 ms
+// against 2.41 in FP32 at 1601x401, four frequencies.  Bound by the dependent
+// rows at two to three waves per SIMD (registers).
+template <typename T, bool TRSM>
+__global__ void __launch_bounds__(64) k_panel_finish(cx<T> *__restrict__ arena, int64_t fstride,
+                                                     const FrontDev *__restrict__ fronts, const int *__restrict__ list,
+                                                     const int *__restrict__ piv, int n, int k0, int nb, int ccols) {
     __shared__ cx<T> U[32][33];
-    __shared__ int ps[32];
+    __shared__ int src[32], dq[32], dr[32];
     const FrontDev F = fronts[list[blockIdx.y]];
     if (F.p <= k0) return;
     const int fq = blockIdx.z;
     cx<T> *G = arena + fq * fstride + F.buf_off;
     const int m = F.m, p = F.p, kb = min(nb, p - k0), tid = threadIdx.x;
-    if ((int)blockIdx.x < ccols) {
-        // columns c outside [k0, k0+kb): the panel's row swaps, in order
-        if (tid < kb) ps[tid] = piv[(int64_t)fq * n + F.pos0 + k0 + tid];
+    const bool cols = (int)blockIdx.x < ccols;
+    if (cols && (int)blockIdx.x * 64 >= m - kb) return;
+    if (!cols && p + ((int)blockIdx.x - ccols) * 64 >= m) return;
+    // the panel's block, 16 entries per thread, all in flight before the stores
+    if (TRSM || !cols) {
+        T ur[16], ui[16];
+        static_for<16>([&](auto u) {
+            const int e = tid + 64 * u, r = e & 31, c = e >> 5;
+            const cx<T> v = G[(k0 + (r < kb ? r : 0)) + (int64_t)(k0 + (c < kb ? c : 0)) * m];
+            ur[u] = v.x;
+            ui[u] = v.y;
+        });
+        static_for<16>([&](auto u) {
+            const int e = tid + 64 * u, r = e & 31, c = e >> 5;
+            U[r][c] = {ur[u], ui[u]};
+        });
+    }
+    if (cols) {
+        // columns c outside [k0, k0+kb)
+        const int pv = (tid & 31) < kb ? piv[(int64_t)fq * n + F.pos0 + k0 + (tid & 31)] : -1;
+        const int row = tid < 32 ? (tid < kb ? k0 + tid : -1) : pv;
+        int pos = row;
+        bool live = tid < 32 ? tid < kb : pv >= k0 + kb;
+        for (int j = 0; j < kb; j++) {
+            const int s = __builtin_amdgcn_readlane(pv, j), a = k0 + j;
+            if (tid - 32 > j && s == row) live = false;   // pulled in before: tracked by that lane
+            pos = pos == a ? s : pos == s ? a : pos;
+        }
+        if (live && pos < k0 + kb) src[pos - k0] = row;
+        const bool out = live && pos >= k0 + kb && pos != row;
+        const unsigned long long outs = __ballot(out);
+        if (out) {
+            const int at = __popcll(outs & ((1ull << tid) - 1));
+            dq[at] = pos;
+            dr[at] = row;
+        }
+        const int nd = __popcll(outs);
+        const bool moved = __ballot(live && pos != row) != 0;
         __syncthreads();
         int c = blockIdx.x * 64 + tid;
-        if (c >= k0) c += kb;
-        if (c >= m) return;
+        const bool beyond = c >= k0;
+        if (beyond) c += kb;
+        if (c >= m || (!moved && !(TRSM && beyond))) return;
         cx<T> *col = G + (int64_t)c * m;
-        for (int j = 0; j < kb; j++) {
-            const int r = ps[j];
-            if (r != k0 + j) {
-                const cx<T> t = col[k0 + j];
-                col[k0 + j] = col[r];
-                col[r] = t;
-            }
+        T xr[32], xi[32];
+        static_for<32>([&](auto t) {
+            const cx<T> v = col[t < kb ? src[t] : k0];
+            xr[t] = v.x;
+            xi[t] = v.y;
+        });
+        for (int k = 0; k < nd; k += 8) {
+            T wr[8], wi[8];
+            static_for<8>([&](auto u) {
+                const cx<T> v = col[k + u < nd ? dr[k + u] : k0];
+                wr[u] = v.x;
+                wi[u] = v.y;
+            });
+            static_for<8>([&](auto u) {
+                if (k + u < nd) col[dq[k + u]] = {wr[u], wi[u]};
+            });
         }
+        if (TRSM && beyond)
+            static_for<31>([&](auto t) {
+                static_for<31 - t>([&](auto d) {
+                    constexpr int i = t + 1 + d;
+                    const cx<T> v = cmsub_f(cx<T>{xr[i], xi[i]}, U[i][t], cx<T>{xr[t], xi[t]});
+                    xr[i] = v.x;
+                    xi[i] = v.y;
+                });
+                // (keeps the scheduler from hoisting the whole block's LDS reads into registers)
+                if constexpr (t % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+            });
+        static_for<32>([&](auto t) {
+            if (t < kb) col[k0 + t] = {xr[t], xi[t]};
+        });
         return;
     }
-    // contribution rows: x U_kk = a, U_kk from the factored panel
-    // the block U_kk (16 entries per thread, all in flight before the stores),
-    // then the row's panel entries (unconditional: columns past kb read column
-    // k0 and are not used)
-    const int i = p + (blockIdx.x - ccols) * 64 + tid, ic = i < m ? i : p;
-    {
-        cx<T> uv[16];
-#pragma unroll
-        for (int u = 0; u < 16; u++) {
-            const int e = tid + 64 * u, r = e & 31, c = e >> 5;
-            uv[u] = G[(k0 + (r < kb ? r : 0)) + (int64_t)(k0 + (c < kb ? c : 0)) * m];
-        }
-#pragma unroll
-        for (int u = 0; u < 16; u++) {
-            const int e = tid + 64 * u, r = e & 31, c = e >> 5;
-            if (r < kb && c < kb) U[r][c] = uv[u];
-        }
-    }
+    // contribution rows: x U_kk = a, U_kk from the factored panel (columns past kb
+    // read column k0 and are not used)
+    const int i = p + ((int)blockIdx.x - ccols) * 64 + tid, ic = i < m ? i : p;
+    T xr[32], xi[32];
+    static_for<32>([&](auto t) {
+        const cx<T> v = G[ic + (int64_t)(k0 + (t < kb ? t : 0)) * m];
+        xr[t] = v.x;
+        xi[t] = v.y;
+    });
     __syncthreads();
-    if (i >= m) return;
-    cx<T> x[32];
-#pragma unroll
-    for (int t = 0; t < 32; t++) x[t] = G[ic + (int64_t)(k0 + (t < kb ? t : 0)) * m];
-#pragma unroll
-    for (int t = 0; t < 32; t++) {
+    const cx<T> rc = crecip(U[tid & 31][tid & 31]);   // lane t: the reciprocal of pivot t
+    static_for<32>([&](auto t) {
         if (t < kb) {
-            cx<T> a = x[t];
-#pragma unroll
-            for (int s = 0; s < t; s++) a = cmsub(a, x[s], U[s][t]);
-            x[t] = cmul(a, crecip(U[t][t]));
+            cx<T> a = {xr[t], xi[t]};
+            static_for<t>([&](auto s) { a = cmsub_f(a, cx<T>{xr[s], xi[s]}, U[s][t]); });
+            a = cmul_f(a, readlane_t(rc, t));
+            xr[t] = a.x;
+            xi[t] = a.y;
         }
-    }
-#pragma unroll
-    for (int t = 0; t < 32; t++)
-        if (t < kb) G[i + (int64_t)(k0 + t) * m] = x[t];
+        __builtin_amdgcn_sched_barrier(0);
+    });
+    if (i < m)
+        static_for<32>([&](auto t) {
+            if (t < kb) G[i + (int64_t)(k0 + t) * m] = {xr[t], xi[t]};
+        });
 }
 
 // U12 rows of the pivot block: rows [k0, k0+kb) of the columns beyond it,
@@ -1612,7 +1732,7 @@ __global__ void __launch_bounds__(256) k_diag_inv(cx<T> *__restrict__ arena, int
 // driver
 // ---------------------------------------------------------------------------
 namespace {
-size_t g_panel_lds_cap = 0;   // 0: the hardware limit
+size_t g_panel_lds_cap = 0;   // 0: none
 // Until a caller selects otherwise (g_deep_min_m < 0): the small fronts level by
 // level, and two panels per step only where the trailing update is bound by
 // its passes over memory.  The persistent subtree launch is a serial chain of
@@ -1644,9 +1764,6 @@ void factor_numeric(const DevPlan &dp, Factors<T> &F, const cx<double> *vals, in
     const int nf = F.nfreq;
     F.vinv_ready = false;   // the single-vector path's inverse squares follow the new factors
     hipLaunchKernelGGL(k_clear_flags, dim3((nf + 63) / 64), dim3(64), 0, st, F.sing, nf);
-    const size_t panel_lds_hw = 160 * 1024 - 1024;    // panels of up to 640 c64 / 320 c128 candidate rows
-    // panels above the cap take the global-memory panel kernel
-    const size_t panel_lds_max = g_panel_lds_cap ? std::min(g_panel_lds_cap, panel_lds_hw) : panel_lds_hw;
     static bool attr_set = false;
     if (!attr_set) {
         // fronts of up to 90x90 complex doubles live in LDS (gfx950: 160 KB per CU)
@@ -1655,10 +1772,6 @@ void factor_numeric(const DevPlan &dp, Factors<T> &F, const cx<double> *vals, in
                               reinterpret_cast<const void *>(&k_small_front<float, 1>),
                               reinterpret_cast<const void *>(&k_small_front<float, 2>)})
             GFDFD_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSmallLdsMax));
-        GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_panel_lu<double>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)panel_lds_hw));
-        GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_panel_lu<float>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)panel_lds_hw));
         GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_subtree_factor<double>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSubLdsMax));
         GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_subtree_factor<float>),
@@ -1723,26 +1836,49 @@ void factor_numeric(const DevPlan &dp, Factors<T> &F, const cx<double> *vals, in
         }
         if (dp.n_large[l] > 0) {
             const size_t lds32 = trsm_lds<T, 32>(), lds64 = trsm_lds<T, 64>();
-            // one 32-column panel of every blocked front of the level: its LU
-            // (in LDS, or in global memory when the candidate rows do not fit)
-            // and the row swaps on the other columns with the contribution rows
-            auto panel = [&](int k0, double flops) {
-                const size_t plds = (size_t)(L.large_pmax - k0) * pl.nb * sizeof(cx<T>);
-                if (plds <= panel_lds_max) {
+            // one 32-column panel of every blocked front of the level: its LU (in
+            // registers, or in global memory when the candidate rows are too many
+            // or exceed the caller's cap), the row permutation on the other columns
+            // with the contribution rows and, with trsm, the U12 rows
+            auto panel = [&](int k0, double flops, bool trsm, double trsm_flops) {
+                const int rows = L.large_pmax - k0;
+                const size_t plds = (size_t)rows * pl.nb * sizeof(cx<T>);
+                const int ccols = (L.large_mmax + 63) / 64;   // m - kb columns of any front fit
+                const int crows = (L.large_mmax + 63) / 64;
+                if (rows <= kPanelRows<T> && (!g_panel_lds_cap || plds <= g_panel_lds_cap)) {
                     {
                         ProfScope ps(K_PANEL, st, flops * nf, 0.0);
-                        hipLaunchKernelGGL(k_panel_lu<T>, dim3(dp.n_large[l], nf), dim3(256), plds, st, F.arena,
-                                           F.fstride, dp.fronts, dp.lv_large[l], F.piv, pl.n, k0, pl.nb, F.sing);
+                        const dim3 g(dp.n_large[l], nf);
+#define PANEL(NW) \
+    hipLaunchKernelGGL((k_panel_reg<T, NW>), g, dim3(64 * NW), 0, st, F.arena, F.fstride, dp.fronts, dp.lv_large[l], \
+                       F.piv, pl.n, k0, pl.nb, F.sing)
+                        if (rows <= 64) PANEL(1);
+                        else if (rows <= 128) PANEL(2);
+                        else if (rows <= 256) PANEL(4);
+                        else if (rows <= 512) PANEL(8);
+                        else if constexpr (sizeof(T) == 4) PANEL(16);
+#undef PANEL
                     }
-                    const int ccols = (L.large_mmax + 63) / 64;   // m - kb columns of any front fit
-                    const int crows = (L.large_mmax + 63) / 64;
-                    ProfScope ps(K_PANEL_APPLY, st, 0.0, 0.0);
-                    hipLaunchKernelGGL(k_panel_apply<T>, dim3(ccols + crows, dp.n_large[l], nf), dim3(64), 0, st,
-                                       F.arena, F.fstride, dp.fronts, dp.lv_large[l], F.piv, pl.n, k0, pl.nb, ccols);
+                    ProfScope ps(K_PANEL_APPLY, st, trsm ? trsm_flops * nf : 0.0, 0.0);
+                    if (trsm)
+                        hipLaunchKernelGGL((k_panel_finish<T, true>), dim3(ccols + crows, dp.n_large[l], nf), dim3(64),
+                                           0, st, F.arena, F.fstride, dp.fronts, dp.lv_large[l], F.piv, pl.n, k0,
+                                           pl.nb, ccols);
+                    else
+                        hipLaunchKernelGGL((k_panel_finish<T, false>), dim3(ccols + crows, dp.n_large[l], nf),
+                                           dim3(64), 0, st, F.arena, F.fstride, dp.fronts, dp.lv_large[l], F.piv, pl.n,
+                                           k0, pl.nb, ccols);
                 } else {
-                    ProfScope ps(K_PANEL, st, flops * nf, 0.0);
-                    hipLaunchKernelGGL(k_panel<T>, dim3(dp.n_large[l], nf), dim3(256), 0, st, F.arena, F.fstride,
-                                       dp.fronts, dp.lv_large[l], F.piv, pl.n, k0, pl.nb, F.sing);
+                    {
+                        ProfScope ps(K_PANEL, st, flops * nf, 0.0);
+                        hipLaunchKernelGGL(k_panel<T>, dim3(dp.n_large[l], nf), dim3(256), 0, st, F.arena, F.fstride,
+                                           dp.fronts, dp.lv_large[l], F.piv, pl.n, k0, pl.nb, F.sing);
+                    }
+                    if (trsm) {
+                        ProfScope ps(K_TRSM, st, trsm_flops * nf, 0.0);
+                        hipLaunchKernelGGL((k_trsm_u<T, 32>), dim3(ccols, dp.n_large[l], nf), dim3(256), lds32, st,
+                                           F.arena, F.fstride, dp.fronts, dp.lv_large[l], k0, 0);
+                    }
                 }
             };
             auto gemm = [&](int64_t off, int cnt, int k0, int depth, int ccap, double flops, double elems) {
@@ -1765,7 +1901,7 @@ void factor_numeric(const DevPlan &dp, Factors<T> &F, const cx<double> *vals, in
                 int bi = 0;
                 for (int b0 = 0; b0 < L.large_pmax; b0 += 64, bi++) {
                     const auto &d = dp.deep_steps[l][bi];
-                    panel(b0, d.panel1_flops);
+                    panel(b0, d.panel1_flops, false, 0.0);
                     if (d.thin_cnt > 0) {
                         {
                             ProfScope ps(K_TRSM, st, d.trsm_thin_flops * nf, 0.0);
@@ -1774,7 +1910,7 @@ void factor_numeric(const DevPlan &dp, Factors<T> &F, const cx<double> *vals, in
                                                b0, 64);
                         }
                         gemm(d.thin_off, d.thin_cnt, b0, 32, 64, d.thin_flops, d.thin_elems);
-                        panel(b0 + 32, d.panel2_flops);
+                        panel(b0 + 32, d.panel2_flops, false, 0.0);
                     }
                     {
                         ProfScope ps(K_TRSM, st, d.trsm_deep_flops * nf, 0.0);
@@ -1788,14 +1924,7 @@ void factor_numeric(const DevPlan &dp, Factors<T> &F, const cx<double> *vals, in
             } else {
                 int si = 0;
                 for (int k0 = 0; k0 < L.large_pmax; k0 += pl.nb, si++) {
-                    panel(k0, cnt.panel_flops[si]);
-                    {
-                        ProfScope ps(K_TRSM, st, cnt.trsm_flops[si] * nf, 0.0);
-                        const int colchunks = (L.large_mmax - k0 + 63) / 64;
-                        hipLaunchKernelGGL((k_trsm_u<T, 32>), dim3(colchunks, dp.n_large[l], nf), dim3(256),
-                                           lds32, st, F.arena, F.fstride, dp.fronts, dp.lv_large[l], k0,
-                                           0);
-                    }
+                    panel(k0, cnt.panel_flops[si], true, cnt.trsm_flops[si]);
                     const auto &sp = dp.steps[l][si];
                     gemm(sp.first, sp.second, k0, 32, 0, cnt.gemm_flops[si], cnt.gemm_elems[si]);
                 }

@@ -101,9 +101,9 @@ NO_DEEP = 1 << 30   # deep_min_m that keeps every level on one panel per step
 
 
 def factor_tuning(panel_lds_cap=0, persistent=1, deep_min_m=0):
-    """Factorisation kernel selection (process-wide): panels needing more than
-    panel_lds_cap bytes of LDS take the global-memory panel kernel (0: the
-    hardware limit); persistent selects the one-launch factorisation of the
+    """Factorisation kernel selection (process-wide): panels of more than
+    panel_lds_cap bytes take the global-memory panel kernel (0: no cap beyond
+    what fits in registers); persistent selects the one-launch factorisation of the
     small subtrees (else level by level); levels whose largest blocked front
     has order >= deep_min_m take the two-panel schedule (trailing update once
     per 64 pivots), the others one panel at a time (NO_DEEP: none).  Until the

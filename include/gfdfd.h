@@ -180,10 +180,10 @@ int gfdfd_residual(gfdfd_plan plan, const double *d_vals, int sys, int nrhs, con
  * 1: the caller's column-major layout, two transposes per correction).      */
 int gfdfd_solve_tuning(int rw_cap, int fused_mmax, int refine_layout);
 /* Factorisation kernel selection (process-wide, for later factorisations and
- * graph captures): a 32-column panel whose candidate rows need more than
- * panel_lds_cap bytes of LDS is factored by the global-memory panel kernel
- * instead of in LDS (0: the hardware limit, 159 KB -- separators above 318
- * rows in FP64, 637 in FP32), which lets small systems exercise that path;
+ * graph captures): a 32-column panel whose candidate rows take more than
+ * panel_lds_cap bytes is factored by the global-memory panel kernel instead
+ * of in registers (0: no cap; panels of more than 512 rows in FP64 and 1024
+ * in FP32 always are), which lets small systems exercise that path;
  * persistent != 0 factors the small subtrees -- fronts of order
  * <= 64 whose descendants are all that small -- in one persistent launch in
  * which a workgroup factors one whole subtree of one frequency per task, 0

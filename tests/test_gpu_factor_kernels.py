@@ -46,3 +46,45 @@ def test_small_fronts_match_oracle(leaf_area, small_max, precision):
         solve_and_check(pl, nx, ny, [random_grid_csc(nx, ny, s) for s in (7, 8)], precision, 1e-8)
     finally:
         fdfd.factor_tuning()
+
+
+# panels in registers at every workgroup width (separators of up to 45, 109, 230, 300 and 530 rows: one to
+# eight waves in FP64 and, past 512 rows, the global-memory panel; sixteen waves in FP32), last panels of
+# fewer than 32 columns, one panel and two per step
+@pytest.mark.parametrize("deep", [0, fdfd.NO_DEEP])
+@pytest.mark.parametrize("precision", [G.FP64, G.FP32])
+@pytest.mark.parametrize("nx,ny", [(61, 45), (131, 109)])
+def test_register_panels_match_oracle(nx, ny, precision, deep):
+    say("register panels", nx, ny, precision, deep)
+    pl = fdfd.Plan(nx, ny, small_max=24)
+    m1, m2 = smooth_model(nx, ny, seed=9)
+    fdfd.factor_tuning(0, 0, deep)
+    try:
+        solve_and_check(pl, nx, ny, [oracle_system(G.AC, nx, ny, 8, 10.0, 6.0, m1, m2)[1], random_grid_csc(nx, ny, 5)],
+                        precision, 1e-8, sys=2)
+    finally:
+        fdfd.factor_tuning()
+
+
+@pytest.mark.parametrize("precision", [G.FP64, G.FP32])
+@pytest.mark.parametrize("nx,ny", [(300, 230), (341, 307), (561, 531)])
+def test_wide_register_panels_residual(nx, ny, precision):
+    """Larger separators: the residual of the solution (FP64, from the values), on random
+    matrices, whose pivoting moves rows between the waves' slots."""
+    say("wide register panels", nx, ny, precision)
+    pl = fdfd.Plan(nx, ny)
+    c = random_grid_csc(nx, ny, 3)
+    vals = dev((c[2] + 1j * c[3])[None, :])
+    rng = np.random.default_rng(1)
+    B = dev(rng.standard_normal((5, nx * ny)) + 1j * rng.standard_normal((5, nx * ny)))
+    fdfd.factor_tuning(0, 0, fdfd.NO_DEEP)
+    try:
+        F = pl.factor(vals, precision)
+    finally:
+        fdfd.factor_tuning()
+    assert F.singular()[0] == 0
+    X, it, rr = F.solve_refine(0, B, tol=1e-12, max_iter=30)
+    R = pl.residual(vals[0], B, X).cpu().numpy()
+    say("  iterations", it, "relres", rr)
+    assert rr <= 1e-12
+    assert np.max(np.linalg.norm(R, axis=1) / np.linalg.norm(B.cpu().numpy(), axis=1)) <= 1e-11
