@@ -306,22 +306,66 @@ def _factors(plan, ws, physics, dh, freqs, m1, m2, precision, **kw):
 
 # ---- shot panels and workflows ---------------------------------------------------
 
+def _rows(k):
+    """Grid rows as an int32 cuda tensor."""
+    import torch
+    return torch.as_tensor(np.asarray(k, np.int32), device="cuda")
+
+
+def _spikes(k, amp, B, stream=None):
+    """The point-source panel of rows k (int32 cuda) into B [len(k), n]."""
+    check(lib().gfdfd_spike_panel(B.shape[1], B.shape[0], _ptr(k), amp.real, amp.imag, _ptr(B), _stream(stream)),
+          "gfdfd_spike_panel")
+
+
 def spike_panel(n, ksrc, amp, stream=None):
     import torch
-    k = torch.as_tensor(np.asarray(ksrc, np.int32), device="cuda")
     B = torch.empty((len(ksrc), n), dtype=torch.complex128, device="cuda")
-    check(lib().gfdfd_spike_panel(n, len(ksrc), _ptr(k), amp.real, amp.imag, _ptr(B), _stream(stream)),
-          "gfdfd_spike_panel")
+    _spikes(_rows(ksrc), amp, B, stream)
     return B
 
 
-def sample(X, krec, stream=None):
+def _sample(X, k, stream=None):
     import torch
     nshots, n = X.shape
-    k = torch.as_tensor(np.asarray(krec, np.int32), device="cuda")
-    P = torch.empty((nshots, len(krec)), dtype=torch.complex64, device="cuda")
-    check(lib().gfdfd_sample(n, nshots, len(krec), _ptr(k), _ptr(X), _ptr(P), _stream(stream)), "gfdfd_sample")
+    P = torch.empty((nshots, len(k)), dtype=torch.complex64, device="cuda")
+    check(lib().gfdfd_sample(n, nshots, len(k), _ptr(k), _ptr(X), _ptr(P), _stream(stream)), "gfdfd_sample")
     return P
+
+
+def sample(X, krec, stream=None):
+    return _sample(X, _rows(krec), stream)
+
+
+# Frequencies whose panels are solved together: as many as keep the group's
+# right-hand sides within this many entries (2 GiB).  A batched solve of one
+# frequency's panel leaves most of the device idle in the upper levels of the
+# tree (801x201, 4 frequencies of 80 shots: one gradient 28.1 ms frequency by
+# frequency, 19.4 together), while a panel of this size fills it by itself, so
+# larger problems keep the memory of one frequency at a time.
+_GROUP_ENTRIES = 1 << 27
+
+
+def _groups(nfreq, nrhs, n):
+    """Index lists of the frequencies solved together (at most 64, the library's batch limit)."""
+    g = max(1, min(64, _GROUP_ENTRIES // max(1, nrhs * n)))
+    return [list(range(f, min(f + g, nfreq))) for f in range(0, nfreq, g)]
+
+
+def _solve_group(F, sel, B, precision, tol, max_iter, sys=0):
+    """Solutions of the frequencies sel on B [len(sel), nrhs, n], with their iterations and residuals."""
+    if precision == FP64 and tol is None:
+        return F.solve_batch(sel, B, sys=sys), [0] * len(sel), [float("nan")] * len(sel)
+    return F.solve_refine_batch(sel, B, sys=sys, tol=tol, max_iter=max_iter)
+
+
+def _source_panels(sel, n, k, amps, out=None):
+    """Point-source panels [len(sel), len(k), n] of the frequencies sel, amps per frequency."""
+    import torch
+    B = torch.empty((len(sel), len(k), n), dtype=torch.complex128, device="cuda") if out is None else out
+    for i, f in enumerate(sel):
+        _spikes(k, amps[f], B[i])
+    return B
 
 
 def adjoint_sources(n, krec, pcal, pobs, dh, stream=None):
@@ -338,15 +382,21 @@ def residual_sources(n, krec, pcal, pobs, dh, misfit=1, stf_inv=0, rtm=False, st
     takes the observed data as the residual.  Returns (adjoint panel [nshots, n]
     complex128, per-shot sum |res|^2 float64, per-shot estimate complex64)."""
     import torch
+    B = torch.empty((pcal.shape[0], n), dtype=torch.complex128, device="cuda")
+    l2, stf = _residual_sources(_rows(krec), pcal, pobs, dh, misfit, stf_inv, rtm, B, stream)
+    return B, l2, stf
+
+
+def _residual_sources(k, pcal, pobs, dh, misfit, stf_inv, rtm, B, stream=None):
+    """residual_sources for receiver rows k (int32 cuda) into the adjoint panel B [nshots, n]."""
+    import torch
     nshots, ntr = pcal.shape
-    k = torch.as_tensor(np.asarray(krec, np.int32), device="cuda")
-    B = torch.empty((nshots, n), dtype=torch.complex128, device="cuda")
     l2 = torch.empty(nshots, dtype=torch.float64, device="cuda")
     stf = torch.empty(nshots, dtype=torch.complex64, device="cuda")
-    check(lib().gfdfd_residual_sources(n, nshots, ntr, _ptr(k), _ptr(pcal.contiguous()), _ptr(pobs.contiguous()), dh,
-                                       int(misfit), int(stf_inv), int(bool(rtm)), _ptr(B), _ptr(l2), _ptr(stf),
-                                       _stream(stream)), "gfdfd_residual_sources")
-    return B, l2, stf
+    check(lib().gfdfd_residual_sources(B.shape[1], nshots, ntr, _ptr(k), _ptr(pcal.contiguous()),
+                                       _ptr(pobs.contiguous()), dh, int(misfit), int(stf_inv), int(bool(rtm)), _ptr(B),
+                                       _ptr(l2), _ptr(stf), _stream(stream)), "gfdfd_residual_sources")
+    return l2, stf
 
 
 def forward_shots(plan, physics, dh, freqs, m1, m2, ksrc, krec=None, npml=0, a0_pml=90.0, s=0.0, free_surf=0,
@@ -359,19 +409,16 @@ def forward_shots(plan, physics, dh, freqs, m1, m2, ksrc, krec=None, npml=0, a0_
     F, vals = _factors(plan, ws, physics, dh, freqs, m1, m2, precision, s=s, npml=npml, a0_pml=a0_pml,
                        free_surf=free_surf)
     data, fields, its, res = [], [], [], []
-    for f, fr in enumerate(freqs):
-        B = spike_panel(plan.n, ksrc, source_amp(physics, fr, s, dh, wavelet))
-        if precision == FP64 and tol is None:
-            X = F.solve(f, B)
-            it, rr = 0, float("nan")
-        else:
-            X, it, rr = F.solve_refine(f, B, tol=tol, max_iter=max_iter)
-        its.append(it)
-        res.append(rr)
+    amps = [source_amp(physics, fr, s, dh, wavelet) for fr in freqs]
+    k, kr = _rows(ksrc), None if krec is None else _rows(krec)
+    for sel in _groups(len(freqs), len(k), plan.n):
+        X, it, rr = _solve_group(F, sel, _source_panels(sel, plan.n, k, amps), precision, tol, max_iter)
+        its += it
+        res += rr
         if krec is not None:
-            data.append(sample(X, krec))
+            data += [_sample(X[i], kr) for i in range(len(sel))]
         if keep_fields:
-            fields.append(X)
+            fields += [X[i] for i in range(len(sel))]
     return dict(data=None if krec is None else data, fields=fields, iters=its, relres=res, factors=F, vals=vals)
 
 
@@ -391,20 +438,19 @@ def hessian_shin(plan, physics, dh, freqs, m1, m2, ksrc, npml=0, a0_pml=90.0, s=
                     free_surf=free_surf)
     h1 = torch.zeros(n, dtype=torch.float64, device="cuda")
     h2 = torch.zeros(n, dtype=torch.float64, device="cuda")
-    for f, fr in enumerate(freqs):
-        B = spike_panel(n, ksrc, source_amp(physics, fr, s, dh, wavelet))
-        if precision == FP64 and tol is None:
-            U = F.solve(f, B)
-        else:
-            U, _, _ = F.solve_refine(f, B, tol=tol, max_iter=max_iter)
-        if physics == AC:
-            o2 = omega2_grad_ac(fr, s)
-            check(lib().gfdfd_hess_shin_ac(n, len(ksrc), o2.ctypes.data, _ptr(U), _ptr(m1.contiguous()),
-                                           _ptr(m2.contiguous()), _ptr(h1), _stream(None)), "gfdfd_hess_shin_ac")
-        else:
-            o2, om = omega(TE, fr, s)
-            check(lib().gfdfd_hess_shin_te(n, len(ksrc), om.ctypes.data, o2.ctypes.data, _ptr(U), _ptr(h1),
-                                           _ptr(h2), _stream(None)), "gfdfd_hess_shin_te")
+    amps = [source_amp(physics, fr, s, dh, wavelet) for fr in freqs]
+    k = _rows(ksrc)
+    for sel in _groups(len(freqs), len(k), n):
+        Us, _, _ = _solve_group(F, sel, _source_panels(sel, n, k, amps), precision, tol, max_iter)
+        for U, f in zip(Us, sel):
+            if physics == AC:
+                o2 = omega2_grad_ac(freqs[f], s)
+                check(lib().gfdfd_hess_shin_ac(n, len(ksrc), o2.ctypes.data, _ptr(U), _ptr(m1.contiguous()),
+                                               _ptr(m2.contiguous()), _ptr(h1), _stream(None)), "gfdfd_hess_shin_ac")
+            else:
+                o2, om = omega(TE, freqs[f], s)
+                check(lib().gfdfd_hess_shin_te(n, len(ksrc), om.ctypes.data, o2.ctypes.data, _ptr(U), _ptr(h1),
+                                               _ptr(h2), _stream(None)), "gfdfd_hess_shin_te")
     return h1 if physics == AC else (h1, h2)
 
 
@@ -425,23 +471,22 @@ def hessian_gn(plan, physics, dh, freqs, m1, m2, ksrc, krec, npml=0, a0_pml=90.0
                     free_surf=free_surf)
     hess = torch.zeros(n, dtype=torch.float64, device="cuda")
     h2 = torch.zeros(n, dtype=torch.float64, device="cuda")
-    for f, fr in enumerate(freqs):
-        B = spike_panel(n, ksrc, source_amp(physics, fr, s, dh, wavelet))
-        BG = spike_panel(n, krec, complex(np.float32(1.0) / np.float32(np.float32(dh) * np.float32(dh))))
-        if precision == FP64 and tol is None:
-            U, GR = F.solve(f, B), F.solve(f, BG)
-        else:
-            U, _, _ = F.solve_refine(f, B, tol=tol, max_iter=max_iter)
-            GR, _, _ = F.solve_refine(f, BG, tol=tol, max_iter=max_iter)
-        if physics == AC:
-            o2 = omega2_grad_ac(fr, s)
-            check(lib().gfdfd_hess_gn_ac(n, len(ksrc), len(krec), o2.ctypes.data, _ptr(U), _ptr(GR),
-                                         _ptr(m1.contiguous()), _ptr(m2.contiguous()), _ptr(hess), _stream(None)),
-                  "gfdfd_hess_gn_ac")
-        else:
-            o2, om = omega(TE, fr, s)
-            check(lib().gfdfd_hess_gn_te(n, len(ksrc), len(krec), om.ctypes.data, o2.ctypes.data, _ptr(U),
-                                         _ptr(GR), _ptr(hess), _ptr(h2), _stream(None)), "gfdfd_hess_gn_te")
+    amps = [source_amp(physics, fr, s, dh, wavelet) for fr in freqs]
+    green = [complex(np.float32(1.0) / np.float32(np.float32(dh) * np.float32(dh)))] * len(freqs)
+    k, kr = _rows(ksrc), _rows(krec)
+    for sel in _groups(len(freqs), max(len(k), len(kr)), n):
+        Us, _, _ = _solve_group(F, sel, _source_panels(sel, n, k, amps), precision, tol, max_iter)
+        GRs, _, _ = _solve_group(F, sel, _source_panels(sel, n, kr, green), precision, tol, max_iter)
+        for U, GR, f in zip(Us, GRs, sel):
+            if physics == AC:
+                o2 = omega2_grad_ac(freqs[f], s)
+                check(lib().gfdfd_hess_gn_ac(n, len(ksrc), len(krec), o2.ctypes.data, _ptr(U), _ptr(GR),
+                                             _ptr(m1.contiguous()), _ptr(m2.contiguous()), _ptr(hess), _stream(None)),
+                      "gfdfd_hess_gn_ac")
+            else:
+                o2, om = omega(TE, freqs[f], s)
+                check(lib().gfdfd_hess_gn_te(n, len(ksrc), len(krec), om.ctypes.data, o2.ctypes.data, _ptr(U),
+                                             _ptr(GR), _ptr(hess), _ptr(h2), _stream(None)), "gfdfd_hess_gn_te")
     return hess if physics == AC else (hess, h2)
 
 
@@ -493,16 +538,16 @@ def objective(plan, physics, dh, freqs, m1, m2, ksrc, krec, pobs, npml=0, a0_pml
     n = plan.n
     F, _ = _factors(plan, ws, physics, dh, freqs, m1, m2, precision, s=s, npml=npml, a0_pml=a0_pml,
                     free_surf=free_surf)
-    l2 = 0.0
-    for f, fr in enumerate(freqs):
-        B = spike_panel(n, ksrc, source_amp(physics, fr, s, dh, wavelet))
-        if precision == FP64 and tol is None:
-            U = F.solve(f, B)
-        else:
-            U, _, _ = F.solve_refine(f, B, tol=tol, max_iter=max_iter)
-        _, l2s, _ = residual_sources(n, krec, sample(U, krec), pobs[f], dh, misfit=misfit, stf_inv=stf_inv)
-        l2 += float(l2s.sum())
-    return 0.5 * l2
+    l2 = []
+    amps = [source_amp(physics, fr, s, dh, wavelet) for fr in freqs]
+    k, kr = _rows(ksrc), _rows(krec)
+    for sel in _groups(len(freqs), len(k), n):
+        B = _source_panels(sel, n, k, amps)
+        Us, _, _ = _solve_group(F, sel, B, precision, tol, max_iter)
+        for i, f in enumerate(sel):
+            l2s, _ = _residual_sources(kr, _sample(Us[i], kr), pobs[f], dh, misfit, stf_inv, False, B[i])
+            l2.append(l2s.sum())
+    return 0.5 * sum(float(v) for v in l2)
 
 
 def initial_step(direction, m, eps_scale):
@@ -792,34 +837,34 @@ def grad_obj(plan, physics, dh, freqs, m1, m2, ksrc, krec, pobs, npml=0, a0_pml=
     tp = None if taper is None else taper.device_struct(len(ksrc))
     g1 = torch.zeros(n, dtype=torch.float64, device="cuda")
     g2 = torch.zeros(n, dtype=torch.float64, device="cuda")
-    l2 = 0.0
+    if physics not in (AC, TE):
+        raise ValueError("SH has no gradient path in the reference (src/germaine.c:112-120)")
+    l2 = []
     adj_sys = 0 if physics == AC else 2      # AC solves with M (grad_obj_AC.c:147), TE with M^T (grad_obj_TE.c:149)
-    k = torch.as_tensor(np.asarray(krec, np.int32), device="cuda")
-    for f, fr in enumerate(freqs):
-        B = spike_panel(n, ksrc, source_amp(physics, fr, s, dh, wavelet))
-        if precision == FP64 and tol is None:
-            U = F.solve(f, B)
-        else:
-            U, _, _ = F.solve_refine(f, B, tol=tol, max_iter=max_iter)
-        pcal = sample(U, krec)
-        BA, l2s, stf = residual_sources(n, krec, pcal, pobs[f], dh, misfit=misfit, stf_inv=stf_inv, rtm=rtm)
-        l2 += float(l2s.sum())
-        if precision == FP64 and tol is None:
-            LAM = F.solve(f, BA, sys=adj_sys)
-        else:
-            LAM, _, _ = F.solve_refine(f, BA, sys=adj_sys, tol=tol, max_iter=max_iter)
-        nshots = len(ksrc)
-        tpp = None if tp is None else C.byref(tp)
-        if physics == AC:
-            o2 = omega2_grad_ac(fr, s)
-            check(lib().gfdfd_grad_ac_taper(n, nshots, o2.ctypes.data, _ptr(U), _ptr(LAM), _ptr(m1.contiguous()),
-                                            _ptr(m2.contiguous()), _ptr(stf), tpp, _ptr(g1), _stream(None)),
-                  "gfdfd_grad_ac_taper")
-        elif physics == TE:
-            o2, om = omega(TE, fr, s)
-            check(lib().gfdfd_grad_te_taper(n, nshots, om.ctypes.data, o2.ctypes.data, _ptr(U), _ptr(LAM), _ptr(stf),
-                                            tpp, _ptr(g1), _ptr(g2), _stream(None)), "gfdfd_grad_te_taper")
-        else:
-            raise ValueError("SH has no gradient path in the reference (src/germaine.c:112-120)")
+    amps = [source_amp(physics, fr, s, dh, wavelet) for fr in freqs]
+    k, kr = _rows(ksrc), _rows(krec)
+    nshots = len(k)
+    tpp = None if tp is None else C.byref(tp)
+    for sel in _groups(len(freqs), nshots, n):
+        B = _source_panels(sel, n, k, amps)
+        Us, _, _ = _solve_group(F, sel, B, precision, tol, max_iter)
+        stfs = []
+        for i, f in enumerate(sel):              # the adjoint panels take the sources' place
+            l2s, stf = _residual_sources(kr, _sample(Us[i], kr), pobs[f], dh, misfit, stf_inv, rtm, B[i])
+            l2.append(l2s.sum())
+            stfs.append(stf)
+        LAMs, _, _ = _solve_group(F, sel, B, precision, tol, max_iter, sys=adj_sys)
+        for i, f in enumerate(sel):
+            U, LAM, stf = Us[i], LAMs[i], stfs[i]
+            if physics == AC:
+                o2 = omega2_grad_ac(freqs[f], s)
+                check(lib().gfdfd_grad_ac_taper(n, nshots, o2.ctypes.data, _ptr(U), _ptr(LAM), _ptr(m1.contiguous()),
+                                                _ptr(m2.contiguous()), _ptr(stf), tpp, _ptr(g1), _stream(None)),
+                      "gfdfd_grad_ac_taper")
+            else:
+                o2, om = omega(TE, freqs[f], s)
+                check(lib().gfdfd_grad_te_taper(n, nshots, om.ctypes.data, o2.ctypes.data, _ptr(U), _ptr(LAM),
+                                                _ptr(stf), tpp, _ptr(g1), _ptr(g2), _stream(None)),
+                      "gfdfd_grad_te_taper")
     grad = g1 if physics == AC else (g1, g2)
-    return 0.5 * l2, grad
+    return 0.5 * sum(float(v) for v in l2), grad
