@@ -218,29 +218,41 @@ __global__ void __launch_bounds__(256) k_fwd_gather(const cx<T> *__restrict__ X,
 }
 
 // ---- panel substitutions on MFMA -------------------------------------------
-// Shared-memory layout of the block kernels (dynamic): right-hand-side block
-// [BK][64] re/im, then the A tile [BK][64] re/im, whose space the diagonal
-// block [BK][BK+1] complex shares: the diagonal product runs (and ends with a
+// Tile shapes of the block kernels: a workgroup covers RT rows x CT right-hand
+// sides, a wave WR x WC of them in 16 x 16 blocks.  A tile's products take one
+// compute unit's matrix cores as long as its RT x CT says (128 x 64 x 64 complex
+// in FP64: 13 us), so a launch with fewer tiles than compute units waits on
+// that; panel_tile (below) picks the small shape there.
+template <int RT_, int CT_, int WR_, int WC_>
+struct BlkTile {
+    static constexpr int RT = RT_, CT = CT_, WR = WR_, WC = WC_;
+    static constexpr int NW = (RT / WR) * (CT / WC), NT = 64 * NW, NA = WR / 16, NB = WC / 16;
+    static_assert(RT >= 64 && RT % WR == 0 && CT % WC == 0 && WR % 16 == 0 && WC % 16 == 0, "tile shape");
+    static __device__ __forceinline__ int wave_row(int w) { return w / (CT / WC) * WR; }
+    static __device__ __forceinline__ int wave_col(int w) { return w % (CT / WC) * WC; }
+};
+// Shared memory of a block kernel (dynamic): right-hand-side block [BK][CT]
+// re/im, then the A tile [BK][RT] re/im, whose space the diagonal block
+// [BK][BK+1] complex shares: the diagonal product runs (and ends with a
 // barrier) before the A tile is stored.
-// RT: rows of the A tile (64, or 128 for the forward block kernel's 8 waves).
-template <typename T, int RT = 64>
+template <typename T, class C>
 struct BlkSmem {
     T *Ar, *Ai, *Yr, *Yi;
     cx<T> *D;
     __device__ BlkSmem(unsigned char *raw) {
         Yr = reinterpret_cast<T *>(raw);
-        Yi = Yr + BK * 64;
-        Ar = Yi + BK * 64;
-        Ai = Ar + BK * RT;
+        Yi = Yr + BK * C::CT;
+        Ar = Yi + BK * C::CT;
+        Ai = Ar + BK * C::RT;
         D = reinterpret_cast<cx<T> *>(Ar);
     }
 };
 static_assert(sizeof(cx<double>) * BK * (BK + 1) <= 2 * sizeof(double) * BK * 64 &&
                   sizeof(cx<float>) * BK * (BK + 1) <= 2 * sizeof(float) * BK * 64,
               "the diagonal block fits in the A tile's space");
-template <typename T, int RT = 64>
+template <typename T, class C>
 constexpr size_t blk_smem_bytes() {
-    return sizeof(T) * (2 * BK * 64 + 2 * BK * RT);
+    return sizeof(T) * (2 * BK * C::CT + 2 * BK * C::RT);
 }
 
 // element (i, t) of the operator that solves 32-row diagonal block b0 in the
@@ -269,63 +281,54 @@ __device__ __forceinline__ cx<T> dop_fix(cx<T> v, int i, int t, int nb, bool fwd
     return cj ? cx<T>{v.x, -v.y} : v;
 }
 
-// acc = A[64 x kb] * Y[kb x 64] from LDS (4 waves in 2x2, 32x32 each), or
-// acc += that when accumulate; column sub-tiles at or beyond ncol (right-hand
-// sides past the end) are skipped
-template <typename T, int RT = 64>
-__device__ __forceinline__ void mma_tile(const BlkSmem<T, RT> &s, int kb, int ncol, cacc3<T> (&c)[2][2],
-                                         bool accumulate = false) {
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, wr = (w >> 1) * 32, wc = (w & 1) * 32;
+// c += A[RT x kb] * Y[kb x CT] from LDS; column sub-tiles at or beyond ncol
+// (right-hand sides past the end) are skipped
+template <typename T, class C>
+__device__ __forceinline__ void mma_tile(const T *Ar, const T *Ai, const T *Yr, const T *Yi, int kb, int ncol,
+                                         cacc3<T> (&c)[C::NA][C::NB]) {
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, wr = C::wave_row(w), wc = C::wave_col(w);
     const int lr = lane & 15, lk = lane >> 4;
-    if (!accumulate)
-        for (int a = 0; a < 2; a++)
-            for (int b = 0; b < 2; b++) c[a][b].zero();
     const int kend = (kb + 3) & ~3;
     for (int kk = 0; kk < kend; kk += 4) {
         const int k = kk + lk;
-        T ar[2], ai[2], br[2], bi[2];
-        for (int a = 0; a < 2; a++) {
-            ar[a] = s.Ar[k * RT + wr + a * 16 + lr];
-            ai[a] = s.Ai[k * RT + wr + a * 16 + lr];
+        T ar[C::NA], ai[C::NA], br[C::NB], bi[C::NB];
+#pragma unroll
+        for (int a = 0; a < C::NA; a++) {
+            ar[a] = Ar[k * C::RT + wr + a * 16 + lr];
+            ai[a] = Ai[k * C::RT + wr + a * 16 + lr];
         }
-        for (int b = 0; b < 2; b++) {
-            br[b] = s.Yr[k * 64 + wc + b * 16 + lr];
-            bi[b] = s.Yi[k * 64 + wc + b * 16 + lr];
+#pragma unroll
+        for (int b = 0; b < C::NB; b++) {
+            br[b] = Yr[k * C::CT + wc + b * 16 + lr];
+            bi[b] = Yi[k * C::CT + wc + b * 16 + lr];
         }
-        for (int b = 0; b < 2; b++)
+#pragma unroll
+        for (int b = 0; b < C::NB; b++)
             if (wc + b * 16 < ncol)
-                for (int a = 0; a < 2; a++) c[a][b].mma(ar[a], ai[a], br[b], bi[b], br[b] + bi[b]);
+#pragma unroll
+                for (int a = 0; a < C::NA; a++) c[a][b].mma(ar[a], ai[a], br[b], bi[b], br[b] + bi[b]);
     }
 }
-
-// rows [row0, row0+64) of w (below rowend) -= acc, right-hand sides [r0, r0+64)
-template <typename T>
-__device__ __forceinline__ void sub_tile(cx<T> *w, int nrhs, int row0, int rowend, int r0,
-                                         typename mfma_t<T>::acc (&cr)[2][2], typename mfma_t<T>::acc (&ci)[2][2]) {
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, wr = (wv >> 1) * 32, wc = (wv & 1) * 32;
-    const int lr = lane & 15, lk = lane >> 4;
-    for (int a = 0; a < 2; a++)
-        for (int b = 0; b < 2; b++)
-            for (int v = 0; v < 4; v++) {
-                const int row = row0 + wr + a * 16 + mfma_t<T>::row(lk, v), col = r0 + wc + b * 16 + lr;
-                if (row < rowend && col < nrhs) {
-                    cx<T> &g = w[(int64_t)row * nrhs + col];
-                    g.x -= cr[a][b][v];
-                    g.y -= ci[a][b][v];
-                }
-            }
+template <typename T, class C>
+__device__ __forceinline__ void zero_tile(cacc3<T> (&c)[C::NA][C::NB]) {
+#pragma unroll
+    for (int a = 0; a < C::NA; a++)
+#pragma unroll
+        for (int b = 0; b < C::NB; b++) c[a][b].zero();
 }
 
-// the same, with the tile's current values of w loaded beforehand into c
-// (load_tile), so the read-modify-write waits on nothing
-template <typename T>
-__device__ __forceinline__ void load_tile(const cx<T> *w, int nrhs, int row0, int rowend, int r0, cx<T> (&c)[2][2][4]) {
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, wr = (wv >> 1) * 32, wc = (wv & 1) * 32;
+// the workgroup's tile of w (rows from row0 below rowend, right-hand sides from
+// r0) loaded into c beforehand, and stored as c - acc: the read-modify-write
+// then waits on nothing
+template <typename T, class C>
+__device__ __forceinline__ void load_tile(const cx<T> *w, int nrhs, int row0, int rowend, int r0,
+                                          cx<T> (&c)[C::NA][C::NB][4]) {
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, wr = C::wave_row(wv), wc = C::wave_col(wv);
     const int lr = lane & 15, lk = lane >> 4;
 #pragma unroll
-    for (int a = 0; a < 2; a++)
+    for (int a = 0; a < C::NA; a++)
 #pragma unroll
-        for (int b = 0; b < 2; b++)
+        for (int b = 0; b < C::NB; b++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 // unconditional: entries outside read w[0] and are never used
@@ -333,15 +336,16 @@ __device__ __forceinline__ void load_tile(const cx<T> *w, int nrhs, int row0, in
                 c[a][b][v] = w[row < rowend && col < nrhs ? (int64_t)row * nrhs + col : 0];
             }
 }
-template <typename T>
+template <typename T, class C>
 __device__ __forceinline__ void sub_tile_from(cx<T> *w, int nrhs, int row0, int rowend, int r0,
-                                              const cx<T> (&c)[2][2][4], const cacc3<T> (&acc)[2][2]) {
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, wr = (wv >> 1) * 32, wc = (wv & 1) * 32;
+                                              const cx<T> (&c)[C::NA][C::NB][4],
+                                              const cacc3<T> (&acc)[C::NA][C::NB]) {
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, wr = C::wave_row(wv), wc = C::wave_col(wv);
     const int lr = lane & 15, lk = lane >> 4;
 #pragma unroll
-    for (int a = 0; a < 2; a++)
+    for (int a = 0; a < C::NA; a++)
 #pragma unroll
-        for (int b = 0; b < 2; b++)
+        for (int b = 0; b < C::NB; b++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const int row = row0 + wr + a * 16 + mfma_t<T>::row(lk, v), col = r0 + wc + b * 16 + lr;
@@ -350,339 +354,235 @@ __device__ __forceinline__ void sub_tile_from(cx<T> *w, int nrhs, int row0, int 
             }
 }
 
-// Y[0:nb] = D Y[0:nb] in LDS (D: the block operator, zero outside nb x nb):
-// waves 0-3 own 16 rows x 32 right-hand sides each (further waves only meet
-// the barriers)
-template <typename T, int RT = 64>
-__device__ __forceinline__ void diag_apply(const BlkSmem<T, RT> &s, int nb, int ncol) {
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, rw = (w >> 1) * 16, wc = (w & 1) * 32;
-    const int lr = lane & 15, lk = lane >> 4;
-    cacc3<T> c[2];
-    for (int b = 0; b < 2; b++) c[b].zero();
-    const bool act = RT == 64 || w < 4;
-    const int kend = act ? (nb + 3) & ~3 : 0;
-    for (int kk = 0; kk < kend; kk += 4) {
-        const int k = kk + lk;
-        const cx<T> a = s.D[(rw + lr) * (BK + 1) + k];
-        for (int b = 0; b < 2; b++)
-            if (wc + b * 16 < ncol) {
-                const T br = s.Yr[k * 64 + wc + b * 16 + lr], bi = s.Yi[k * 64 + wc + b * 16 + lr];
-                c[b].mma(a.x, a.y, br, bi, br + bi);
+// D Y[0:kb] in LDS (D: 32 rows in the diagonal block's layout, row i at
+// D[i * (BK + 1)]), one 16 x 16 tile at a time over the waves.  SUB: Z -= D Y on
+// the first nb rows of another block Z; else Y = D Y in place.  Ends with a
+// barrier.
+template <typename T, class C, bool SUB>
+__device__ __forceinline__ void diag_product(const cx<T> *D, T *Yr, T *Yi, T *Zr, T *Zi, int kb, int nb, int ncol) {
+    constexpr int NTL = 2 * (C::CT / 16), PW = (NTL + C::NW - 1) / C::NW;   // 16 x 16 tiles, tiles per wave
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, lr = lane & 15, lk = lane >> 4;
+    cacc3<T> c[PW];
+    const int kend = (kb + 3) & ~3;
+#pragma unroll
+    for (int q = 0; q < PW; q++) {
+        c[q].zero();
+        const int t = w + q * C::NW, rw = (t & 1) * 16, wc = (t >> 1) * 16;
+        if (t < NTL && wc < ncol)
+            for (int kk = 0; kk < kend; kk += 4) {
+                const int k = kk + lk;
+                const cx<T> a = D[(rw + lr) * (BK + 1) + k];
+                const T br = Yr[k * C::CT + wc + lr], bi = Yi[k * C::CT + wc + lr];
+                c[q].mma(a.x, a.y, br, bi, br + bi);
             }
     }
-    __syncthreads();
-    if (act)
-        for (int b = 0; b < 2; b++)
+    if (!SUB) __syncthreads();   // every wave has read Y
+#pragma unroll
+    for (int q = 0; q < PW; q++) {
+        const int t = w + q * C::NW, rw = (t & 1) * 16, wc = (t >> 1) * 16;
+        if (t < NTL)
+#pragma unroll
             for (int v = 0; v < 4; v++) {
-                const int row = rw + mfma_t<T>::row(lk, v), col = wc + b * 16 + lr;
+                const int row = rw + mfma_t<T>::row(lk, v), at = row * C::CT + wc + lr;
                 if (row < nb) {
-                    s.Yr[row * 64 + col] = c[b].re(v);
-                    s.Yi[row * 64 + col] = c[b].im(v);
+                    if (SUB) {
+                        Zr[at] -= c[q].re(v);
+                        Zi[at] -= c[q].im(v);
+                    } else {
+                        Yr[at] = c[q].re(v);
+                        Yi[at] = c[q].im(v);
+                    }
                 }
             }
-    __syncthreads();
-}
-
-// forward block b0 of every front of a level: y_b = Dop_bb w_b (written to X
-// by the row-tile-0 workgroup), then rows [b0+nb, m) of W -= Lop[:, b] y_b.
-// Everything the workgroup reads -- the diagonal operator, y's rows, the
-// operator block below and the rows it updates -- is requested before the
-// first barrier, so the workgroup waits on global memory once.
-// grid: (row tiles, fronts, right-hand-side tiles)
-constexpr int kFwdRT = 128;   // rows per forward block workgroup (8 waves of 32x32 tiles)
-template <typename T>
-__global__ void __launch_bounds__(4 * kFwdRT) k_fwd_blk(const cx<T> *__restrict__ arena, int64_t fstride,
-                                                 const FrontDev *__restrict__ fronts, const int *__restrict__ list,
-                                                 cx<T> *__restrict__ X, cx<T> *__restrict__ W, int n, int64_t wstride,
-                                                 int nrhs, int rt, int b0, int trans, int cj, Sel sel) {
-    constexpr int RT = kFwdRT, NT = 4 * RT;
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    BlkSmem<T, RT> s(smem_raw);
-    const FrontDev F = fronts[list[blockIdx.y]];
-    if (F.p <= b0) return;
-    const int m = F.m, nb = min(BK, F.p - b0), tid = threadIdx.x;
-    const int row0 = b0 + nb + blockIdx.x * RT;
-    if (blockIdx.x > 0 && row0 >= m) return;
-    const bool upd = row0 < m;
-    const int z = blockIdx.z / rt, r0 = (blockIdx.z - z * rt) * 64, ncol = min(64, nrhs - r0);
-    const cx<T> *G = arena + sel.f[z] * fstride + F.buf_off;
-    X += (int64_t)sel.s[z] * n * nrhs;
-    cx<T> *w = W + sel.s[z] * wstride + F.fv_off * nrhs;
-    auto Lop = [&](int i, int t) { return trans ? ld(G + t + (int64_t)i * m, cj) : ld(G + i + (int64_t)t * m, cj); };
-    cx<T> wold[2][2][4];
-    if (upd) load_tile<T>(w, nrhs, row0, m, r0, wold);
-    {
-        cx<T> dv[BK * BK / NT], yv[BK * 64 / NT], av[BK * RT / NT];
-#pragma unroll
-        for (int u = 0; u < BK * BK / NT; u++) {
-            const int e = tid + NT * u, i = e % BK, t = e / BK;
-            dv[u] = (i < nb && t < nb) ? dop(G, m, b0, i, t, true, trans, cj) : cx<T>{T(0), T(0)};
-        }
-#pragma unroll
-        for (int u = 0; u < BK * 64 / NT; u++) {
-            const int e = tid + NT * u, k = e >> 6, j = e & 63;
-            yv[u] = (k < nb && j < ncol) ? w[(int64_t)(b0 + k) * nrhs + r0 + j] : cx<T>{T(0), T(0)};
-        }
-#pragma unroll
-        for (int u = 0; u < BK * RT / NT; u++) {
-            const int e = tid + NT * u;
-            int k, i;
-            if (!trans) { i = e % RT; k = e / RT; }        // column-major L: coalesced along rows
-            else { k = e % BK; i = e / BK; }               // U^T: coalesced along k
-            av[u] = (upd && k < nb && row0 + i < m) ? Lop(row0 + i, b0 + k) : cx<T>{T(0), T(0)};
-        }
-#pragma unroll
-        for (int u = 0; u < BK * BK / NT; u++) {
-            const int e = tid + NT * u;
-            s.D[(e % BK) * (BK + 1) + e / BK] = dv[u];
-        }
-#pragma unroll
-        for (int u = 0; u < BK * 64 / NT; u++) {
-            const int e = tid + NT * u;
-            s.Yr[e] = yv[u].x;
-            s.Yi[e] = yv[u].y;
-        }
-        __syncthreads();
-        diag_apply<T, RT>(s, nb, ncol);   // ends with a barrier: D's space is free
-#pragma unroll
-        for (int u = 0; u < BK * RT / NT; u++) {
-            const int e = tid + NT * u;
-            int k, i;
-            if (!trans) { i = e % RT; k = e / RT; }
-            else { k = e % BK; i = e / BK; }
-            s.Ar[k * RT + i] = av[u].x;
-            s.Ai[k * RT + i] = av[u].y;
-        }
     }
     __syncthreads();
-    if (blockIdx.x == 0)
-        for (int e = tid; e < nb * 64; e += NT) {
-            int k = e >> 6, j = e & 63;
-            if (j < ncol) X[(int64_t)(F.pos0 + b0 + k) * nrhs + r0 + j] = {s.Yr[e], s.Yi[e]};
-        }
-    if (!upd) return;
-    cacc3<T> acc[2][2];
-    mma_tile<T, RT>(s, nb, ncol, acc);
-    sub_tile_from<T>(w, nrhs, row0, m, r0, wold, acc);
 }
 
-// Y1[0:nb1] -= L Y0[0:kb] in LDS (L: nb1 x kb in the diagonal block's layout,
-// row i at L[i * (BK + 1)]): waves 0-3 own 16 rows x 32 right-hand sides each,
-// as in diag_apply; ends with a barrier
-template <typename T>
-__device__ __forceinline__ void blk_couple(const cx<T> *L, const T *Y0r, const T *Y0i, T *Y1r, T *Y1i, int kb, int nb1,
-                                           int ncol) {
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, rw = (w >> 1) * 16, wc = (w & 1) * 32;
-    const int lr = lane & 15, lk = lane >> 4;
-    cacc3<T> c[2];
-    for (int b = 0; b < 2; b++) c[b].zero();
-    const bool act = w < 4;
-    const int kend = act ? (kb + 3) & ~3 : 0;
-    for (int kk = 0; kk < kend; kk += 4) {
-        const int k = kk + lk;
-        const cx<T> a = L[(rw + lr) * (BK + 1) + k];
-        for (int b = 0; b < 2; b++)
-            if (wc + b * 16 < ncol) {
-                const T br = Y0r[k * 64 + wc + b * 16 + lr], bi = Y0i[k * 64 + wc + b * 16 + lr];
-                c[b].mma(a.x, a.y, br, bi, br + bi);
-            }
-    }
-    if (act)
-        for (int b = 0; b < 2; b++)
-            for (int v = 0; v < 4; v++) {
-                const int row = rw + mfma_t<T>::row(lk, v), col = wc + b * 16 + lr;
-                if (row < nb1) {
-                    Y1r[row * 64 + col] -= c[b].re(v);
-                    Y1i[row * 64 + col] -= c[b].im(v);
-                }
-            }
-    __syncthreads();
-}
-
-// forward blocks b0 and b0 + 32 of every front of a level in one launch:
-// y_0 = Dop_0 w_0, w_1 -= Lop[b1, b0] y_0, y_1 = Dop_1 w_1 (both written to X
-// by the row-tile-0 workgroup), then rows [b0 + 64, m) of W -= Lop[:, b0:b0+64]
-// [y_0; y_1] as one depth-64 update -- the rows below pass through memory once
-// per two blocks instead of once per block.  Every operand but the second block
-// column of Lop is requested before the first barrier; that one is loaded
-// during the first column's products.  A front with a single block left takes
-// the first half alone.  LDS: [Y1 | Y0 | A tile], the A tile's space holding
-// Dop_0, Lop[b1, b0] and Dop_1 in turn.  grid: (row tiles, fronts, rhs tiles)
-template <typename T>
+// The two 32-pivot blocks of rows [b0, b0 + 64) of every front of a level, in
+// one launch.  Forward: y_0 = Dop_0 w_0, w_1 -= Lop[b1, b0] y_0, y_1 = Dop_1 w_1
+// (both to X by the row-tile-0 workgroup), then the rows below W -= Lop y as one
+// depth-64 update, so those rows pass through memory once per two blocks.
+// Backward the mirror image: the upper block first, the update on rows
+// [0, b0).  Every operand but the second block column of the update is
+// requested before the first barrier, unconditionally (entries outside read a
+// valid address of the front or panel and are masked when staged); that one is
+// loaded during the first column's products.  A front with a single block left
+// takes the first half alone.  LDS: [second Y | first Y | A tile], the A tile's
+// space holding the diagonal blocks and their coupling in turn.
+// grid: (row tiles, fronts, rhs tiles x slots)
+template <typename T, class C>
 constexpr size_t blk2_smem_bytes() {
-    return sizeof(T) * 2 * BK * 64 + blk_smem_bytes<T, kFwdRT>();
+    return sizeof(T) * 2 * BK * C::CT + blk_smem_bytes<T, C>();
 }
-template <typename T>
-__global__ void __launch_bounds__(4 * kFwdRT) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 1))) k_fwd_blk2(const cx<T> *__restrict__ arena, int64_t fstride,
-                                                  const FrontDev *__restrict__ fronts, const int *__restrict__ list,
-                                                  cx<T> *__restrict__ X, cx<T> *__restrict__ W, int n, int64_t wstride,
-                                                  int nrhs, int rt, int b0, int trans, int cj, Sel sel) {
-    constexpr int RT = kFwdRT, NT = 4 * RT;
+template <typename T, class C, bool FWD>
+__global__ void __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && C::NT == 512 ? 4 : 1)))
+k_blk2(const cx<T> *__restrict__ arena, int64_t fstride, const FrontDev *__restrict__ fronts,
+       const int *__restrict__ list, cx<T> *__restrict__ X, cx<T> *__restrict__ W, int n, int64_t wstride, int nrhs,
+       int rt, int b0, int trans, int cj, Sel sel) {
+    constexpr int RT = C::RT, CT = C::CT, NT = C::NT;
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    BlkSmem<T, RT> s0(smem_raw + sizeof(T) * 2 * BK * 64);   // Y0 and the A tile
-    BlkSmem<T, RT> s1 = s0;                                   // Y1 and the same A tile
-    s1.Yr = reinterpret_cast<T *>(smem_raw);
-    s1.Yi = s1.Yr + BK * 64;
+    BlkSmem<T, C> s(smem_raw + sizeof(T) * 2 * BK * CT);   // the first block's Y and the A tile
+    T *Sr = reinterpret_cast<T *>(smem_raw), *Si = Sr + BK * CT;   // the second block's Y
     const FrontDev F = fronts[list[blockIdx.y]];
     if (F.p <= b0) return;
-    const int m = F.m, nb0 = min(BK, F.p - b0), nb1 = max(0, min(BK, F.p - b0 - BK)), tid = threadIdx.x;
-    const int row0 = b0 + nb0 + nb1 + blockIdx.x * RT;
-    if (blockIdx.x > 0 && row0 >= m) return;
-    const bool upd = row0 < m;
-    const int z = blockIdx.z / rt, r0 = (blockIdx.z - z * rt) * 64, ncol = min(64, nrhs - r0);
+    const int m = F.m, tid = threadIdx.x;
+    const int lo = min(BK, F.p - b0), hi = max(0, min(BK, F.p - b0 - BK));
+    const int f0 = FWD || hi == 0 ? b0 : b0 + BK, s0 = FWD ? b0 + BK : b0;   // first and second block
+    const int nf = FWD || hi == 0 ? lo : hi, ns = hi == 0 ? 0 : FWD ? hi : lo;
+    const int row0 = (FWD ? b0 + lo + hi : 0) + blockIdx.x * RT, rowend = FWD ? m : b0;
+    if (blockIdx.x > 0 && row0 >= rowend) return;
+    const bool upd = row0 < rowend;
+    const int z = blockIdx.z / rt, r0 = (blockIdx.z - z * rt) * CT, ncol = min(CT, nrhs - r0);
     const cx<T> *G = arena + sel.f[z] * fstride + F.buf_off;
     X += (int64_t)sel.s[z] * n * nrhs;
     cx<T> *w = W + sel.s[z] * wstride + F.fv_off * nrhs;
-    cx<T> wold[2][2][4];
-    if (upd) load_tile<T>(w, nrhs, row0, m, r0, wold);
-    cx<T> d0[BK * BK / NT], d1[BK * BK / NT], l10[BK * BK / NT], y0v[BK * 64 / NT], y1v[BK * 64 / NT],
-        av[BK * RT / NT];
-    // every load is unconditional (entries outside read a valid address of
-    // the front or panel), and its masks are applied when it is staged, so
-    // the whole set is in flight at once
-    auto lop_at = [&](int i, int t) { return trans ? t + (int64_t)i * m : i + (int64_t)t * m; };
+    cx<T> wold[C::NA][C::NB][4];
+    if (upd) load_tile<T, C>(w, nrhs, row0, rowend, r0, wold);
+    constexpr int PD = BK * BK / NT, PY = BK * CT / NT, PA = BK * RT / NT;
+    cx<T> df[PD], ds[PD], cs[PD], yf[PY], ys[PY], av[PA];
+    auto op_at = [&](int i, int t) { return trans ? t + (int64_t)i * m : i + (int64_t)t * m; };
 #pragma unroll
-    for (int u = 0; u < BK * BK / NT; u++) {
+    for (int u = 0; u < PD; u++) {
         const int e = tid + NT * u, i = e % BK, t = e / BK;
-        d0[u] = dop_raw(G, m, b0, i, t, nb0, trans);
-        d1[u] = dop_raw(G, m, b0 + BK, i, t, nb1, trans);
-        l10[u] = G[i < nb1 && t < nb0 ? lop_at(b0 + BK + i, b0 + t) : 0];
+        df[u] = dop_raw(G, m, f0, i, t, nf, trans);
+        ds[u] = dop_raw(G, m, ns ? s0 : f0, i, t, ns, trans);
+        cs[u] = G[i < ns && t < nf ? op_at(s0 + i, f0 + t) : 0];
     }
-    const int64_t wc0 = r0;
 #pragma unroll
-    for (int u = 0; u < BK * 64 / NT; u++) {
-        const int e = tid + NT * u, k = e >> 6, j = e & 63;
-        y0v[u] = w[k < nb0 && j < ncol ? (int64_t)(b0 + k) * nrhs + wc0 + j : 0];
-        y1v[u] = w[k < nb1 && j < ncol ? (int64_t)(b0 + BK + k) * nrhs + wc0 + j : 0];
+    for (int u = 0; u < PY; u++) {
+        const int e = tid + NT * u, k = e / CT, j = e % CT;
+        yf[u] = w[k < nf && j < ncol ? (int64_t)(f0 + k) * nrhs + r0 + j : 0];
+        ys[u] = w[k < ns && j < ncol ? (int64_t)(s0 + k) * nrhs + r0 + j : 0];
     }
     int akb = 0;   // columns of the A tile in av
     auto load_a = [&](int c0, int kb) {   // the A tile of block column c0 (kb columns) into av
         akb = kb;
 #pragma unroll
-        for (int u = 0; u < BK * RT / NT; u++) {
+        for (int u = 0; u < PA; u++) {
             const int e = tid + NT * u;
             int k, i;
-            if (!trans) { i = e % RT; k = e / RT; }        // column-major L: coalesced along rows
-            else { k = e % BK; i = e / BK; }               // U^T: coalesced along k
-            av[u] = G[upd && k < kb && row0 + i < m ? lop_at(row0 + i, c0 + k) : 0];
+            if (!trans) { i = e % RT; k = e / RT; }        // column-major: coalesced along rows
+            else { k = e % BK; i = e / BK; }               // transposed: coalesced along k
+            av[u] = G[upd && k < kb && row0 + i < rowend ? op_at(row0 + i, c0 + k) : 0];
         }
     };
     auto stage_a = [&]() {
 #pragma unroll
-        for (int u = 0; u < BK * RT / NT; u++) {
+        for (int u = 0; u < PA; u++) {
             const int e = tid + NT * u;
             int k, i;
             if (!trans) { i = e % RT; k = e / RT; }
             else { k = e % BK; i = e / BK; }
-            const bool in = upd && k < akb && row0 + i < m;
-            s0.Ar[k * RT + i] = in ? av[u].x : T(0);
-            s0.Ai[k * RT + i] = in ? (cj ? -av[u].y : av[u].y) : T(0);
+            const bool in = upd && k < akb && row0 + i < rowend;
+            s.Ar[k * RT + i] = in ? av[u].x : T(0);
+            s.Ai[k * RT + i] = in ? (cj ? -av[u].y : av[u].y) : T(0);
         }
     };
-    auto stage_d = [&](const cx<T>(&v)[BK * BK / NT], int nb) {   // a diagonal block operator
+    auto stage_d = [&](const cx<T>(&v)[PD], int nb) {   // a diagonal block operator
 #pragma unroll
-        for (int u = 0; u < BK * BK / NT; u++) {
+        for (int u = 0; u < PD; u++) {
             const int e = tid + NT * u;
-            s0.D[(e % BK) * (BK + 1) + e / BK] = dop_fix(v[u], e % BK, e / BK, nb, true, trans, cj);
+            s.D[(e % BK) * (BK + 1) + e / BK] = dop_fix(v[u], e % BK, e / BK, nb, FWD, trans, cj);
         }
     };
-    load_a(b0, nb0);
-    stage_d(d0, nb0);
+    load_a(f0, nf);
+    stage_d(df, nf);
 #pragma unroll
-    for (int u = 0; u < BK * 64 / NT; u++) {
-        const int e = tid + NT * u, k = e >> 6, j = e & 63;
-        const bool in0 = k < nb0 && j < ncol, in1 = k < nb1 && j < ncol;
-        s0.Yr[e] = in0 ? y0v[u].x : T(0);
-        s0.Yi[e] = in0 ? y0v[u].y : T(0);
-        s1.Yr[e] = in1 ? y1v[u].x : T(0);
-        s1.Yi[e] = in1 ? y1v[u].y : T(0);
+    for (int u = 0; u < PY; u++) {
+        const int e = tid + NT * u, k = e / CT, j = e % CT;
+        const bool inf = k < nf && j < ncol, ins = k < ns && j < ncol;
+        s.Yr[e] = inf ? yf[u].x : T(0);
+        s.Yi[e] = inf ? yf[u].y : T(0);
+        Sr[e] = ins ? ys[u].x : T(0);
+        Si[e] = ins ? ys[u].y : T(0);
     }
     __syncthreads();
-    diag_apply<T, RT>(s0, nb0, ncol);   // y_0; ends with a barrier
-    if (nb1 > 0) {
+    diag_product<T, C, false>(s.D, s.Yr, s.Yi, nullptr, nullptr, nf, nf, ncol);   // y of the first block
+    if (ns > 0) {
 #pragma unroll
-        for (int u = 0; u < BK * BK / NT; u++) {   // Lop[b1, b0]
+        for (int u = 0; u < PD; u++) {   // the coupling block
             const int e = tid + NT * u, i = e % BK, t = e / BK;
-            const cx<T> v = l10[u];
-            s0.D[i * (BK + 1) + t] = i < nb1 && t < nb0 ? (cj ? cx<T>{v.x, -v.y} : v) : cx<T>{T(0), T(0)};
+            const cx<T> v = cs[u];
+            s.D[i * (BK + 1) + t] = i < ns && t < nf ? (cj ? cx<T>{v.x, -v.y} : v) : cx<T>{T(0), T(0)};
         }
         __syncthreads();
-        blk_couple<T>(s0.D, s0.Yr, s0.Yi, s1.Yr, s1.Yi, nb0, nb1, ncol);   // w_1 -= L10 y_0
-        stage_d(d1, nb1);
+        diag_product<T, C, true>(s.D, s.Yr, s.Yi, Sr, Si, nf, ns, ncol);   // second block -= coupling y
+        stage_d(ds, ns);
         __syncthreads();
-        diag_apply<T, RT>(s1, nb1, ncol);   // y_1
+        diag_product<T, C, false>(s.D, Sr, Si, nullptr, nullptr, ns, ns, ncol);   // y of the second block
     }
     if (blockIdx.x == 0)
-        for (int e = tid; e < (nb0 + nb1) * 64; e += NT) {
-            const int k = e >> 6, j = e & 63;
+        for (int e = tid; e < (nf + ns) * CT; e += NT) {
+            const int k = e / CT, j = e % CT;
             if (j < ncol) {
-                const int kk = k < nb0 ? k : k - nb0;
-                const T *yr = k < nb0 ? s0.Yr : s1.Yr, *yi = k < nb0 ? s0.Yi : s1.Yi;
-                X[(int64_t)(F.pos0 + b0 + k) * nrhs + r0 + j] = {yr[kk * 64 + j], yi[kk * 64 + j]};
+                const int kk = k < nf ? k : k - nf, row = k < nf ? f0 + k : s0 + kk;
+                const T *yr = k < nf ? s.Yr : Sr, *yi = k < nf ? s.Yi : Si;
+                X[(int64_t)(F.pos0 + row) * nrhs + r0 + j] = {yr[kk * CT + j], yi[kk * CT + j]};
             }
         }
     if (!upd) return;
-    stage_a();   // the diagonal blocks' space is free (diag_apply ended with a barrier)
+    stage_a();   // the diagonal blocks' space is free (diag_product ended with a barrier)
     __syncthreads();
-    if (nb1 > 0) load_a(b0 + BK, nb1);   // in flight during the first column's products
-    cacc3<T> acc[2][2];
-    mma_tile<T, RT>(s0, nb0, ncol, acc);
-    if (nb1 > 0) {
+    if (ns > 0) load_a(s0, ns);   // in flight during the first column's products
+    cacc3<T> acc[C::NA][C::NB];
+    zero_tile<T, C>(acc);
+    mma_tile<T, C>(s.Ar, s.Ai, s.Yr, s.Yi, nf, ncol, acc);
+    if (ns > 0) {
         __syncthreads();   // the first column's tile is no longer read
         stage_a();
         __syncthreads();
-        mma_tile<T, RT>(s1, nb1, ncol, acc, true);
+        mma_tile<T, C>(s.Ar, s.Ai, Sr, Si, ns, ncol, acc);
     }
-    sub_tile_from<T>(w, nrhs, row0, m, r0, wold, acc);
+    sub_tile_from<T, C>(w, nrhs, row0, rowend, r0, wold, acc);
 }
 
 // backward, ancestors: W[f][0:p] = y1 - Uop12 x2, x2 gathered from X at the
 // contribution positions.  The positions are staged in LDS first (after the
 // block tiles, m - p ints), so each 32-column chunk of Uop12 and x2 is one
 // memory round trip, loaded into registers while the previous chunk's products
-// run.  grid: (row tiles over p, fronts, rhs tiles)
+// run.  grid: (row tiles over p, fronts, rhs tiles x slots)
 constexpr int kContribRowsMax = 16384;   // m - p of any front on this path
-template <typename T>
-__global__ void __launch_bounds__(256) k_bwd_contrib(const cx<T> *__restrict__ arena, int64_t fstride,
-                                                     const FrontDev *__restrict__ fronts, const int *__restrict__ list,
-                                                     const int *__restrict__ idx, const cx<T> *__restrict__ X,
-                                                     cx<T> *__restrict__ W, int n, int64_t wstride, int nrhs, int rt,
-                                                     int trans, int cj, Sel sel) {
+template <typename T, class C>
+__global__ void __launch_bounds__(C::NT) k_bwd_contrib(const cx<T> *__restrict__ arena, int64_t fstride,
+                                                       const FrontDev *__restrict__ fronts,
+                                                       const int *__restrict__ list, const int *__restrict__ idx,
+                                                       const cx<T> *__restrict__ X, cx<T> *__restrict__ W, int n,
+                                                       int64_t wstride, int nrhs, int rt, int trans, int cj, Sel sel) {
+    constexpr int RT = C::RT, CT = C::CT, NT = C::NT;
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    BlkSmem<T> s(smem_raw);
-    int *srow = reinterpret_cast<int *>(smem_raw + blk_smem_bytes<T>());
+    BlkSmem<T, C> s(smem_raw);
+    int *srow = reinterpret_cast<int *>(smem_raw + blk_smem_bytes<T, C>());
     const FrontDev F = fronts[list[blockIdx.y]];
     const int m = F.m, p = F.p, tid = threadIdx.x;
-    const int row0 = blockIdx.x * 64;
+    const int row0 = blockIdx.x * RT;
     if (row0 >= p) return;
-    for (int e = tid; e < m - p; e += 256) srow[e] = idx[F.idx_off + p + e];
+    for (int e = tid; e < m - p; e += NT) srow[e] = idx[F.idx_off + p + e];
     __syncthreads();
-    const int z = blockIdx.z / rt, r0 = (blockIdx.z - z * rt) * 64, ncol = min(64, nrhs - r0);
+    const int z = blockIdx.z / rt, r0 = (blockIdx.z - z * rt) * CT, ncol = min(CT, nrhs - r0);
     const cx<T> *G = arena + sel.f[z] * fstride + F.buf_off;
     X += (int64_t)sel.s[z] * n * nrhs;
     cx<T> *w = W + sel.s[z] * wstride + F.fv_off * nrhs;
     auto uop_at = [&](int i, int t) { return trans ? t + (int64_t)i * m : i + (int64_t)t * m; };
-    cacc3<T> acc[2][2];
-    for (int a = 0; a < 2; a++)
-        for (int b = 0; b < 2; b++) acc[a][b].zero();
-    constexpr int PER = BK * 64 / 256;
-    cx<T> av[PER], yv[PER];
+    cacc3<T> acc[C::NA][C::NB];
+    zero_tile<T, C>(acc);
+    constexpr int PA = BK * RT / NT, PY = BK * CT / NT;
+    cx<T> av[PA], yv[PY];
     // a chunk's operands, loaded unconditionally (entries outside read a valid
     // address and are zeroed when staged), so they stay in flight during the
     // previous chunk's products
     auto fetch = [&](int s0) {
         const int kb = min(BK, m - s0);
 #pragma unroll
-        for (int u = 0; u < PER; u++) {
-            const int e = tid + 256 * u;
+        for (int u = 0; u < PA; u++) {
+            const int e = tid + NT * u;
             int k, i;
-            if (!trans) { i = e & 63; k = e >> 6; }
+            if (!trans) { i = e % RT; k = e / RT; }
             else { k = e % BK; i = e / BK; }
             av[u] = G[k < kb && row0 + i < p ? uop_at(row0 + i, s0 + k) : 0];
         }
 #pragma unroll
-        for (int u = 0; u < PER; u++) {
-            const int e = tid + 256 * u, k = e >> 6, j = e & 63;
+        for (int u = 0; u < PY; u++) {
+            const int e = tid + NT * u, k = e / CT, j = e % CT;
             const bool in = k < kb && j < ncol;
             yv[u] = X[(int64_t)srow[s0 - p + (in ? k : 0)] * nrhs + (in ? r0 + j : 0)];
         }
@@ -692,108 +592,30 @@ __global__ void __launch_bounds__(256) k_bwd_contrib(const cx<T> *__restrict__ a
         const int kb = min(BK, m - s0);
         __syncthreads();   // the previous chunk's operands are no longer read
 #pragma unroll
-        for (int u = 0; u < PER; u++) {
-            const int e = tid + 256 * u;
+        for (int u = 0; u < PA; u++) {
+            const int e = tid + NT * u;
             int k, i;
-            if (!trans) { i = e & 63; k = e >> 6; }
+            if (!trans) { i = e % RT; k = e / RT; }
             else { k = e % BK; i = e / BK; }
             const bool ain = k < kb && row0 + i < p;
-            s.Ar[k * 64 + i] = ain ? av[u].x : T(0);
-            s.Ai[k * 64 + i] = ain ? (cj ? -av[u].y : av[u].y) : T(0);
-            const int ky = e >> 6, j = e & 63;
-            const bool yin = ky < kb && j < ncol;
+            s.Ar[k * RT + i] = ain ? av[u].x : T(0);
+            s.Ai[k * RT + i] = ain ? (cj ? -av[u].y : av[u].y) : T(0);
+        }
+#pragma unroll
+        for (int u = 0; u < PY; u++) {
+            const int e = tid + NT * u, k = e / CT, j = e % CT;
+            const bool yin = k < kb && j < ncol;
             s.Yr[e] = yin ? yv[u].x : T(0);
             s.Yi[e] = yin ? yv[u].y : T(0);
         }
         __syncthreads();
         if (s0 + BK < m) fetch(s0 + BK);   // in flight during this chunk's products
-        mma_tile<T>(s, kb, ncol, acc, true);
+        mma_tile<T, C>(s.Ar, s.Ai, s.Yr, s.Yi, kb, ncol, acc);
     }
     // w[0:p] = y1 - accumulated product
-    cx<T> y1[2][2][4];
-    load_tile<T>(X + (int64_t)F.pos0 * nrhs, nrhs, row0, p, r0, y1);
-    sub_tile_from<T>(w, nrhs, row0, p, r0, y1, acc);
-}
-
-// backward block b0 (blocks from the bottom): x_b = Dop_bb z_b (to X by the
-// row-tile-0 workgroup), then rows [0, b0) of W -= Uop[:, b] x_b
-template <typename T>
-__global__ void __launch_bounds__(256) k_bwd_blk(const cx<T> *__restrict__ arena, int64_t fstride,
-                                                 const FrontDev *__restrict__ fronts, const int *__restrict__ list,
-                                                 cx<T> *__restrict__ X, cx<T> *__restrict__ W, int n, int64_t wstride,
-                                                 int nrhs, int rt, int b0, int trans, int cj, Sel sel) {
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    BlkSmem<T> s(smem_raw);
-    const FrontDev F = fronts[list[blockIdx.y]];
-    if (F.p <= b0) return;
-    const int m = F.m, nb = min(BK, F.p - b0), tid = threadIdx.x;
-    const int row0 = blockIdx.x * 64;
-    if (blockIdx.x > 0 && row0 >= b0) return;
-    const int z = blockIdx.z / rt, r0 = (blockIdx.z - z * rt) * 64, ncol = min(64, nrhs - r0);
-    const cx<T> *G = arena + sel.f[z] * fstride + F.buf_off;
-    X += (int64_t)sel.s[z] * n * nrhs;
-    cx<T> *w = W + sel.s[z] * wstride + F.fv_off * nrhs;
-    auto uop_at = [&](int i, int t) { return trans ? t + (int64_t)i * m : i + (int64_t)t * m; };
-    const bool upd = row0 < b0;
-    // every load before the first barrier, unconditional (entries outside read
-    // a valid address of the front or panel; masks applied when staged)
-    cx<T> wold[2][2][4];
-    if (upd) load_tile<T>(w, nrhs, row0, b0, r0, wold);
-    {
-        cx<T> dv[BK * BK / 256], yv[BK * 64 / 256], av[BK * 64 / 256];
-#pragma unroll
-        for (int u = 0; u < BK * BK / 256; u++) {
-            const int e = tid + 256 * u, i = e % BK, t = e / BK;
-            dv[u] = dop_raw(G, m, b0, i, t, nb, trans);
-        }
-#pragma unroll
-        for (int u = 0; u < BK * 64 / 256; u++) {
-            const int e = tid + 256 * u, k = e >> 6, j = e & 63;
-            yv[u] = w[k < nb && j < ncol ? (int64_t)(b0 + k) * nrhs + r0 + j : 0];
-        }
-#pragma unroll
-        for (int u = 0; u < BK * 64 / 256; u++) {
-            const int e = tid + 256 * u;
-            int k, i;
-            if (!trans) { i = e & 63; k = e >> 6; }
-            else { k = e % BK; i = e / BK; }
-            av[u] = G[upd && k < nb && row0 + i < b0 ? uop_at(row0 + i, b0 + k) : 0];
-        }
-#pragma unroll
-        for (int u = 0; u < BK * BK / 256; u++) {
-            const int e = tid + 256 * u;
-            s.D[(e % BK) * (BK + 1) + e / BK] = dop_fix(dv[u], e % BK, e / BK, nb, false, trans, cj);
-        }
-#pragma unroll
-        for (int u = 0; u < BK * 64 / 256; u++) {
-            const int e = tid + 256 * u, k = e >> 6, j = e & 63;
-            const bool in = k < nb && j < ncol;
-            s.Yr[e] = in ? yv[u].x : T(0);
-            s.Yi[e] = in ? yv[u].y : T(0);
-        }
-        __syncthreads();
-        diag_apply<T>(s, nb, ncol);   // ends with a barrier: D's space is free
-#pragma unroll
-        for (int u = 0; u < BK * 64 / 256; u++) {
-            const int e = tid + 256 * u;
-            int k, i;
-            if (!trans) { i = e & 63; k = e >> 6; }
-            else { k = e % BK; i = e / BK; }
-            const bool in = upd && k < nb && row0 + i < b0;
-            s.Ar[k * 64 + i] = in ? av[u].x : T(0);
-            s.Ai[k * 64 + i] = in ? (cj ? -av[u].y : av[u].y) : T(0);
-        }
-    }
-    __syncthreads();
-    if (blockIdx.x == 0)
-        for (int e = tid; e < nb * 64; e += 256) {
-            int k = e >> 6, j = e & 63;
-            if (j < ncol) X[(int64_t)(F.pos0 + b0 + k) * nrhs + r0 + j] = {s.Yr[e], s.Yi[e]};
-        }
-    if (!upd) return;
-    cacc3<T> acc[2][2];
-    mma_tile<T>(s, nb, ncol, acc);
-    sub_tile_from<T>(w, nrhs, row0, b0, r0, wold, acc);
+    cx<T> y1[C::NA][C::NB][4];
+    load_tile<T, C>(X + (int64_t)F.pos0 * nrhs, nrhs, row0, p, r0, y1);
+    sub_tile_from<T, C>(w, nrhs, row0, p, r0, y1, acc);
 }
 
 // ---- fused per-front substitutions (fronts whose panel fits in LDS) ---------
@@ -3039,6 +2861,28 @@ inline WaveLaunch small_launch(int nfr, int nrhs, int nslots, size_t lds, int ma
     return {dim3(((nfr + 7) / 8) * 8 * rtg, nslots), dim3(64 * wpg), (lds + 15) & ~size_t(15), rtg, 0};
 }
 
+// Tile shapes of the block kernels and the rule between them.  A big tile reads
+// each operator entry once per 64 right-hand sides but holds one compute unit
+// for its whole product; when the big tiles would not fill the 256 compute
+// units the launch lasts as long as one of them, so the work goes out in tiles
+// of 16 right-hand sides, and of 32 while they would fill the units less than
+// twice (128-row tiles).  One FP64 solve pass: 403x207, 2 frequencies x 31
+// right-hand sides, 1.37 ms with big tiles only and 1.01 by the rule; 801x201, 4 x
+// 80, 4.69 and 4.33; at 1601x401, 4 x 200, 16-wide tiles up to 1024 big
+// ones cost 5.51 ms of forward blocks against 5.23.
+using TileFwd = BlkTile<128, 64, 32, 32>;
+using TileBwd = BlkTile<64, 64, 32, 32>;
+using TileMid = BlkTile<64, 32, 16, 32>;
+using TileSmall = BlkTile<64, 16, 16, 16>;
+template <class Big, typename Fn>
+void with_tile(int rows, int nfr, int nrhs, int ns, Fn &&launch) {
+    const int64_t wgs =
+        (int64_t)std::max(1, (rows + Big::RT - 1) / Big::RT) * nfr * ((nrhs + Big::CT - 1) / Big::CT) * ns;
+    if (wgs <= 256) launch(TileSmall{});
+    else if (wgs <= 512 * (128 / Big::RT)) launch(TileMid{});
+    else launch(Big{});
+}
+
 #define FUSED_LAUNCH(kern, T, rw, grid, lds, st, ...)                                                   \
     do {                                                                                              \
         if ((rw) == 64) hipLaunchKernelGGL((kern<T, 64>), grid, dim3(256), lds, st, __VA_ARGS__);     \
@@ -3058,15 +2902,21 @@ void set_smem_attrs() {
                                   hipFuncAttributeMaxDynamicSharedMemorySize, big));
     GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_bwd_vec<T>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, big));
-    const int blk = (int)blk_smem_bytes<T>();
-    GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_fwd_blk<T>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)blk_smem_bytes<T, kFwdRT>()));
-    GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_fwd_blk2<T>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)blk2_smem_bytes<T>()));
-    GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_bwd_blk<T>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, blk));
-    GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_bwd_contrib<T>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, blk + 4 * kContribRowsMax));
+    auto blk_attrs = [](auto c, bool big) {
+        using C = decltype(c);
+        const int b2 = (int)blk2_smem_bytes<T, C>(), bc = (int)blk_smem_bytes<T, C>() + 4 * kContribRowsMax;
+        GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_blk2<T, C, true>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, b2));
+        GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_blk2<T, C, false>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, b2));
+        if (!big)
+            GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_bwd_contrib<T, C>),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, bc));
+    };
+    blk_attrs(TileFwd{}, true);
+    blk_attrs(TileBwd{}, false);
+    blk_attrs(TileSmall{}, false);
+    blk_attrs(TileMid{}, false);
     // the refinement step's per-wave column sums: up to 64 KB at 1024 right-hand sides
     GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_ir_step<T>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, kIrWaves * 8 * 1024));
@@ -3132,8 +2982,6 @@ void sweeps(const Factors<T> &F, const Sel &in, int sys, int nrhs, cx<T> *Xp, cx
     const bool trans = sys != 0, cj = sys == 1;
     const int64_t wstride = pl.fv_rows * (int64_t)nrhs;
     const double nr = nreal, nz = ns, es = sizeof(cx<T>);
-    const size_t blk = blk_smem_bytes<T>();
-    const int rt = (nrhs + 63) / 64;
     const bool prof = prof_enabled();
     for (int l = 0; l < pl.nlevels; l++) {
         if (dp.n_all[l] == 0) continue;
@@ -3189,24 +3037,21 @@ void sweeps(const Factors<T> &F, const Sel &in, int sys, int nrhs, cx<T> *Xp, cx
                                wstride, nrhs, in);
         }
         const int pmax = dp.pmax_all[l];
-        static const bool one_block = std::getenv("GFDFD_FWD_BLK1") != nullptr;
-        for (int b0 = 0; b0 < pmax; b0 += one_block ? BK : 2 * BK) {
+        for (int b0 = 0; b0 < pmax; b0 += 2 * BK) {
             // factor entries of the block columns, and the panel rows below them read and written
-            const int nbk = one_block || b0 + BK >= pmax ? 1 : 2;
+            const int nbk = b0 + BK >= pmax ? 1 : 2;
             double fe = 0.0;
             if (prof)
                 for (int q = 0; q < nbk; q++) fe += c.fwd_blk_elems[b0 / BK + q];
             ProfScope ps(K_FWD_BLK, st, nz * 8.0 * nr * fe, nz * (fe + 2.0 * nr * fe / (nbk * BK)) * es);
-            const int tiles = std::max(1, (dp.mmax_all[l] - b0 - 1) / kFwdRT + 1);
-            const size_t fblk = blk_smem_bytes<T, kFwdRT>();
-            if (one_block)
-                hipLaunchKernelGGL(k_fwd_blk<T>, dim3(tiles, nfr, rt * ns), dim3(4 * kFwdRT), fblk, st, F.arena,
+            with_tile<TileFwd>(dp.mmax_all[l] - b0, nfr, nrhs, ns, [&](auto t) {
+                using C = decltype(t);
+                const int tiles = std::max(1, (dp.mmax_all[l] - b0 - 1) / C::RT + 1), rt = (nrhs + C::CT - 1) / C::CT;
+                const size_t lds = blk2_smem_bytes<T, C>();
+                hipLaunchKernelGGL((k_blk2<T, C, true>), dim3(tiles, nfr, rt * ns), dim3(C::NT), lds, st, F.arena,
                                    F.fstride, dp.fronts, dp.lv_all[l], Xp, Wp, n, wstride, nrhs, rt, b0, (int)trans,
                                    (int)cj, in);
-            else
-                hipLaunchKernelGGL(k_fwd_blk2<T>, dim3(tiles, nfr, rt * ns), dim3(4 * kFwdRT), blk2_smem_bytes<T>(), st,
-                                   F.arena, F.fstride, dp.fronts, dp.lv_all[l], Xp, Wp, n, wstride, nrhs, rt, b0,
-                                   (int)trans, (int)cj, in);
+            });
         }
     }
     for (int l = pl.nlevels - 1; l >= 0; l--) {
@@ -3248,17 +3093,28 @@ void sweeps(const Factors<T> &F, const Sel &in, int sys, int nrhs, cx<T> *Xp, cx
             ProfScope ps(K_BWD_CONTRIB, st, nz * 8.0 * nr * c.contrib_elems,
                          nz * (c.contrib_elems + (c.sum_m + c.sum_p) * nr) * es);
             if (dp.mmax_all[l] > kContribRowsMax) throw std::logic_error("front too large for the contribution kernel");
-            hipLaunchKernelGGL(k_bwd_contrib<T>, dim3((pmax + 63) / 64, nfr, rt * ns), dim3(256),
-                               blk + 4 * (size_t)dp.mmax_all[l], st, F.arena,
-                               F.fstride, dp.fronts, dp.lv_all[l], dp.idx, Xp, Wp, n, wstride, nrhs, rt, (int)trans,
-                               (int)cj, in);
+            with_tile<TileBwd>(pmax, nfr, nrhs, ns, [&](auto t) {
+                using C = decltype(t);
+                const int rt = (nrhs + C::CT - 1) / C::CT;
+                const size_t lds = blk_smem_bytes<T, C>() + 4 * (size_t)dp.mmax_all[l];
+                hipLaunchKernelGGL((k_bwd_contrib<T, C>), dim3((pmax + C::RT - 1) / C::RT, nfr, rt * ns), dim3(C::NT),
+                                   lds, st, F.arena, F.fstride, dp.fronts, dp.lv_all[l], dp.idx, Xp, Wp, n, wstride, nrhs, rt, (int)trans, (int)cj,
+                                   in);
+            });
         }
-        for (int b0 = ((pmax - 1) / BK) * BK; b0 >= 0; b0 -= BK) {
-            const double be = prof ? c.bwd_blk_elems[b0 / BK] : 0.0;
-            ProfScope ps(K_BWD_BLK, st, nz * 8.0 * nr * be, nz * (be + 2.0 * nr * be / BK) * es);
-            const int tiles = std::max(1, (b0 + 63) / 64);
-            hipLaunchKernelGGL(k_bwd_blk<T>, dim3(tiles, nfr, rt * ns), dim3(256), blk, st, F.arena, F.fstride,
-                               dp.fronts, dp.lv_all[l], Xp, Wp, n, wstride, nrhs, rt, b0, (int)trans, (int)cj, in);
+        for (int b0 = (pmax - 1) / (2 * BK) * (2 * BK); b0 >= 0; b0 -= 2 * BK) {
+            const int nbk = b0 + BK >= pmax ? 1 : 2;
+            double be = 0.0;
+            if (prof)
+                for (int q = 0; q < nbk; q++) be += c.bwd_blk_elems[b0 / BK + q];
+            ProfScope ps(K_BWD_BLK, st, nz * 8.0 * nr * be, nz * (be + 2.0 * nr * be / (nbk * BK)) * es);
+            with_tile<TileBwd>(b0, nfr, nrhs, ns, [&](auto t) {
+                using C = decltype(t);
+                const int tiles = std::max(1, (b0 + C::RT - 1) / C::RT), rt = (nrhs + C::CT - 1) / C::CT;
+                const size_t lds = blk2_smem_bytes<T, C>();
+                hipLaunchKernelGGL((k_blk2<T, C, false>), dim3(tiles, nfr, rt * ns), dim3(C::NT), lds, st, F.arena, F.fstride, dp.fronts, dp.lv_all[l], Xp, Wp, n,
+                                   wstride, nrhs, rt, b0, (int)trans, (int)cj, in);
+            });
         }
         if (trans) {
             ProfScope ps(K_PIV_UNSWAP, st, 0.0, nz * 4.0 * c.sum_p * nr * es);

@@ -88,3 +88,26 @@ def test_wide_register_panels_residual(nx, ny, precision):
     say("  iterations", it, "relres", rr)
     assert rr <= 1e-12
     assert np.max(np.linalg.norm(R, axis=1) / np.linalg.norm(B.cpu().numpy(), axis=1)) <= 1e-11
+
+
+# panel sweeps of the multi-block levels at each tile width (16, 32 and 64 right-hand sides per workgroup, by
+# how many tiles a launch has): one column past a tile, several frequencies, single last blocks
+@pytest.mark.parametrize("sys", [0, 1, 2])
+@pytest.mark.parametrize("nf,nrhs,precision", [(1, 17, G.FP64), (3, 33, G.FP64), (8, 129, G.FP64), (3, 65, G.FP32)])
+def test_block_tiles_match_oracle(nf, nrhs, precision, sys):
+    nx, ny = 131, 109
+    say("block tiles", nf, nrhs, precision, sys)
+    pl = fdfd.Plan(nx, ny)
+    m1, m2 = smooth_model(nx, ny, seed=2)
+    mats = [oracle_system(G.AC, nx, ny, 8, 10.0, 3.0 + f, m1, m2)[1] for f in range(nf)]
+    F = pl.factor(dev(np.stack([c[2] + 1j * c[3] for c in mats])), precision)
+    rng = np.random.default_rng(nrhs)
+    B = rng.standard_normal((nf, nrhs, nx * ny)) + 1j * rng.standard_normal((nf, nrhs, nx * ny))
+    if precision == G.FP64:
+        X = F.solve_batch(list(range(nf)), dev(B), sys=sys).cpu().numpy()
+    else:
+        X = F.solve_refine_batch(list(range(nf)), dev(B), sys=sys, tol=1e-12, max_iter=30)[0].cpu().numpy()
+    cols = [0, nrhs // 2, nrhs - 1]
+    for z, c in enumerate(mats):
+        Xr, _ = O.band_solve(*c, B[z][cols].T, sys=sys, perm=O.grid_transpose_perm(nx, ny))
+        assert rel(X[z][cols], Xr.T) <= (1e-10 if precision == G.FP64 else 1e-8), z
