@@ -19,6 +19,8 @@ struct alignas(2 * sizeof(T)) cx {
 // Compact front descriptor as the kernels read it.
 struct FrontDev {
     int p, m, pos0, nchild, child_off, level;
+    int slot;   // small fronts: index of their original-entry range; blocked fronts: offset of their column pointers
+    int pad;
     int64_t buf_off, fv_off, idx_off, inv_off;
 };
 

@@ -25,7 +25,7 @@ struct DevPlan {
     int *children = nullptr, *idx = nullptr, *inv = nullptr, *perm = nullptr, *iperm = nullptr;
     int *colptr = nullptr, *rowind = nullptr;
     int64_t *tq = nullptr;                 // CSR-of-M position -> CSC index (symmetric pattern)
-    std::vector<int *> lv_small, lv_large, lv_all;
+    std::vector<int *> lv_all;
     std::vector<int> n_small, n_large, n_all, mmax_all, pmax_all;
     TileDev *tiles = nullptr;
     std::vector<std::vector<std::pair<int64_t, int>>> steps;   // [level][step] -> (offset, count)
@@ -69,18 +69,19 @@ struct DevPlan {
     int vinv_n = 0, vinv_pmax = 0;
     int vinv_rect_tiles = 0;                        // most 64 x 64 rectangle tiles of one front
     int *gsrc_id = nullptr;                         // [fv_rows][3] gather sources of front rows before pivoting
-    std::vector<FrontDev *> lv_fr;                  // per level: the level's fronts, contiguous
+    std::vector<FrontDev *> lv_fr;                  // per level: the level's fronts, contiguous (small, then blocked)
     std::vector<int> lv_children;                   // per level: 1 if any front has children
 
     // Small fronts (order <= small_max), each assembled and factored by one
-    // workgroup: a slot per front with its original entries.
-    int *slot_of = nullptr;                         // [nfronts] small-front slot, -1 for blocked fronts
+    // workgroup: a slot per front (FrontDev::slot) with its original entries.
     int64_t *small_optr = nullptr;                  // [slots + 1] ranges of the slots' original entries
     int64_t *small_oq = nullptr;                    // CSC index of each such entry
     int *small_ooff = nullptr;                      // its local offset r + c m in the front
-    // the blocked fronts' original entries, by level
-    int64_t *orig_q_large = nullptr, *orig_dst_large = nullptr;
-    std::vector<std::pair<int64_t, int64_t>> orig_large_range;   // per level [begin, end)
+    // the blocked fronts' original entries, by column: column c's are
+    // [large_cptr[slot + c], large_cptr[slot + c + 1])
+    int *large_cptr = nullptr;
+    int64_t *large_oq = nullptr;                    // CSC index of each entry
+    int *large_ooff = nullptr;                      // its local offset r + c m in the front
     std::vector<double> asm_elems_large;            // per level: entries of the blocked fronts
 
     // Small subtrees (fronts whose whole subtree has m <= small_max), which one
@@ -91,12 +92,12 @@ struct DevPlan {
     int nroots = 0, sub_mmax = 0;
     int *root_first = nullptr, *root_last = nullptr;   // [nroots] front range of each subtree
     double sub_flops = 0, sub_elems = 0;            // algorithmic counts of the launch (per frequency)
-    std::vector<int *> lv_small_rest;               // per level: small fronts outside the subtrees
+    std::vector<FrontDev *> lv_small_rest;          // per level: small fronts outside the subtrees
     std::vector<int> n_small_rest, small_mmax_rest;
     std::vector<double> small_rest_flops, small_rest_elems;   // per level: those fronts
 
     explicit DevPlan(std::shared_ptr<const Plan> p);
-    void build_small(const Plan &pl);
+    void build_small(const Plan &pl, std::vector<FrontDev> &fd);
     ~DevPlan();
     DevPlan(const DevPlan &) = delete;
     DevPlan &operator=(const DevPlan &) = delete;
@@ -109,7 +110,7 @@ struct Factors {
     int nfreq = 0;
     int64_t fstride = 0;            // arena elements per frequency
     cx<T> *arena = nullptr;         // fronts, column-major, factors in place
-    int *piv = nullptr;             // nfreq * n local row swaps
+    int *piv = nullptr;             // nfreq * n row swaps of the register panels (k_panel_finish replays them)
     int *rowperm = nullptr;         // nfreq * n: local source row of each pivot position after all swaps
     int *sing = nullptr;            // nfreq flags: zero pivot met
     int *gsrc = nullptr;            // nfreq * fv_rows * 3: gather sources after pivoting (forward sweep of M)

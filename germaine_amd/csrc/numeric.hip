@@ -30,13 +30,13 @@ namespace gfdfd {
 // ---------------------------------------------------------------------------
 // Small fronts (order <= the plan's small_max) are assembled and factored in
 // one kernel each, so every small front gets a slot with its own list of
-// original entries; the blocked fronts' entries are listed by level.
+// original entries; the blocked fronts' entries are listed by column.
 // Small subtrees: a front belongs when its order is at most small_max and all
 // its children belong (leaves included), so a whole subtree can be factored
 // by the persistent launch and the level path never waits on it.
 // Fronts are in postorder, so each maximal subtree is a contiguous range
 // ending at its root.
-void DevPlan::build_small(const Plan &pl) {
+void DevPlan::build_small(const Plan &pl, std::vector<FrontDev> &fd) {
     const int nfr = (int)pl.fronts.size();
     std::vector<char> in(nfr, 0), small(nfr, 0);
     for (const LevelPlan &L : pl.levels)
@@ -72,9 +72,18 @@ void DevPlan::build_small(const Plan &pl) {
             }
         }
     nroots = (int)first.size();
-    // original entries: the small fronts' by slot (local offsets), the rest by level
+    // original entries: the small fronts' by slot (local offsets), the blocked fronts' by column
     std::vector<std::vector<std::pair<int64_t, int>>> per_slot(nslot);
-    std::vector<std::vector<std::pair<int64_t, int64_t>>> rest(pl.nlevels);
+    std::vector<int> cptr;
+    for (int f = 0; f < nfr; f++) {
+        if (slot[f] < 0) {
+            fd[f].slot = (int)cptr.size();
+            cptr.resize(cptr.size() + pl.fronts[f].m + 1, 0);
+        } else {
+            fd[f].slot = slot[f];
+        }
+    }
+    std::vector<std::vector<std::pair<int64_t, int>>> per_col(cptr.size());
     std::vector<std::pair<int64_t, int>> starts;   // buf_off -> front
     for (int f = 0; f < nfr; f++) starts.push_back({pl.fronts[f].buf_off, f});
     std::sort(starts.begin(), starts.end());
@@ -84,9 +93,10 @@ void DevPlan::build_small(const Plan &pl) {
         if (it == starts.begin()) throw std::logic_error("original entry before the first front");
         const int f = std::prev(it)->second;
         const Front &F = pl.fronts[f];
-        if (d - F.buf_off >= (int64_t)F.m * F.m) throw std::logic_error("original entry outside its front");
-        if (slot[f] >= 0) per_slot[slot[f]].push_back({pl.orig_q[e], (int)(d - F.buf_off)});
-        else rest[F.level].push_back({pl.orig_q[e], d});
+        const int64_t o = d - F.buf_off;
+        if (o >= (int64_t)F.m * F.m) throw std::logic_error("original entry outside its front");
+        if (slot[f] >= 0) per_slot[slot[f]].push_back({pl.orig_q[e], (int)o});
+        else per_col[fd[f].slot + o / F.m].push_back({pl.orig_q[e], (int)o});
     }
     std::vector<int64_t> optr(nslot + 1, 0), oq;
     std::vector<int> ooff;
@@ -94,31 +104,31 @@ void DevPlan::build_small(const Plan &pl) {
         for (auto &e : per_slot[k]) { oq.push_back(e.first); ooff.push_back(e.second); }
         optr[k + 1] = (int64_t)oq.size();
     }
-    std::vector<int64_t> rq, rd;
-    for (int l = 0; l < pl.nlevels; l++) {
-        const int64_t b = (int64_t)rq.size();
-        for (auto &e : rest[l]) { rq.push_back(e.first); rd.push_back(e.second); }
-        orig_large_range.push_back({b, (int64_t)rq.size()});
+    std::vector<int64_t> lq;
+    std::vector<int> loff;
+    for (size_t c = 0; c < cptr.size(); c++) {
+        cptr[c] = (int)lq.size();
+        for (auto &e : per_col[c]) { lq.push_back(e.first); loff.push_back(e.second); }
     }
     root_first = dev_upload(first);
     root_last = dev_upload(last);
-    slot_of = dev_upload(slot);
     small_optr = dev_upload(optr);
     small_oq = dev_upload(oq);
     small_ooff = dev_upload(ooff);
-    orig_q_large = dev_upload(rq);
-    orig_dst_large = dev_upload(rd);
-    bytes += (2 * first.size() + slot.size() + ooff.size()) * 4 + (optr.size() + oq.size() + rq.size() + rd.size()) * 8;
+    large_cptr = dev_upload(cptr);
+    large_oq = dev_upload(lq);
+    large_ooff = dev_upload(loff);
+    bytes += (2 * first.size() + ooff.size() + cptr.size() + loff.size()) * 4 + (optr.size() + oq.size() + lq.size()) * 8;
     for (int l = 0; l < pl.nlevels; l++) {
         const LevelPlan &L = pl.levels[l];
         // the level's small fronts outside the subtrees
-        std::vector<int> sm;
+        std::vector<FrontDev> sm;
         int smm = 0;
         double el = 0, sfl = 0, sel = 0;
         for (int f : L.small)
             if (!in[f]) {
                 const Front &F = pl.fronts[f];
-                sm.push_back(f);
+                sm.push_back(fd[f]);
                 smm = std::max(smm, F.m);
                 sel += 2.0 * F.m * F.m;
                 for (int k = 0; k < F.p; k++) {
@@ -141,8 +151,9 @@ DevPlan::DevPlan(std::shared_ptr<const Plan> p) : host(std::move(p)) {
     std::vector<FrontDev> fd(pl.fronts.size());
     for (size_t f = 0; f < pl.fronts.size(); f++) {
         const Front &F = pl.fronts[f];
-        fd[f] = {F.p, F.m, F.pos0, F.nchild, F.child_off, F.level, F.buf_off, F.fv_off, F.idx_off, F.inv_off};
+        fd[f] = {F.p, F.m, F.pos0, F.nchild, F.child_off, F.level, -1, 0, F.buf_off, F.fv_off, F.idx_off, F.inv_off};
     }
+    build_small(pl, fd);
     fronts = dev_upload(fd);
     children = dev_upload(pl.children);
     idx = dev_upload(pl.idx);
@@ -197,8 +208,6 @@ DevPlan::DevPlan(std::shared_ptr<const Plan> p) : host(std::move(p)) {
         }
         lv_children.push_back(haskids);
         lv_fr.push_back(dev_upload(lf));
-        lv_small.push_back(dev_upload(L.small));
-        lv_large.push_back(dev_upload(L.large));
         lv_all.push_back(dev_upload(all));
         n_small.push_back((int)L.small.size());
         n_large.push_back((int)L.large.size());
@@ -301,7 +310,6 @@ DevPlan::DevPlan(std::shared_ptr<const Plan> p) : host(std::move(p)) {
         vinv_list_off = dev_upload(loff);
         bytes += lst.size() * 12;
     }
-    build_small(pl);
     counts.resize(pl.levels.size());
     for (size_t l = 0; l < pl.levels.size(); l++) {
         const LevelPlan &L = pl.levels[l];
@@ -367,12 +375,10 @@ DevPlan::~DevPlan() {
     for (auto p : vinv_off) dev_free(p);
     dev_free(vinv_list);
     dev_free(vinv_list_off);
-    dev_free(root_first); dev_free(root_last); dev_free(slot_of); dev_free(small_optr);
-    dev_free(small_oq); dev_free(small_ooff); dev_free(orig_q_large); dev_free(orig_dst_large);
+    dev_free(root_first); dev_free(root_last); dev_free(small_optr); dev_free(small_oq);
+    dev_free(small_ooff); dev_free(large_cptr); dev_free(large_oq); dev_free(large_ooff);
     for (auto p : lv_small_rest) dev_free(p);
     for (auto p : lv_fr) dev_free(p);
-    for (auto p : lv_small) dev_free(p);
-    for (auto p : lv_large) dev_free(p);
     for (auto p : lv_all) dev_free(p);
 }
 
@@ -391,50 +397,58 @@ Factors<T>::~Factors() {
 template struct Factors<double>;
 template struct Factors<float>;
 
+// 1+2: assembly of the blocked fronts
 // ---------------------------------------------------------------------------
-// 1+2: front assembly
-// ---------------------------------------------------------------------------
+// A workgroup writes a block of whole columns of one front, every entry once,
+// as the sum of the children's Schur complements, then adds the columns'
+// original entries (each destination is unique, and only this workgroup
+// touches these columns: a barrier separates the two, where a scatter launch of
+// its own cost 5 us a level).  With up to two children (the grid plans' fronts)
+// their values are loaded unconditionally (an entry a child does not cover
+// reads the child's block origin and is dropped), four entries at a time, so
+// eight loads are in flight before the first add.  grid (fronts, column blocks, nfreq)
 template <typename T>
 __global__ void __launch_bounds__(256) k_front_assemble(cx<T> *__restrict__ arena, int64_t fstride,
+                                                        const FrontDev *__restrict__ lvF,
                                                         const FrontDev *__restrict__ fronts,
-                                                        const int *__restrict__ list, const int *__restrict__ children,
-                                                        const int *__restrict__ inv) {
+                                                        const int *__restrict__ children, const int *__restrict__ inv,
+                                                        const int *__restrict__ cptr, const int64_t *__restrict__ oq,
+                                                        const int *__restrict__ ooff,
+                                                        const cx<double> *__restrict__ vals, int64_t vstride,
+                                                        int ncols) {
     extern __shared__ int cmap[];   // [nchild][m]: child row of each front row, or -1
     __shared__ int64_t cbase[kAsmMaxChildren];
     __shared__ int cstride[kAsmMaxChildren];
-    const FrontDev F = fronts[list[blockIdx.x]];
+    const FrontDev F = lvF[blockIdx.x];
+    const int m = F.m, nc = F.nchild, c0 = blockIdx.y * ncols, c1 = min(m, c0 + ncols);
+    if (c0 >= m) return;
     cx<T> *A = arena + blockIdx.z * fstride;
     cx<T> *G = A + F.buf_off;
-    const int m = F.m, nc = F.nchild;
+    const int tid = threadIdx.x;
+    const int o0 = cptr[F.slot + c0], o1 = cptr[F.slot + c1];
     // the children's row maps and block origins, staged once: each entry below
     // then waits on one value load only
-    if (threadIdx.x < nc) {
-        const FrontDev C = fronts[children[F.child_off + threadIdx.x]];
-        cbase[threadIdx.x] = C.buf_off + C.p + (int64_t)C.p * C.m;   // contribution block origin
-        cstride[threadIdx.x] = C.m;
+    if (tid < nc) {
+        const FrontDev C = fronts[children[F.child_off + tid]];
+        cbase[tid] = C.buf_off + C.p + (int64_t)C.p * C.m;   // contribution block origin
+        cstride[tid] = C.m;
     }
     for (int c = 0; c < nc; c++) {
         const int io = fronts[children[F.child_off + c]].inv_off;
-        for (int r = threadIdx.x; r < m; r += blockDim.x) cmap[c * m + r] = inv[io + r];
+        for (int r = tid; r < m; r += 256) cmap[c * m + r] = inv[io + r];
     }
     __syncthreads();
-    const int64_t total = (int64_t)m * m;
-    const int64_t step = (int64_t)gridDim.y * blockDim.x;
-    if (nc <= 2 && total < (int64_t(1) << 31)) {
-        // up to two children (the grid plans' fronts): each entry's child
-        // values are loaded unconditionally (an entry a child does not cover
-        // reads the child's block origin and is dropped), four entries at a
-        // time, so eight loads are in flight before the first add
-        // (entry indices in 32 bits)
+    const int64_t beg = (int64_t)c0 * m, end = (int64_t)c1 * m;
+    if (nc <= 2 && end < (int64_t(1) << 31)) {
         constexpr int U = 4;
-        const int tot = (int)total, stp = (int)step;
-        for (int e0 = blockIdx.y * blockDim.x + threadIdx.x; e0 < tot; e0 += U * stp) {
+        const int tot = (int)end;
+        for (int e0 = (int)beg + tid; e0 < tot; e0 += U * 256) {
             cx<T> w[U][2];
             bool ok[U][2];
 #pragma unroll
             for (int u = 0; u < U; u++) {
-                const int e = e0 + u * stp;
-                const int ec = e < tot ? e : 0;
+                const int e = e0 + u * 256;
+                const int ec = e < tot ? e : (int)beg;
                 const int s = ec / m, r = ec - s * m;
 #pragma unroll
                 for (int c = 0; c < 2; c++) {
@@ -445,7 +459,7 @@ __global__ void __launch_bounds__(256) k_front_assemble(cx<T> *__restrict__ aren
             }
 #pragma unroll
             for (int u = 0; u < U; u++) {
-                const int e = e0 + u * stp;
+                const int e = e0 + u * 256;
                 if (e >= tot) break;
                 cx<T> v = {T(0), T(0)};
                 if (ok[u][0]) v = w[u][0];
@@ -453,31 +467,22 @@ __global__ void __launch_bounds__(256) k_front_assemble(cx<T> *__restrict__ aren
                 G[e] = v;
             }
         }
-        return;
-    }
-    // unrolled: several entries' value loads in flight at once
-#pragma unroll 4
-    for (int64_t e = (int64_t)blockIdx.y * blockDim.x + threadIdx.x; e < total; e += step) {
-        const int s = (int)(e / m), r = (int)(e - (int64_t)s * m);
-        cx<T> v = {T(0), T(0)};
-        for (int c = 0; c < nc; c++) {
-            const int a = cmap[c * m + r], b = cmap[c * m + s];
-            if (a >= 0 && b >= 0) v = cadd(v, A[cbase[c] + a + (int64_t)b * cstride[c]]);
+    } else {
+        for (int64_t e = beg + tid; e < end; e += 256) {
+            const int s = (int)(e / m), r = (int)(e - (int64_t)s * m);
+            cx<T> v = {T(0), T(0)};
+            for (int c = 0; c < nc; c++) {
+                const int a = cmap[c * m + r], b = cmap[c * m + s];
+                if (a >= 0 && b >= 0) v = cadd(v, A[cbase[c] + a + (int64_t)b * cstride[c]]);
+            }
+            G[e] = v;
         }
-        G[e] = v;
     }
-}
-
-template <typename T>
-__global__ void __launch_bounds__(256) k_scatter_orig(cx<T> *__restrict__ arena, int64_t fstride,
-                                                      const cx<double> *__restrict__ vals, int64_t vstride,
-                                                      const int64_t *__restrict__ q, const int64_t *__restrict__ dst,
-                                                      int64_t count) {
-    cx<T> *A = arena + blockIdx.y * fstride;
-    const cx<double> *V = vals + blockIdx.y * vstride;
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < count; e += (int64_t)gridDim.x * blockDim.x) {
-        cx<double> v = V[q[e]];
-        cx<T> &d = A[dst[e]];
+    __syncthreads();
+    const cx<double> *V = vals + blockIdx.z * vstride;
+    for (int e = o0 + tid; e < o1; e += 256) {
+        const cx<double> v = V[oq[e]];
+        cx<T> &d = G[ooff[e]];
         d.x += (T)v.x;
         d.y += (T)v.y;
     }
@@ -574,7 +579,7 @@ __device__ __forceinline__ int wave_min(int v) {
 }
 
 // Partial LU of an m x m front held column-major in LDS (p pivots, row
-// pivoting within the p fully-summed rows); the swap of step j goes to piv[j].
+// pivoting within the p fully-summed rows); rp[i] is the row that ends at position i.
 // All 256 threads of the workgroup call it.  Blocked by kLuNb pivots, three
 // barriers per panel:
 //   - wave 0 factors the panel's kLuNb columns with its rows in registers (lane
@@ -599,9 +604,11 @@ struct LuPerm {
     int nd;
 };
 template <typename T, int NR>
-__device__ __forceinline__ void small_lu_lds(cx<T> *S, int m, int p, int *__restrict__ piv, int *__restrict__ sing,
-                                             LuPerm *pm) {
+__device__ __forceinline__ void small_lu_lds(cx<T> *S, int m, int p, int *rp, int *__restrict__ sing, LuPerm *pm) {
     const int tid = threadIdx.x, bs = 256, lane = tid & 63;
+    int row[NR];   // wave 0: the row (before all swaps) at the lane's position
+#pragma unroll
+    for (int k = 0; k < NR; k++) row[k] = lane + 64 * k;
     for (int jb = 0; jb < p; jb += kLuNb) {
         const int je = min(p, jb + kLuNb), nb = je - jb;   // panel columns [jb, je)
         if (tid < 64) {
@@ -643,7 +650,6 @@ __device__ __forceinline__ void small_lu_lds(cx<T> *S, int m, int p, int *__rest
                 }
                 const int pr = __builtin_amdgcn_readlane(bp, L);
                 zero |= mx == T(0);
-                if (lane == 0) piv[j] = pr;
                 const cx<T> d = readlane_t(rc, L);
                 cx<T> u[kLuNb];
 #pragma unroll
@@ -678,6 +684,7 @@ __device__ __forceinline__ void small_lu_lds(cx<T> *S, int m, int p, int *__rest
                     for (int c = 0; c < kLuNb; c++)
                         if (c < nb) S[pos[k] + (jb + c) * m] = a[k][c];
                     if (pos[k] < je) pm->top[pos[k] - jb] = r;
+                    rp[pos[k]] = row[k];
                 }
                 const bool moved = in && pos[k] >= je && pos[k] != r;
                 const unsigned long long mv = __ballot(moved);
@@ -689,6 +696,10 @@ __device__ __forceinline__ void small_lu_lds(cx<T> *S, int m, int p, int *__rest
                 base += __popcll(mv);
             }
             if (lane == 0) pm->nd = base;
+            // (one wave: its LDS operations complete in order)
+#pragma unroll
+            for (int k = 0; k < NR; k++)
+                if (lane + 64 * k >= jb && lane + 64 * k < p) row[k] = rp[lane + 64 * k];
         }
         __syncthreads();
         // the other columns: rows of the panel and the rows it displaced, through
@@ -754,17 +765,18 @@ __device__ __forceinline__ void small_lu_lds(cx<T> *S, int m, int p, int *__rest
 // what a small front's assembly and LU read of the plan and write beside the arena
 struct SmallDev {
     const FrontDev *fronts;
-    const int *slot_of, *children, *inv;
+    const int *children, *inv;
     const int64_t *optr, *oq;
     const int *ooff;
     const cx<double> *vals;
     int64_t vstride;
-    int *piv;
+    int *rowperm;
     int n;
     int *sing;
 };
 struct SmallShared {
     LuPerm pm;
+    int rp[96];   // row (before all swaps) at each position
     int64_t cbase[kAsmMaxChildren];
     int cstride[kAsmMaxChildren];
 };
@@ -773,7 +785,7 @@ template <typename T>
 constexpr size_t small_front_lds(int mmax, int max_children) {
     return sizeof(cx<T>) * (size_t)mmax * mmax + sizeof(int) * (size_t)mmax * max_children;
 }
-constexpr size_t kSmallLdsMax = 160 * 1024 - 512, kSubLdsMax = 68 * 1024;
+constexpr size_t kSmallLdsMax = 160 * 1024 - 1024, kSubLdsMax = 68 * 1024;
 
 // One small front of one frequency, by 256 threads: pull-assembly in LDS from
 // the children's contribution blocks, the original entries added, the partial
@@ -787,13 +799,11 @@ constexpr size_t kSmallLdsMax = 160 * 1024 - 512, kSubLdsMax = 68 * 1024;
 // frequencies: small fronts 4.7 ms in FP64 and 2.3 in FP32, the factorisation
 // 38.6 to 34.6 ms and 24.4 to 22.1.
 template <typename T, int NR>
-__device__ __forceinline__ void small_front(cx<T> *__restrict__ A, const SmallDev &d, int f, int fq, cx<T> *S,
-                                            SmallShared &sh) {
-    const FrontDev F = d.fronts[f];
+__device__ __forceinline__ void small_front(cx<T> *__restrict__ A, const SmallDev &d, const FrontDev &F, int fq,
+                                            cx<T> *S, SmallShared &sh) {
     const int m = F.m, mm = m * m, nc = F.nchild, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     int *cmap = reinterpret_cast<int *>(S + mm);   // [nchild][m]: child row of each front row, or -1
-    const int slot = d.slot_of[f];
-    const int64_t o0 = d.optr[slot], o1 = d.optr[slot + 1];
+    const int64_t o0 = d.optr[F.slot], o1 = d.optr[F.slot + 1];
     if (nc > 0) {
         if (tid < nc) {
             const FrontDev C = d.fronts[d.children[F.child_off + tid]];
@@ -846,7 +856,8 @@ __device__ __forceinline__ void small_front(cx<T> *__restrict__ A, const SmallDe
         t.y += (T)v.y;
     }
     __syncthreads();
-    small_lu_lds<T, NR>(S, m, F.p, d.piv + (int64_t)fq * d.n + F.pos0, d.sing + fq, &sh.pm);
+    small_lu_lds<T, NR>(S, m, F.p, sh.rp, d.sing + fq, &sh.pm);
+    for (int r = tid; r < F.p; r += 256) d.rowperm[(int64_t)fq * d.n + F.pos0 + r] = sh.rp[r];
     cx<T> *G = A + F.buf_off;
     for (int e = tid; e < mm; e += 256) G[e] = S[e];
 }
@@ -854,11 +865,12 @@ __device__ __forceinline__ void small_front(cx<T> *__restrict__ A, const SmallDe
 // grid (the level's small fronts, nfreq)
 template <typename T, int NR>
 __global__ void __launch_bounds__(256) k_small_front(cx<T> *__restrict__ arena, int64_t fstride, SmallDev d,
-                                                     const int *__restrict__ list) {
+                                                     const FrontDev *__restrict__ lvF) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     __shared__ SmallShared sh;
     const int fq = blockIdx.y;
-    small_front<T, NR>(arena + fq * fstride, d, list[blockIdx.x], fq, reinterpret_cast<cx<T> *>(smem_raw), sh);
+    const FrontDev F = lvF[blockIdx.x];
+    small_front<T, NR>(arena + fq * fstride, d, F, fq, reinterpret_cast<cx<T> *>(smem_raw), sh);
 }
 
 // ---------------------------------------------------------------------------
@@ -889,7 +901,8 @@ __global__ void __launch_bounds__(256) k_subtree_factor(cx<T> *arena, int64_t fs
         const int r = t / nf, fq = t - r * nf;
         const int f0 = root_first[r], f1 = root_last[r];
         for (int f = f0; f <= f1; f++) {
-            small_front<T, 1>(arena + (int64_t)fq * fstride, d, f, fq, reinterpret_cast<cx<T> *>(smem_raw), sh);
+            const FrontDev F = d.fronts[f];
+            small_front<T, 1>(arena + (int64_t)fq * fstride, d, F, fq, reinterpret_cast<cx<T> *>(smem_raw), sh);
             __syncthreads();   // the parent, later in this loop, reads this block
         }
     }
@@ -900,13 +913,18 @@ __global__ void __launch_bounds__(256) k_subtree_factor(cx<T> *arena, int64_t fs
 // ---------------------------------------------------------------------------
 template <typename T>
 __global__ void __launch_bounds__(256) k_panel(cx<T> *__restrict__ arena, int64_t fstride,
-                                               const FrontDev *__restrict__ fronts, const int *__restrict__ list,
-                                               int *__restrict__ piv, int n, int k0, int nb, int *__restrict__ sing) {
+                                               const FrontDev *__restrict__ lvF, int *__restrict__ rowperm, int n,
+                                               int k0, int nb, int *__restrict__ sing) {
     __shared__ T sb[4];
     __shared__ int si[4];
-    const FrontDev F = fronts[list[blockIdx.x]];
+    const FrontDev F = lvF[blockIdx.x];
     if (F.p <= k0) return;
     const int fq = blockIdx.y;
+    int *rp = rowperm + (int64_t)fq * n + F.pos0;
+    if (k0 == 0) {
+        for (int r = threadIdx.x; r < F.p; r += blockDim.x) rp[r] = r;
+        __syncthreads();
+    }
     cx<T> *G = arena + fq * fstride + F.buf_off;
     const int m = F.m, p = F.p, kb = min(nb, p - k0), tid = threadIdx.x, bs = blockDim.x;
     for (int j = k0; j < k0 + kb; j++) {
@@ -915,7 +933,9 @@ __global__ void __launch_bounds__(256) k_panel(cx<T> *__restrict__ arena, int64_
         for (int r = j + tid; r < p; r += bs) better(best, bi, cabs1(G[r + (int64_t)j * m]), r);
         const int pr = block_argmax(best, bi, sb, si);
         if (tid == 0) {
-            piv[(int64_t)fq * n + F.pos0 + j] = pr;
+            const int a = rp[j];
+            rp[j] = rp[pr];
+            rp[pr] = a;
             if (sb[0] == T(0)) atomicOr(sing + fq, 1);
         }
         if (pr != j)
@@ -963,11 +983,11 @@ struct PanelSlot {
 };
 template <typename T, int NW>
 __global__ void __launch_bounds__(64 * NW) k_panel_reg(cx<T> *__restrict__ arena, int64_t fstride,
-                                                       const FrontDev *__restrict__ fronts,
-                                                       const int *__restrict__ list, int *__restrict__ piv, int n,
-                                                       int k0, int nb, int *__restrict__ sing) {
+                                                       const FrontDev *__restrict__ lvF, int *__restrict__ piv,
+                                                       int *__restrict__ rowperm, int n, int k0, int nb,
+                                                       int *__restrict__ sing) {
     __shared__ PanelSlot<T> slot[2][NW];
-    const FrontDev F = fronts[list[blockIdx.x]];
+    const FrontDev F = lvF[blockIdx.x];
     if (F.p <= k0) return;
     const int fq = blockIdx.y;
     cx<T> *G = arena + fq * fstride + F.buf_off;
@@ -981,6 +1001,8 @@ __global__ void __launch_bounds__(64 * NW) k_panel_reg(cx<T> *__restrict__ arena
         ar[c] = in && c < kb ? v.x : T(0);
         ai[c] = in && c < kb ? v.y : T(0);
     });
+    int *rp = rowperm + (int64_t)fq * n + F.pos0 + k0;
+    const int row = in ? (k0 == 0 ? tid : rp[tid]) : 0;   // (before all swaps) at the thread's position
     int pos = tid;
     bool zero = false;
     const int n8 = (kb + 7) >> 3;
@@ -1071,6 +1093,7 @@ __global__ void __launch_bounds__(64 * NW) k_panel_reg(cx<T> *__restrict__ arena
         });
     }
     if (zero && tid == 0) atomicOr(sing + fq, 1);
+    if (in) rp[pos] = row;   // (every thread read its row before the first barrier)
     if (in)
         static_for<32>([&](auto c) {
             if (c < kb) G[(k0 + pos) + (int64_t)(k0 + c) * m] = {ar[c], ai[c]};
@@ -1096,11 +1119,11 @@ constexpr int kPanelRows = sizeof(T) == 8 ? 512 : 1024;
 // rows at two to three waves per SIMD (registers).
 template <typename T, bool TRSM>
 __global__ void __launch_bounds__(64) k_panel_finish(cx<T> *__restrict__ arena, int64_t fstride,
-                                                     const FrontDev *__restrict__ fronts, const int *__restrict__ list,
-                                                     const int *__restrict__ piv, int n, int k0, int nb, int ccols) {
+                                                     const FrontDev *__restrict__ lvF, const int *__restrict__ piv,
+                                                     int n, int k0, int nb, int ccols) {
     __shared__ cx<T> U[32][33];
     __shared__ int src[32], dq[32], dr[32];
-    const FrontDev F = fronts[list[blockIdx.y]];
+    const FrontDev F = lvF[blockIdx.y];
     if (F.p <= k0) return;
     const int fq = blockIdx.z;
     cx<T> *G = arena + fq * fstride + F.buf_off;
@@ -1108,7 +1131,17 @@ __global__ void __launch_bounds__(64) k_panel_finish(cx<T> *__restrict__ arena, 
     const bool cols = (int)blockIdx.x < ccols;
     if (cols && (int)blockIdx.x * 64 >= m - kb) return;
     if (!cols && p + ((int)blockIdx.x - ccols) * 64 >= m) return;
-    // the panel's block, 16 entries per thread, all in flight before the stores
+    // a contribution row's panel entries (columns past kb read column k0 and are
+    // not used), then the panel's block, 16 entries per thread, all in flight
+    // before the first is used
+    T xr[32], xi[32];
+    const int i = p + ((int)blockIdx.x - ccols) * 64 + tid;
+    if (!cols)
+        static_for<32>([&](auto t) {
+            const cx<T> v = G[(i < m ? i : p) + (int64_t)(k0 + (t < kb ? t : 0)) * m];
+            xr[t] = v.x;
+            xi[t] = v.y;
+        });
     if (TRSM || !cols) {
         T ur[16], ui[16];
         static_for<16>([&](auto u) {
@@ -1149,7 +1182,6 @@ __global__ void __launch_bounds__(64) k_panel_finish(cx<T> *__restrict__ arena, 
         if (beyond) c += kb;
         if (c >= m || (!moved && !(TRSM && beyond))) return;
         cx<T> *col = G + (int64_t)c * m;
-        T xr[32], xi[32];
         static_for<32>([&](auto t) {
             const cx<T> v = col[t < kb ? src[t] : k0];
             xr[t] = v.x;
@@ -1175,33 +1207,29 @@ __global__ void __launch_bounds__(64) k_panel_finish(cx<T> *__restrict__ arena, 
                     xi[i] = v.y;
                 });
                 // (keeps the scheduler from hoisting the whole block's LDS reads into registers)
-                if constexpr (t % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+                if constexpr (sizeof(T) == 8 || t % 2 == 1) __builtin_amdgcn_sched_barrier(0);
             });
         static_for<32>([&](auto t) {
             if (t < kb) col[k0 + t] = {xr[t], xi[t]};
         });
         return;
     }
-    // contribution rows: x U_kk = a, U_kk from the factored panel (columns past kb
-    // read column k0 and are not used)
-    const int i = p + ((int)blockIdx.x - ccols) * 64 + tid, ic = i < m ? i : p;
-    T xr[32], xi[32];
-    static_for<32>([&](auto t) {
-        const cx<T> v = G[ic + (int64_t)(k0 + (t < kb ? t : 0)) * m];
-        xr[t] = v.x;
-        xi[t] = v.y;
-    });
+    // contribution rows: x U_kk = a, U_kk from the factored panel
     __syncthreads();
     const cx<T> rc = crecip(U[tid & 31][tid & 31]);   // lane t: the reciprocal of pivot t
     static_for<32>([&](auto t) {
         if (t < kb) {
-            cx<T> a = {xr[t], xi[t]};
-            static_for<t>([&](auto s) { a = cmsub_f(a, cx<T>{xr[s], xi[s]}, U[s][t]); });
-            a = cmul_f(a, readlane_t(rc, t));
-            xr[t] = a.x;
-            xi[t] = a.y;
+            const cx<T> x = cmul_f(cx<T>{xr[t], xi[t]}, readlane_t(rc, t));
+            xr[t] = x.x;
+            xi[t] = x.y;
+            static_for<31 - t>([&](auto d) {
+                constexpr int s = t + 1 + d;
+                const cx<T> v = cmsub_f(cx<T>{xr[s], xi[s]}, x, U[t][s]);
+                xr[s] = v.x;
+                xi[s] = v.y;
+            });
         }
-        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (sizeof(T) == 8 || t % 2 == 1) __builtin_amdgcn_sched_barrier(0);
     });
     if (i < m)
         static_for<32>([&](auto t) {
@@ -1217,13 +1245,12 @@ __global__ void __launch_bounds__(64) k_panel_finish(cx<T> *__restrict__ arena, 
 // second panel's columns only), else at m.  grid (column chunks, fronts, nfreq)
 template <typename T, int KB>
 __global__ void __launch_bounds__(256) k_trsm_u(cx<T> *__restrict__ arena, int64_t fstride,
-                                               const FrontDev *__restrict__ fronts, const int *__restrict__ list,
-                                               int k0, int ccap) {
+                                               const FrontDev *__restrict__ lvF, int k0, int ccap) {
     constexpr int XW = KB == 32 ? 64 : 32, LPC = 256 / XW;   // columns per workgroup, lanes per column
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T>(*Ls)[KB + 1] = reinterpret_cast<cx<T>(*)[KB + 1]>(smem_raw);
     cx<T>(*Xs)[XW + 1] = reinterpret_cast<cx<T>(*)[XW + 1]>(smem_raw + sizeof(cx<T>) * KB * (KB + 1));
-    const FrontDev F = fronts[list[blockIdx.y]];
+    const FrontDev F = lvF[blockIdx.y];
     if (F.p <= k0) return;
     const int m = F.m, kb = min(KB, F.p - k0), cend = ccap > 0 ? min(k0 + ccap, F.p) : m;
     const int c0 = k0 + kb + blockIdx.x * XW;
@@ -1296,12 +1323,12 @@ constexpr size_t trsm_lds() {
 // ---------------------------------------------------------------------------
 template <typename T, bool DEEP>
 __global__ void __launch_bounds__(256) k_gemm_update(cx<T> *__restrict__ arena, int64_t fstride,
-                                                     const FrontDev *__restrict__ fronts, const int *__restrict__ list,
+                                                     const FrontDev *__restrict__ lvF,
                                                      const TileDev *__restrict__ tiles, int k0, int depth, int ccap) {
     constexpr int KB = 32;
     __shared__ T Ar[KB][64], Ai[KB][64], Br[KB][64], Bi[KB][64];
     const TileDev tl = tiles[blockIdx.x];
-    const FrontDev F = fronts[list[tl.front]];
+    const FrontDev F = lvF[tl.front];
     const int m = F.m, kd = min(depth, F.p - k0);
     const int base = k0 + kd, cend = ccap > 0 ? min(k0 + ccap, F.p) : m;
     const int r0 = base + tl.ti * 64, c0 = base + tl.tj * 64;
@@ -1412,30 +1439,11 @@ __global__ void __launch_bounds__(256) k_gemm_update(cx<T> *__restrict__ arena, 
             }
 }
 
-// ---------------------------------------------------------------------------
-// row permutation of every front from its swap sequence: rowperm[pos0+i] is
-// the local row that ends at position i
-// ---------------------------------------------------------------------------
 // zero-pivot flags cleared by a kernel rather than a memset node, so the
 // factorisation can be captured into a graph and replayed
 __global__ void k_clear_flags(int *__restrict__ flags, int count) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < count) flags[i] = 0;
-}
-
-__global__ void k_rowperm(const FrontDev *__restrict__ fronts, int nfronts, const int *__restrict__ piv, int n,
-                          int *__restrict__ rowperm) {
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= nfronts) return;
-    const FrontDev F = fronts[f];
-    const int64_t o = (int64_t)blockIdx.y * n;
-    int *rp = rowperm + o + F.pos0;
-    const int *pv = piv + o + F.pos0;
-    for (int i = 0; i < F.p; i++) rp[i] = i;
-    for (int j = 0; j < F.p; j++) {
-        int t = pv[j];
-        if (t != j) { int a = rp[j]; rp[j] = rp[t]; rp[t] = a; }
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1783,8 +1791,8 @@ void factor_numeric(const DevPlan &dp, Factors<T> &F, const cx<double> *vals, in
         attr_set = true;
     }
     const bool sub = g_persistent && dp.nroots > 0 && F.sched;
-    const SmallDev sd{dp.fronts, dp.slot_of, dp.children, dp.inv, dp.small_optr, dp.small_oq, dp.small_ooff,
-                      vals,      vstride,    F.piv,       pl.n,   F.sing};
+    const SmallDev sd{dp.fronts, dp.children, dp.inv, dp.small_optr, dp.small_oq, dp.small_ooff,
+                      vals,      vstride,     F.rowperm, pl.n,     F.sing};
     if (dp.max_children > kAsmMaxChildren) throw std::logic_error("front assembly: too many children");
     if (sub) {
         const int ntask = dp.nroots * nf;
@@ -1809,7 +1817,7 @@ void factor_numeric(const DevPlan &dp, Factors<T> &F, const cx<double> *vals, in
             if (lds > kSmallLdsMax) throw std::logic_error("small front exceeds LDS");
             ProfScope ps(K_SMALL_LU, st, (sub ? dp.small_rest_flops[l] : cnt.small_flops) * nf,
                          (sub ? dp.small_rest_elems[l] : cnt.small_elems) * es);
-            const int *list = sub ? dp.lv_small_rest[l] : dp.lv_small[l];
+            const FrontDev *list = sub ? dp.lv_small_rest[l] : dp.lv_fr[l];
             if (smm <= 64)
                 hipLaunchKernelGGL((k_small_front<T, 1>), dim3(n_small, nf), dim3(256), lds, st, F.arena, F.fstride,
                                    sd, list);
@@ -1817,22 +1825,16 @@ void factor_numeric(const DevPlan &dp, Factors<T> &F, const cx<double> *vals, in
                 hipLaunchKernelGGL((k_small_front<T, 2>), dim3(n_small, nf), dim3(256), lds, st, F.arena, F.fstride,
                                    sd, list);
         }
+        const FrontDev *lvL = dp.lv_fr[l] + dp.n_small[l];   // the level's blocked fronts
         if (dp.n_large[l] > 0) {
             ProfScope ps(K_FRONT_ASSEMBLE, st, 0.0, dp.asm_elems_large[l] * es);
-            int64_t mm = (int64_t)L.large_mmax * L.large_mmax;
-            // about 16 entries per thread (measured faster than 4 or 8)
-            int chunks = (int)std::min<int64_t>(std::max<int64_t>(1, mm / (256 * 16)), 256);
+            // about 16 entries per thread, in whole columns
+            const int ncols = std::max(1, 4096 / L.large_mmax);
             const size_t lds = sizeof(int) * (size_t)dp.max_children * L.large_mmax;
             if (lds > 64 * 1024) throw std::logic_error("front assembly: too large a front for the row maps");
-            hipLaunchKernelGGL(k_front_assemble<T>, dim3(dp.n_large[l], chunks, nf), dim3(256), lds, st, F.arena,
-                               F.fstride, dp.fronts, dp.lv_large[l], dp.children, dp.inv);
-        }
-        const int64_t obeg = dp.orig_large_range[l].first, ocnt = dp.orig_large_range[l].second - obeg;
-        if (ocnt > 0) {
-            ProfScope ps(K_SCATTER, st, 0.0, (double)ocnt * (16.0 + 16.0 + 2 * sizeof(cx<T>)) * nf);
-            int blocks = (int)std::min<int64_t>((ocnt + 255) / 256, 4096);
-            hipLaunchKernelGGL(k_scatter_orig<T>, dim3(blocks, nf), dim3(256), 0, st, F.arena, F.fstride, vals,
-                               vstride, dp.orig_q_large + obeg, dp.orig_dst_large + obeg, ocnt);
+            hipLaunchKernelGGL(k_front_assemble<T>, dim3(dp.n_large[l], (L.large_mmax + ncols - 1) / ncols, nf),
+                               dim3(256), lds, st, F.arena, F.fstride, lvL, dp.fronts, dp.children, dp.inv,
+                               dp.large_cptr, dp.large_oq, dp.large_ooff, vals, vstride, ncols);
         }
         if (dp.n_large[l] > 0) {
             const size_t lds32 = trsm_lds<T, 32>(), lds64 = trsm_lds<T, 64>();
@@ -1850,8 +1852,8 @@ void factor_numeric(const DevPlan &dp, Factors<T> &F, const cx<double> *vals, in
                         ProfScope ps(K_PANEL, st, flops * nf, 0.0);
                         const dim3 g(dp.n_large[l], nf);
 #define PANEL(NW) \
-    hipLaunchKernelGGL((k_panel_reg<T, NW>), g, dim3(64 * NW), 0, st, F.arena, F.fstride, dp.fronts, dp.lv_large[l], \
-                       F.piv, pl.n, k0, pl.nb, F.sing)
+    hipLaunchKernelGGL((k_panel_reg<T, NW>), g, dim3(64 * NW), 0, st, F.arena, F.fstride, lvL, F.piv, F.rowperm, pl.n, k0, \
+                       pl.nb, F.sing)
                         if (rows <= 64) PANEL(1);
                         else if (rows <= 128) PANEL(2);
                         else if (rows <= 256) PANEL(4);
@@ -1862,22 +1864,22 @@ void factor_numeric(const DevPlan &dp, Factors<T> &F, const cx<double> *vals, in
                     ProfScope ps(K_PANEL_APPLY, st, trsm ? trsm_flops * nf : 0.0, 0.0);
                     if (trsm)
                         hipLaunchKernelGGL((k_panel_finish<T, true>), dim3(ccols + crows, dp.n_large[l], nf), dim3(64),
-                                           0, st, F.arena, F.fstride, dp.fronts, dp.lv_large[l], F.piv, pl.n, k0,
+                                           0, st, F.arena, F.fstride, lvL, F.piv, pl.n, k0,
                                            pl.nb, ccols);
                     else
                         hipLaunchKernelGGL((k_panel_finish<T, false>), dim3(ccols + crows, dp.n_large[l], nf),
-                                           dim3(64), 0, st, F.arena, F.fstride, dp.fronts, dp.lv_large[l], F.piv, pl.n,
+                                           dim3(64), 0, st, F.arena, F.fstride, lvL, F.piv, pl.n,
                                            k0, pl.nb, ccols);
                 } else {
                     {
                         ProfScope ps(K_PANEL, st, flops * nf, 0.0);
                         hipLaunchKernelGGL(k_panel<T>, dim3(dp.n_large[l], nf), dim3(256), 0, st, F.arena, F.fstride,
-                                           dp.fronts, dp.lv_large[l], F.piv, pl.n, k0, pl.nb, F.sing);
+                                           lvL, F.rowperm, pl.n, k0, pl.nb, F.sing);
                     }
                     if (trsm) {
                         ProfScope ps(K_TRSM, st, trsm_flops * nf, 0.0);
                         hipLaunchKernelGGL((k_trsm_u<T, 32>), dim3(ccols, dp.n_large[l], nf), dim3(256), lds32, st,
-                                           F.arena, F.fstride, dp.fronts, dp.lv_large[l], k0, 0);
+                                           F.arena, F.fstride, lvL, k0, 0);
                     }
                 }
             };
@@ -1886,10 +1888,10 @@ void factor_numeric(const DevPlan &dp, Factors<T> &F, const cx<double> *vals, in
                 ProfScope ps(K_GEMM, st, flops * nf, elems * es);
                 if (depth > 32)
                     hipLaunchKernelGGL((k_gemm_update<T, true>), dim3(cnt, nf), dim3(256), 0, st, F.arena, F.fstride,
-                                       dp.fronts, dp.lv_large[l], dp.tiles + off, k0, depth, ccap);
+                                       lvL, dp.tiles + off, k0, depth, ccap);
                 else
                     hipLaunchKernelGGL((k_gemm_update<T, false>), dim3(cnt, nf), dim3(256), 0, st, F.arena,
-                                       F.fstride, dp.fronts, dp.lv_large[l], dp.tiles + off, k0, depth, ccap);
+                                       F.fstride, lvL, dp.tiles + off, k0, depth, ccap);
             };
             if (deep_level<T>(L, dp.deep_steps[l][0], nf)) {
                 // two panels per block: panel 1; its U rows and update on panel 2's
@@ -1906,7 +1908,7 @@ void factor_numeric(const DevPlan &dp, Factors<T> &F, const cx<double> *vals, in
                         {
                             ProfScope ps(K_TRSM, st, d.trsm_thin_flops * nf, 0.0);
                             hipLaunchKernelGGL((k_trsm_u<T, 32>), dim3(1, dp.n_large[l], nf), dim3(256),
-                                               lds32, st, F.arena, F.fstride, dp.fronts, dp.lv_large[l],
+                                               lds32, st, F.arena, F.fstride, lvL,
                                                b0, 64);
                         }
                         gemm(d.thin_off, d.thin_cnt, b0, 32, 64, d.thin_flops, d.thin_elems);
@@ -1916,7 +1918,7 @@ void factor_numeric(const DevPlan &dp, Factors<T> &F, const cx<double> *vals, in
                         ProfScope ps(K_TRSM, st, d.trsm_deep_flops * nf, 0.0);
                         const int colchunks = (L.large_mmax - b0 + 31) / 32;
                         hipLaunchKernelGGL((k_trsm_u<T, 64>), dim3(colchunks, dp.n_large[l], nf), dim3(256),
-                                           lds64, st, F.arena, F.fstride, dp.fronts, dp.lv_large[l], b0,
+                                           lds64, st, F.arena, F.fstride, lvL, b0,
                                            0);
                     }
                     gemm(d.deep_off, d.deep_cnt, b0, 64, 0, d.deep_flops, d.deep_elems);
@@ -1932,8 +1934,6 @@ void factor_numeric(const DevPlan &dp, Factors<T> &F, const cx<double> *vals, in
         }
     }
     const int nfr = (int)pl.fronts.size();
-    hipLaunchKernelGGL(k_rowperm, dim3((nfr + 63) / 64, nf), dim3(64), 0, st, dp.fronts, nfr, F.piv, pl.n,
-                       F.rowperm);
     hipLaunchKernelGGL(k_gsrc, dim3(nfr, nf), dim3(64), 0, st, dp.fronts, nfr, F.rowperm, pl.n, dp.gsrc_id, pl.fv_rows,
                        F.gsrc);
     {

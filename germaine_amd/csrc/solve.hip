@@ -182,10 +182,10 @@ __device__ __forceinline__ cx<T> front_row(const FrontDev &F, int i, int r, int 
 // grid (fronts, chunks, slots)
 template <typename T>
 __global__ void __launch_bounds__(256) k_fwd_gather(const cx<T> *__restrict__ X, cx<T> *__restrict__ W,
-                                                    const FrontDev *__restrict__ fronts, const int *__restrict__ list,
+                                                    const FrontDev *__restrict__ lvF,
                                                     const int *__restrict__ gsrc, int64_t gstride, int n,
                                                     int64_t wstride, int nrhs, Sel sel) {
-    const FrontDev F = fronts[list[blockIdx.x]];
+    const FrontDev F = lvF[blockIdx.x];
     const int z = blockIdx.z;
     const int64_t total = (int64_t)F.m * nrhs;
     X += (int64_t)sel.s[z] * n * nrhs;
@@ -416,14 +416,13 @@ constexpr size_t blk2_smem_bytes() {
 }
 template <typename T, class C, bool FWD>
 __global__ void __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && C::NT == 512 ? 4 : 1)))
-k_blk2(const cx<T> *__restrict__ arena, int64_t fstride, const FrontDev *__restrict__ fronts,
-       const int *__restrict__ list, cx<T> *__restrict__ X, cx<T> *__restrict__ W, int n, int64_t wstride, int nrhs,
+k_blk2(const cx<T> *__restrict__ arena, int64_t fstride, const FrontDev *__restrict__ lvF, cx<T> *__restrict__ X, cx<T> *__restrict__ W, int n, int64_t wstride, int nrhs,
        int rt, int b0, int trans, int cj, Sel sel) {
     constexpr int RT = C::RT, CT = C::CT, NT = C::NT;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     BlkSmem<T, C> s(smem_raw + sizeof(T) * 2 * BK * CT);   // the first block's Y and the A tile
     T *Sr = reinterpret_cast<T *>(smem_raw), *Si = Sr + BK * CT;   // the second block's Y
-    const FrontDev F = fronts[list[blockIdx.y]];
+    const FrontDev F = lvF[blockIdx.y];
     if (F.p <= b0) return;
     const int m = F.m, tid = threadIdx.x;
     const int lo = min(BK, F.p - b0), hi = max(0, min(BK, F.p - b0 - BK));
@@ -544,15 +543,14 @@ k_blk2(const cx<T> *__restrict__ arena, int64_t fstride, const FrontDev *__restr
 constexpr int kContribRowsMax = 16384;   // m - p of any front on this path
 template <typename T, class C>
 __global__ void __launch_bounds__(C::NT) k_bwd_contrib(const cx<T> *__restrict__ arena, int64_t fstride,
-                                                       const FrontDev *__restrict__ fronts,
-                                                       const int *__restrict__ list, const int *__restrict__ idx,
+                                                       const FrontDev *__restrict__ lvF, const int *__restrict__ idx,
                                                        const cx<T> *__restrict__ X, cx<T> *__restrict__ W, int n,
                                                        int64_t wstride, int nrhs, int rt, int trans, int cj, Sel sel) {
     constexpr int RT = C::RT, CT = C::CT, NT = C::NT;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     BlkSmem<T, C> s(smem_raw);
     int *srow = reinterpret_cast<int *>(smem_raw + blk_smem_bytes<T, C>());
-    const FrontDev F = fronts[list[blockIdx.y]];
+    const FrontDev F = lvF[blockIdx.y];
     const int m = F.m, p = F.p, tid = threadIdx.x;
     const int row0 = blockIdx.x * RT;
     if (row0 >= p) return;
@@ -1558,10 +1556,10 @@ __global__ void __launch_bounds__(256) k_bwd_front(const cx<T> *__restrict__ are
 // transposed solves, after a level's backward blocks: x = P_f^T w for every
 // front of the level, through W rows [0, p) as scratch (copy, then scatter)
 template <typename T>
-__global__ void __launch_bounds__(256) k_piv_copy(const FrontDev *__restrict__ fronts, const int *__restrict__ list,
+__global__ void __launch_bounds__(256) k_piv_copy(const FrontDev *__restrict__ lvF,
                                                   const cx<T> *__restrict__ X, cx<T> *__restrict__ W, int n,
                                                   int64_t wstride, int nrhs, Sel sel) {
-    const FrontDev F = fronts[list[blockIdx.x]];
+    const FrontDev F = lvF[blockIdx.x];
     X += (int64_t)sel.s[blockIdx.z] * n * nrhs;
     W += sel.s[blockIdx.z] * wstride;
     const int64_t total = (int64_t)F.p * nrhs;
@@ -1569,11 +1567,11 @@ __global__ void __launch_bounds__(256) k_piv_copy(const FrontDev *__restrict__ f
         W[F.fv_off * nrhs + e] = X[(int64_t)F.pos0 * nrhs + e];
 }
 template <typename T>
-__global__ void __launch_bounds__(256) k_piv_unswap(const FrontDev *__restrict__ fronts, const int *__restrict__ list,
+__global__ void __launch_bounds__(256) k_piv_unswap(const FrontDev *__restrict__ lvF,
                                                     const int *__restrict__ rowperm, cx<T> *__restrict__ X,
                                                     const cx<T> *__restrict__ W, int n, int64_t wstride, int nrhs,
                                                     Sel sel) {
-    const FrontDev F = fronts[list[blockIdx.x]];
+    const FrontDev F = lvF[blockIdx.x];
     X += (int64_t)sel.s[blockIdx.z] * n * nrhs;
     W += sel.s[blockIdx.z] * wstride;
     rowperm += (int64_t)sel.f[blockIdx.z] * n;
@@ -3032,8 +3030,8 @@ void sweeps(const Factors<T> &F, const Sel &in, int sys, int nrhs, cx<T> *Xp, cx
             ProfScope ps(K_FWD_GATHER, st, 0.0, nz * 2.0 * c.sum_m * nr * es);
             int64_t work = (int64_t)dp.mmax_all[l] * nrhs;
             int chunks = (int)std::min<int64_t>(std::max<int64_t>(1, work / 1024), 256);
-            hipLaunchKernelGGL(k_fwd_gather<T>, dim3(nfr, chunks, ns), dim3(256), 0, st, Xp, Wp, dp.fronts,
-                               dp.lv_all[l], trans ? dp.gsrc_id : F.gsrc, trans ? (int64_t)0 : pl.fv_rows * 3, n,
+            hipLaunchKernelGGL(k_fwd_gather<T>, dim3(nfr, chunks, ns), dim3(256), 0, st, Xp, Wp, dp.lv_fr[l],
+                               trans ? dp.gsrc_id : F.gsrc, trans ? (int64_t)0 : pl.fv_rows * 3, n,
                                wstride, nrhs, in);
         }
         const int pmax = dp.pmax_all[l];
@@ -3049,7 +3047,7 @@ void sweeps(const Factors<T> &F, const Sel &in, int sys, int nrhs, cx<T> *Xp, cx
                 const int tiles = std::max(1, (dp.mmax_all[l] - b0 - 1) / C::RT + 1), rt = (nrhs + C::CT - 1) / C::CT;
                 const size_t lds = blk2_smem_bytes<T, C>();
                 hipLaunchKernelGGL((k_blk2<T, C, true>), dim3(tiles, nfr, rt * ns), dim3(C::NT), lds, st, F.arena,
-                                   F.fstride, dp.fronts, dp.lv_all[l], Xp, Wp, n, wstride, nrhs, rt, b0, (int)trans,
+                                   F.fstride, dp.lv_fr[l], Xp, Wp, n, wstride, nrhs, rt, b0, (int)trans,
                                    (int)cj, in);
             });
         }
@@ -3098,7 +3096,7 @@ void sweeps(const Factors<T> &F, const Sel &in, int sys, int nrhs, cx<T> *Xp, cx
                 const int rt = (nrhs + C::CT - 1) / C::CT;
                 const size_t lds = blk_smem_bytes<T, C>() + 4 * (size_t)dp.mmax_all[l];
                 hipLaunchKernelGGL((k_bwd_contrib<T, C>), dim3((pmax + C::RT - 1) / C::RT, nfr, rt * ns), dim3(C::NT),
-                                   lds, st, F.arena, F.fstride, dp.fronts, dp.lv_all[l], dp.idx, Xp, Wp, n, wstride, nrhs, rt, (int)trans, (int)cj,
+                                   lds, st, F.arena, F.fstride, dp.lv_fr[l], dp.idx, Xp, Wp, n, wstride, nrhs, rt, (int)trans, (int)cj,
                                    in);
             });
         }
@@ -3112,16 +3110,16 @@ void sweeps(const Factors<T> &F, const Sel &in, int sys, int nrhs, cx<T> *Xp, cx
                 using C = decltype(t);
                 const int tiles = std::max(1, (b0 + C::RT - 1) / C::RT), rt = (nrhs + C::CT - 1) / C::CT;
                 const size_t lds = blk2_smem_bytes<T, C>();
-                hipLaunchKernelGGL((k_blk2<T, C, false>), dim3(tiles, nfr, rt * ns), dim3(C::NT), lds, st, F.arena, F.fstride, dp.fronts, dp.lv_all[l], Xp, Wp, n,
+                hipLaunchKernelGGL((k_blk2<T, C, false>), dim3(tiles, nfr, rt * ns), dim3(C::NT), lds, st, F.arena, F.fstride, dp.lv_fr[l], Xp, Wp, n,
                                    wstride, nrhs, rt, b0, (int)trans, (int)cj, in);
             });
         }
         if (trans) {
             ProfScope ps(K_PIV_UNSWAP, st, 0.0, nz * 4.0 * c.sum_p * nr * es);
             const int chunks = (int)std::min<int64_t>(std::max<int64_t>(1, (int64_t)pmax * nrhs / 1024), 256);
-            hipLaunchKernelGGL(k_piv_copy<T>, dim3(nfr, chunks, ns), dim3(256), 0, st, dp.fronts, dp.lv_all[l], Xp,
+            hipLaunchKernelGGL(k_piv_copy<T>, dim3(nfr, chunks, ns), dim3(256), 0, st, dp.lv_fr[l], Xp,
                                Wp, n, wstride, nrhs, in);
-            hipLaunchKernelGGL(k_piv_unswap<T>, dim3(nfr, chunks, ns), dim3(256), 0, st, dp.fronts, dp.lv_all[l],
+            hipLaunchKernelGGL(k_piv_unswap<T>, dim3(nfr, chunks, ns), dim3(256), 0, st, dp.lv_fr[l],
                                F.rowperm, Xp, Wp, n, wstride, nrhs, in);
         }
     }
