@@ -106,16 +106,16 @@ template <typename T>
 __device__ __forceinline__ T cabs1(cx<T> a) {
     return fabs(a.x) + fabs(a.y);
 }
-// 1/a by Smith's method (no overflow for large pivots)
+// 1/a by Smith's method (no overflow for large pivots), without a branch: in a
+// wave whose lanes differ both sides would run one after the other, and a
+// branch keeps the divisions from overlapping what stands around them
 template <typename T>
 __device__ __forceinline__ cx<T> crecip(cx<T> a) {
-    if (fabs(a.x) >= fabs(a.y)) {
-        T r = a.y / a.x, d = a.x + a.y * r;
-        return {T(1) / d, -r / d};
-    } else {
-        T r = a.x / a.y, d = a.x * r + a.y;
-        return {r / d, T(-1) / d};
-    }
+    const bool big = fabs(a.x) >= fabs(a.y);
+    const T u = big ? a.x : a.y, v = big ? a.y : a.x;
+    const T r = v / u, d = u + v * r;
+    const T e = T(1) / d, g = r / d;
+    return {big ? e : g, big ? -g : -e};
 }
 // a / b by Smith's method
 template <typename T>

@@ -558,15 +558,28 @@ template <typename T>
 __device__ __forceinline__ cx<T> readlane_t(cx<T> v, int l) {
     return {readlane_t(v.x, l), readlane_t(v.y, l)};
 }
+// (neither argument is ever a NaN; fmax would quiet each of them first)
+__device__ __forceinline__ float max_raw(float a, float b) { return fmax(a, b); }
+__device__ __forceinline__ double max_raw(double a, double b) {
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
 template <typename T>
 __device__ __forceinline__ T wave_max(T v) {
-    v = fmax(v, dpp_f<0x111, 0xF>(v));   // row_shr 1, 2, 4, 8
-    v = fmax(v, dpp_f<0x112, 0xF>(v));
-    v = fmax(v, dpp_f<0x114, 0xF>(v));
-    v = fmax(v, dpp_f<0x118, 0xF>(v));
-    v = fmax(v, dpp_f<0x142, 0xA>(v));   // row_bcast 15 into rows 1 and 3
-    v = fmax(v, dpp_f<0x143, 0xC>(v));   // row_bcast 31 into rows 2 and 3
+    v = max_raw(v, dpp_f<0x111, 0xF>(v));   // row_shr 1, 2, 4, 8
+    v = max_raw(v, dpp_f<0x112, 0xF>(v));
+    v = max_raw(v, dpp_f<0x114, 0xF>(v));
+    v = max_raw(v, dpp_f<0x118, 0xF>(v));
+    v = max_raw(v, dpp_f<0x142, 0xA>(v));   // row_bcast 15 into rows 1 and 3
+    v = max_raw(v, dpp_f<0x143, 0xC>(v));   // row_bcast 31 into rows 2 and 3
     return readlane_t(v, 63);
+}
+// holds a value's computation where it is called: the reciprocals then run
+// beside the pivot search instead of being sunk below it
+template <typename T>
+__device__ __forceinline__ void pin(cx<T> v) {
+    asm volatile("" ::"v"(v.x), "v"(v.y));
 }
 __device__ __forceinline__ int wave_min(int v) {
     v = min(v, dpp_i<0x111, 0xF>(v));
@@ -642,6 +655,7 @@ __device__ __forceinline__ void small_lu_lds(cx<T> *S, int m, int p, int *rp, in
                     }
                 const cx<T> rc = crecip(ca);
                 const T mx = wave_max(best);
+                pin(rc);
                 const unsigned long long tie = __ballot(best == mx);
                 int L = __ffsll((unsigned long long)tie) - 1;
                 if (tie & (tie - 1)) {
@@ -962,24 +976,27 @@ __global__ void __launch_bounds__(256) k_panel(cx<T> *__restrict__ arena, int64_
 // 32-column panel are the front's remaining fully-summed rows [k0, p), one row
 // per thread, all its panel columns in that thread's registers.  Rows do not
 // move while the panel is factored: each thread carries the position its row
-// has reached.  Per column every wave finds its best candidate (DPP maximum
-// and a ballot) and that lane publishes value, position, reciprocal and row in
-// the wave's slot; one barrier later every thread picks the winning wave and
-// updates its own row from that slot (slots alternate, so a step has one
-// barrier).  Eight columns are unrolled, then the row is rotated by eight
-// registers, so the code stays short enough for the instruction cache.
-// k_panel_finish then applies the panel's permutation to the front's other
+// has reached.  The panel goes eight columns at a time.  Per column every wave
+// finds its best candidate (DPP maximum and a ballot) and that lane publishes
+// value, position, reciprocal and its entries of the eight columns in the
+// wave's slot; one barrier later every thread picks the winning wave and updates
+// its own eight entries from that slot (slots alternate, so a step has one
+// barrier).  After eight columns the pivot rows' other entries are solved in LDS
+// (one lane per column) and every remaining row takes one rank-8 update, which
+// keeps those columns off the chain of pivot steps; then the row is rotated
+// by eight registers, so the code stays short enough for the instruction
+// cache.  k_panel_finish applies the panel's permutation to the front's other
 // columns.  Bound by the 32-step chain: a panel in LDS with three barriers per
-// column took 48 us (270x145, one FP64 frequency, event-timed), this 32; the 69
+// column took 48 us (270x145, one FP64 frequency, event-timed), this 28; the 69
 // panels of 1601x401, four frequencies, 8.5 ms (those above 318 rows in global
-// memory) and 3.5.
+// memory) and 2.9.
 // ---------------------------------------------------------------------------
 template <typename T>
 struct PanelSlot {
     T best;
     int pos;
     cx<T> rc;
-    cx<T> row[32];
+    cx<T> row[8];
 };
 template <typename T, int NW>
 __global__ void __launch_bounds__(64 * NW) k_panel_reg(cx<T> *__restrict__ arena, int64_t fstride,
@@ -987,6 +1004,7 @@ __global__ void __launch_bounds__(64 * NW) k_panel_reg(cx<T> *__restrict__ arena
                                                        int *__restrict__ rowperm, int n, int k0, int nb,
                                                        int *__restrict__ sing) {
     __shared__ PanelSlot<T> slot[2][NW];
+    __shared__ cx<T> Lb[8][8], Ub[8][24];   // the block's pivot rows: multipliers, entries of the later columns
     const FrontDev F = lvF[blockIdx.x];
     if (F.p <= k0) return;
     const int fq = blockIdx.y;
@@ -1016,6 +1034,7 @@ __global__ void __launch_bounds__(64 * NW) k_panel_reg(cx<T> *__restrict__ arena
                 const T best = in && pos >= j ? (v >= T(0) ? v : T(-1)) : T(-2);
                 const cx<T> rc = crecip(cx<T>{ar[jj], ai[jj]});
                 const T mx = wave_max(best);
+                pin(rc);
                 const unsigned long long tie = __ballot(best == mx);
                 int L = __ffsll((unsigned long long)tie) - 1;
                 if (tie & (tie - 1)) {
@@ -1029,12 +1048,7 @@ __global__ void __launch_bounds__(64 * NW) k_panel_reg(cx<T> *__restrict__ arena
                     s.pos = pos;
                     s.rc = rc;
                     static_for<8>([&](auto c) {
-                        if (c >= jj) s.row[c] = {ar[c], ai[c]};
-                    });
-                    static_for<3>([&](auto g) {
-                        if (b + g + 1 < n8) static_for<8>([&](auto c) {
-                            s.row[8 * g + 8 + c] = {ar[8 * g + 8 + c], ai[8 * g + 8 + c]};
-                        });
+                        if (c > jj) s.row[c] = {ar[c], ai[c]};
                     });
                 }
                 __syncthreads();
@@ -1066,17 +1080,58 @@ __global__ void __launch_bounds__(64 * NW) k_panel_reg(cx<T> *__restrict__ arena
                             ai[c] = a.y;
                         }
                     });
-                    static_for<3>([&](auto g) {
-                        if (b + g + 1 < n8) static_for<8>([&](auto cc) {
-                            constexpr int c = 8 * g + 8 + cc;
-                            const cx<T> a = cmsub_f(cx<T>{ar[c], ai[c]}, l, s.row[c]);
-                            ar[c] = a.x;
-                            ai[c] = a.y;
-                        });
-                    });
                 }
             }
         });
+        if (b + 1 < n8) {
+            // (a block before the last is full: its eight pivots are the positions 8b .. 8b + 7)
+            const int t0 = pos - 8 * b;
+            const bool piv_row = in && t0 >= 0 && t0 < 8;
+            if (piv_row) {
+                static_for<8>([&](auto c) { Lb[t0][c] = {ar[c], ai[c]}; });
+                static_for<3>([&](auto g) {
+                    if (b + g + 1 < n8) static_for<8>([&](auto c) {
+                        Ub[t0][8 * g + c] = {ar[8 * g + 8 + c], ai[8 * g + 8 + c]};
+                    });
+                });
+            }
+            __syncthreads();
+            if (tid < 8 * (n8 - b - 1)) {
+                T ur[8], ui[8];
+                static_for<8>([&](auto t) {
+                    ur[t] = Ub[t][tid].x;
+                    ui[t] = Ub[t][tid].y;
+                });
+                static_for<7>([&](auto s) {
+                    static_for<7 - s>([&](auto d) {
+                        constexpr int t = s + 1 + d;
+                        const cx<T> u = cmsub_f(cx<T>{ur[t], ui[t]}, Lb[t][s], cx<T>{ur[s], ui[s]});
+                        ur[t] = u.x;
+                        ui[t] = u.y;
+                    });
+                });
+                static_for<8>([&](auto t) { Ub[t][tid] = {ur[t], ui[t]}; });
+            }
+            __syncthreads();
+            static_for<3>([&](auto g) {
+                if (b + g + 1 < n8) {
+                    if (piv_row)
+                        static_for<8>([&](auto c) {
+                            ar[8 * g + 8 + c] = Ub[t0][8 * g + c].x;
+                            ai[8 * g + 8 + c] = Ub[t0][8 * g + c].y;
+                        });
+                    else if (in && t0 >= 8)
+                        static_for<8>([&](auto t) {
+                            static_for<8>([&](auto cc) {
+                                constexpr int c = 8 * g + 8 + cc;
+                                const cx<T> a = cmsub_f(cx<T>{ar[c], ai[c]}, cx<T>{ar[t], ai[t]}, Ub[t][8 * g + cc]);
+                                ar[c] = a.x;
+                                ai[c] = a.y;
+                            });
+                        });
+                }
+            });
+        }
         // the next eight columns to the front; after four rotations the order is the first one
         T tr[8], ti[8];
         static_for<8>([&](auto c) {
