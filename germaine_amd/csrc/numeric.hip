@@ -1362,26 +1362,34 @@ constexpr size_t trsm_lds() {
 }
 
 // ---------------------------------------------------------------------------
-// trailing update C -= A*B on MFMA (complex = 3 real products in FP32, 4 in FP64), 64x64 tiles.
-// The product's depth is the front's next min(depth, p - k0) pivot columns
-// (depth 32: one panel; 64: two panels), taken 32 at a time through the same
-// LDS while the C tile stays in the accumulators, so C is read and written once
-// per `depth` pivots.  The updated block starts at row and column k0 + that
-// depth; ccap > 0 ends its columns at min(k0 + ccap, p) (the thin update of the
-// second panel's columns), else at m.
-// DEEP = false compiles the one-chunk form (depth <= 32) without the second
-// chunk's prefetch registers, which would cost occupancy.
+// trailing update C -= A*B on MFMA, four real products per complex product,
+// 64x64 tiles.  The product's depth is the front's next min(depth, p - k0)
+// pivot columns (depth 32: one panel; 64: two panels), taken KB at a time
+// through the same LDS with the next chunk's loads in flight during a chunk's
+// products, so C is read and written once per `depth` pivots.  C is loaded into
+// the accumulators themselves and A staged negated, which leaves the registers
+// for a tile of C beside them to more waves; the operands are staged as complex
+// entries, A by columns and B by its rows, each with the lanes that write it
+// along the contiguous direction (staging B by columns put 32 lanes on one bank).
+// The updated block starts at row and column k0 + that depth; ccap > 0 ends
+// its columns at min(k0 + ccap, p) (the thin update of the second panel's
+// columns), else at m.  Bound by each tile's load-stage-product chain at three to
+// four workgroups per CU: 1601x401, four frequencies, 10.2 ms a factorisation with C
+// and both chunks' operands in registers and LDS (FP64, two per CU), now 9.3; FP32
+// 7.1 and 6.6.
 // 4 waves in 2x2, each wave 32x32 = 2x2 blocks of 16x16.
 // MFMA 16x16x4 operand layout: A lane l -> (row l%16, k l/16), B lane l ->
 // (k l/16, col l%16).  Accumulator register v of lane l holds column l%16 and
 // row 4*(l/16)+v for f32, but row 4*v+l/16 for f64.
 // ---------------------------------------------------------------------------
-template <typename T, bool DEEP>
-__global__ void __launch_bounds__(256) k_gemm_update(cx<T> *__restrict__ arena, int64_t fstride,
+template <typename T>
+constexpr int kGemmKB = sizeof(T) == 8 ? 16 : 32;
+template <typename T>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k_gemm_update(cx<T> *__restrict__ arena, int64_t fstride,
                                                      const FrontDev *__restrict__ lvF,
                                                      const TileDev *__restrict__ tiles, int k0, int depth, int ccap) {
-    constexpr int KB = 32;
-    __shared__ T Ar[KB][64], Ai[KB][64], Br[KB][64], Bi[KB][64];
+    constexpr int KB = kGemmKB<T>, PER = KB * 64 / 256;
+    __shared__ cx<T> As[KB][64], Bs[64][KB + 1];
     const TileDev tl = tiles[blockIdx.x];
     const FrontDev F = lvF[tl.front];
     const int m = F.m, kd = min(depth, F.p - k0);
@@ -1391,106 +1399,82 @@ __global__ void __launch_bounds__(256) k_gemm_update(cx<T> *__restrict__ arena, 
     const int tid = threadIdx.x;
     const int lane = tid & 63, w = tid >> 6, wr = (w >> 1) * 32, wc = (w & 1) * 32;
     const int lr = lane & 15, lk = lane >> 4;
-    // the lane's 16 entries of C: loaded up front with the first operand chunk
-    // (one chunk), or after the products (two chunks: registers for occupancy)
-    cx<T> c[2][2][4];
-    auto load_c = [&]() {
-#pragma unroll
-        for (int a = 0; a < 2; a++)
-#pragma unroll
-            for (int b = 0; b < 2; b++)
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    // FP64: unconditional (entries outside the block read G[0] and are never
-                    // stored); FP32 keeps the conditional form, which measured as fast
-                    const int row = r0 + wr + a * 16 + mfma_t<T>::row(lk, v), col = c0 + wc + b * 16 + lr;
-                    const bool in = row < m && col < cend;
-                    if constexpr (sizeof(T) == 8) c[a][b][v] = G[in ? row + (int64_t)col * m : 0];
-                    else c[a][b][v] = in ? G[row + (int64_t)col * m] : cx<T>{T(0), T(0)};
-                }
-    };
-    if (!DEEP) load_c();
-    cx<T> av[KB * 64 / 256], bv[KB * 64 / 256];
-    // operand columns/rows k0+kc .. k0+kc+31 into registers; FP64 loads them
-    // unconditionally (entries outside read G[0]) so they stay in flight
-    // (19.4 against 20.8 ms per factorisation), FP32 conditionally (measured as
-    // fast); stage_chunk zeroes the entries outside as it stores them
-    int lkb = 0;   // columns of the chunk in av/bv
+    // addresses: a uniform base per operand and 32-bit byte offsets within 64 columns of it
+    const char *Ga = reinterpret_cast<const char *>(G + (int64_t)k0 * m + r0);   // column k of A at k m
+    char *Gc = reinterpret_cast<char *>(G + (int64_t)c0 * m);                    // column j of B and C at j m
+    auto at = [](const char *base, int e) { return *reinterpret_cast<const cx<T> *>(base + (unsigned)e * (unsigned)sizeof(cx<T>)); };
+    // a chunk's operands, loaded unconditionally (entries outside read the
+    // operand's first and are zeroed when staged) so that they stay in flight
+    T ax[PER], ay[PER], bx[PER], by[PER];
     auto load_chunk = [&](int kc) {
         const int kb = min(KB, kd - kc);
-        lkb = kb;
-#pragma unroll
-        for (int u = 0; u < KB * 64 / 256; u++) {
+        static_for<PER>([&](auto u) {
             const int e = tid + 256 * u, i = e & 63, k = e >> 6;
-            const bool in = k < kb && r0 + i < m;
-            if constexpr (sizeof(T) == 8) av[u] = G[in ? (r0 + i) + (int64_t)(k0 + kc + k) * m : 0];
-            else av[u] = in ? G[(r0 + i) + (int64_t)(k0 + kc + k) * m] : cx<T>{T(0), T(0)};
-        }
-#pragma unroll
-        for (int u = 0; u < KB * 64 / 256; u++) {
+            const cx<T> v = at(Ga, k < kb && r0 + i < m ? i + (kc + k) * m : 0);
+            ax[u] = v.x;
+            ay[u] = v.y;
+        });
+        static_for<PER>([&](auto u) {
             const int e = tid + 256 * u, k = e % KB, j = e / KB;
-            const bool in = k < kb && c0 + j < cend;
-            if constexpr (sizeof(T) == 8) bv[u] = G[in ? (k0 + kc + k) + (int64_t)(c0 + j) * m : 0];
-            else bv[u] = in ? G[(k0 + kc + k) + (int64_t)(c0 + j) * m] : cx<T>{T(0), T(0)};
-        }
+            const cx<T> v = at(Gc, k < kb && c0 + j < cend ? (k0 + kc + k) + j * m : 0);
+            bx[u] = v.x;
+            by[u] = v.y;
+        });
     };
-    auto stage_chunk = [&]() {
-#pragma unroll
-        for (int u = 0; u < KB * 64 / 256; u++) {
-            const int e = tid + 256 * u, ia = e & 63, ka = e >> 6, kbb = e % KB, jb = e / KB;
-            const bool ina = ka < lkb && r0 + ia < m, inb = kbb < lkb && c0 + jb < cend;
-            Ar[ka][ia] = ina ? av[u].x : T(0);
-            Ai[ka][ia] = ina ? av[u].y : T(0);
-            Br[kbb][jb] = inb ? bv[u].x : T(0);
-            Bi[kbb][jb] = inb ? bv[u].y : T(0);
-        }
+    auto stage_chunk = [&](int kc) {
+        const int kb = min(KB, kd - kc);
+        static_for<PER>([&](auto u) {
+            const int e = tid + 256 * u, i = e & 63, ka = e >> 6, kb2 = e % KB, j = e / KB;
+            const bool ina = ka < kb && r0 + i < m, inb = kb2 < kb && c0 + j < cend;
+            As[ka][i] = {ina ? -ax[u] : T(0), ina ? -ay[u] : T(0)};
+            Bs[j][kb2] = {inb ? bx[u] : T(0), inb ? by[u] : T(0)};
+        });
     };
-    cacc3<T> acc[2][2];   // three real products per complex product
-    for (int a = 0; a < 2; a++)
-        for (int b = 0; b < 2; b++) acc[a][b].zero();
     load_chunk(0);
-    stage_chunk();
-    __syncthreads();
-    // FP32: the next chunk's loads in flight during this chunk's products; FP64
-    // loads it after them (its prefetch registers would halve the occupancy)
-    constexpr bool kPrefetch = sizeof(T) == 4;
-    for (int kc = 0; kc < kd; kc += KB) {
-        const bool more = DEEP && kc + KB < kd;
-        if (kPrefetch && more) load_chunk(kc + KB);
-        const int kend = (min(KB, kd - kc) + 3) & ~3;
-        for (int kk = 0; kk < kend; kk += 4) {
-            const int k = kk + lk;
-            T ar[2], ai[2], br[2], bi[2];
-            for (int a = 0; a < 2; a++) {
-                ar[a] = Ar[k][wr + a * 16 + lr];
-                ai[a] = Ai[k][wr + a * 16 + lr];
-            }
-            for (int b = 0; b < 2; b++) {
-                br[b] = Br[k][wc + b * 16 + lr];
-                bi[b] = Bi[k][wc + b * 16 + lr];
-            }
-            for (int b = 0; b < 2; b++) {
-                const T bs = br[b] + bi[b];
-                for (int a = 0; a < 2; a++) acc[a][b].mma(ar[a], ai[a], br[b], bi[b], bs);
-            }
-        }
-        if (more) {
-            __syncthreads();   // every wave is done with this chunk
-            if (!kPrefetch) load_chunk(kc + KB);
-            stage_chunk();
-            __syncthreads();
-        }
-    }
-    if (DEEP) load_c();
+    typename mfma_t<T>::acc cr[2][2], ci[2][2];
 #pragma unroll
     for (int a = 0; a < 2; a++)
 #pragma unroll
         for (int b = 0; b < 2; b++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                const int row = r0 + wr + a * 16 + mfma_t<T>::row(lk, v), col = c0 + wc + b * 16 + lr;
-                if (row < m && col < cend)
-                    G[row + (int64_t)col * m] = {c[a][b][v].x - acc[a][b].re(v), c[a][b][v].y - acc[a][b].im(v)};
+                const int row = r0 + wr + a * 16 + mfma_t<T>::row(lk, v), j = wc + b * 16 + lr;
+                const cx<T> c = at(Gc, row < m && c0 + j < cend ? row + j * m : 0);
+                cr[a][b][v] = c.x;
+                ci[a][b][v] = c.y;
+            }
+    for (int kc = 0; kc < kd; kc += KB) {
+        if (kc > 0) __syncthreads();   // every wave is done with the previous chunk
+        stage_chunk(kc);
+        __syncthreads();
+        if (kc + KB < kd) load_chunk(kc + KB);   // in flight during this chunk's products
+        const int kend = (min(KB, kd - kc) + 3) & ~3;
+#pragma unroll 1
+        for (int kk = 0; kk < kend; kk += 4) {
+            const int k = kk + lk;
+            cx<T> av[2], bv[2];
+#pragma unroll
+            for (int a = 0; a < 2; a++) av[a] = As[k][wr + a * 16 + lr];
+#pragma unroll
+            for (int b = 0; b < 2; b++) bv[b] = Bs[wc + b * 16 + lr][k];
+#pragma unroll
+            for (int b = 0; b < 2; b++)
+#pragma unroll
+                for (int a = 0; a < 2; a++) cmma<T>(av[a].x, av[a].y, bv[b].x, bv[b].y, cr[a][b], ci[a][b]);
+        }
+    }
+    int ms = m;
+    asm("" : "+s"(ms));   // (the stores' offsets computed anew rather than kept through the products)
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int row = r0 + wr + a * 16 + mfma_t<T>::row(lk, v), j = wc + b * 16 + lr;
+                if (row < ms && c0 + j < cend)
+                    *reinterpret_cast<cx<T> *>(Gc + (unsigned)(row + j * ms) * (unsigned)sizeof(cx<T>)) = {cr[a][b][v],
+                                                                                                        ci[a][b][v]};
             }
 }
 
@@ -1941,12 +1925,8 @@ void factor_numeric(const DevPlan &dp, Factors<T> &F, const cx<double> *vals, in
             auto gemm = [&](int64_t off, int cnt, int k0, int depth, int ccap, double flops, double elems) {
                 if (cnt <= 0) return;
                 ProfScope ps(K_GEMM, st, flops * nf, elems * es);
-                if (depth > 32)
-                    hipLaunchKernelGGL((k_gemm_update<T, true>), dim3(cnt, nf), dim3(256), 0, st, F.arena, F.fstride,
-                                       lvL, dp.tiles + off, k0, depth, ccap);
-                else
-                    hipLaunchKernelGGL((k_gemm_update<T, false>), dim3(cnt, nf), dim3(256), 0, st, F.arena,
-                                       F.fstride, lvL, dp.tiles + off, k0, depth, ccap);
+                hipLaunchKernelGGL(k_gemm_update<T>, dim3(cnt, nf), dim3(256), 0, st, F.arena, F.fstride, lvL,
+                                   dp.tiles + off, k0, depth, ccap);
             };
             if (deep_level<T>(L, dp.deep_steps[l][0], nf)) {
                 // two panels per block: panel 1; its U rows and update on panel 2's
