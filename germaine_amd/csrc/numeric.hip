@@ -1519,8 +1519,11 @@ __global__ void k_gsrc(const FrontDev *__restrict__ fronts, int nfronts, const i
 // x1 = [inv(U11), -inv(U11) U12] [y1; x2].  Computed in FP64 for both factor
 // precisions (the block is staged in the factor precision, exact in FP64).
 // One workgroup per front, grid (fronts, nfreq); every global load of the
-// front is issued a phase ahead of its use (the next block, or the first
-// row and column chunk of the rectangles, while a block is inverted).
+// front is issued a phase ahead of its use (the next block, or the rows below,
+// while a block is inverted; the columns beyond, during the rows' products).
+// Bound by each workgroup's serial path: three per compute unit (registers
+// held to that, LDS allows no more) take 2.7 ms at 1601x401, four FP64
+// frequencies, where two took 3.6.
 // ---------------------------------------------------------------------------
 // every lane takes the value that lane q of its group of four holds (DPP quad permute)
 __device__ __forceinline__ int quad_bcast_i(int v, int q) {
@@ -1685,7 +1688,7 @@ __device__ __forceinline__ void u12_mfma(const cx<T> (*V)[33], const cx<double> 
 }
 
 template <typename T>
-__global__ void __launch_bounds__(256) k_diag_inv(cx<T> *__restrict__ arena, int64_t fstride,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k_diag_inv(cx<T> *__restrict__ arena, int64_t fstride,
                                                   const FrontDev *__restrict__ fronts,
                                                   const int *__restrict__ lv_single) {
     __shared__ cx<T> D[32][33];   // the block being inverted, then the rectangles' chunks
@@ -1722,12 +1725,7 @@ __global__ void __launch_bounds__(256) k_diag_inv(cx<T> *__restrict__ arena, int
         }
     };
     load_block(0);
-    if (single) {
-        if (p < m) {
-            load_l21(p);
-            load_u12(p);
-        }
-    }
+    if (single && p < m) load_l21(p);
     for (int b0 = 0; b0 < p; b0 += 32) {
         const int kb = min(32, p - b0);
 #pragma unroll
@@ -1751,6 +1749,7 @@ __global__ void __launch_bounds__(256) k_diag_inv(cx<T> *__restrict__ arena, int
     }
     if (!single) return;
     const int wave = tid >> 6, lane = tid & 63;
+    if (p < m) load_u12(p);   // in flight during the L21 products
     for (int r0 = p; r0 < m; r0 += 32) {
 #pragma unroll
         for (int u = 0; u < 4; u++) {
