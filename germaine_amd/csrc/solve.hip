@@ -234,7 +234,15 @@ struct BlkTile {
 // Shared memory of a block kernel (dynamic): right-hand-side block [BK][CT]
 // re/im, then the A tile [BK][RT] re/im, whose space the diagonal block
 // [BK][BK+1] complex shares: the diagonal product runs (and ends with a
-// barrier) before the A tile is stored.
+// barrier) before the A tile is stored.  The A tile's rows are padded: a
+// transposed operator is stored down the rows, and with a stride of whole bank
+// rounds all 32 lanes of such a store met on the same banks (M^T pass of
+// 1601x401, 4 frequencies x 200 right-hand sides: contribution launches
+// 2390 -> 1280 us FP32, 3473 -> 2630 us FP64, block launches 4263 -> 3210 and
+// 7841 -> 6660 us; M passes, stored along the rows, do not change.  The same
+// padding of the right-hand-side rows gave nothing).
+template <typename T, class C>
+constexpr int kAStride = C::RT + (sizeof(T) == 4 ? 17 : 1);
 template <typename T, class C>
 struct BlkSmem {
     T *Ar, *Ai, *Yr, *Yi;
@@ -243,7 +251,7 @@ struct BlkSmem {
         Yr = reinterpret_cast<T *>(raw);
         Yi = Yr + BK * C::CT;
         Ar = Yi + BK * C::CT;
-        Ai = Ar + BK * C::RT;
+        Ai = Ar + BK * kAStride<T, C>;
         D = reinterpret_cast<cx<T> *>(Ar);
     }
 };
@@ -252,7 +260,7 @@ static_assert(sizeof(cx<double>) * BK * (BK + 1) <= 2 * sizeof(double) * BK * 64
               "the diagonal block fits in the A tile's space");
 template <typename T, class C>
 constexpr size_t blk_smem_bytes() {
-    return sizeof(T) * (2 * BK * C::CT + 2 * BK * C::RT);
+    return sizeof(T) * (2 * BK * C::CT + 2 * BK * kAStride<T, C>);
 }
 
 // element (i, t) of the operator that solves 32-row diagonal block b0 in the
@@ -294,8 +302,8 @@ __device__ __forceinline__ void mma_tile(const T *Ar, const T *Ai, const T *Yr, 
         T ar[C::NA], ai[C::NA], br[C::NB], bi[C::NB];
 #pragma unroll
         for (int a = 0; a < C::NA; a++) {
-            ar[a] = Ar[k * C::RT + wr + a * 16 + lr];
-            ai[a] = Ai[k * C::RT + wr + a * 16 + lr];
+            ar[a] = Ar[k * kAStride<T, C> + wr + a * 16 + lr];
+            ai[a] = Ai[k * kAStride<T, C> + wr + a * 16 + lr];
         }
 #pragma unroll
         for (int b = 0; b < C::NB; b++) {
@@ -418,7 +426,7 @@ template <typename T, class C, bool FWD>
 __global__ void __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && C::NT == 512 ? 4 : 1)))
 k_blk2(const cx<T> *__restrict__ arena, int64_t fstride, const FrontDev *__restrict__ lvF, cx<T> *__restrict__ X, cx<T> *__restrict__ W, int n, int64_t wstride, int nrhs,
        int rt, int b0, int trans, int cj, Sel sel) {
-    constexpr int RT = C::RT, CT = C::CT, NT = C::NT;
+    constexpr int RT = C::RT, CT = C::CT, NT = C::NT, AS = kAStride<T, C>;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     BlkSmem<T, C> s(smem_raw + sizeof(T) * 2 * BK * CT);   // the first block's Y and the A tile
     T *Sr = reinterpret_cast<T *>(smem_raw), *Si = Sr + BK * CT;   // the second block's Y
@@ -473,8 +481,8 @@ k_blk2(const cx<T> *__restrict__ arena, int64_t fstride, const FrontDev *__restr
             if (!trans) { i = e % RT; k = e / RT; }
             else { k = e % BK; i = e / BK; }
             const bool in = upd && k < akb && row0 + i < rowend;
-            s.Ar[k * RT + i] = in ? av[u].x : T(0);
-            s.Ai[k * RT + i] = in ? (cj ? -av[u].y : av[u].y) : T(0);
+            s.Ar[k * AS + i] = in ? av[u].x : T(0);
+            s.Ai[k * AS + i] = in ? (cj ? -av[u].y : av[u].y) : T(0);
         }
     };
     auto stage_d = [&](const cx<T>(&v)[PD], int nb) {   // a diagonal block operator
@@ -546,7 +554,7 @@ __global__ void __launch_bounds__(C::NT) k_bwd_contrib(const cx<T> *__restrict__
                                                        const FrontDev *__restrict__ lvF, const int *__restrict__ idx,
                                                        const cx<T> *__restrict__ X, cx<T> *__restrict__ W, int n,
                                                        int64_t wstride, int nrhs, int rt, int trans, int cj, Sel sel) {
-    constexpr int RT = C::RT, CT = C::CT, NT = C::NT;
+    constexpr int RT = C::RT, CT = C::CT, NT = C::NT, AS = kAStride<T, C>;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     BlkSmem<T, C> s(smem_raw);
     int *srow = reinterpret_cast<int *>(smem_raw + blk_smem_bytes<T, C>());
@@ -596,8 +604,8 @@ __global__ void __launch_bounds__(C::NT) k_bwd_contrib(const cx<T> *__restrict__
             if (!trans) { i = e % RT; k = e / RT; }
             else { k = e % BK; i = e / BK; }
             const bool ain = k < kb && row0 + i < p;
-            s.Ar[k * RT + i] = ain ? av[u].x : T(0);
-            s.Ai[k * RT + i] = ain ? (cj ? -av[u].y : av[u].y) : T(0);
+            s.Ar[k * AS + i] = ain ? av[u].x : T(0);
+            s.Ai[k * AS + i] = ain ? (cj ? -av[u].y : av[u].y) : T(0);
         }
 #pragma unroll
         for (int u = 0; u < PY; u++) {
