@@ -22,6 +22,7 @@
 #include <cstdlib>
 #include <cstdio>
 #include <cstring>
+#include <limits>
 #include <mutex>
 
 #include "engine.hpp"
@@ -2468,7 +2469,8 @@ __global__ void __launch_bounds__(256) k_ir_in(const cx<double> *__restrict__ B,
 // One refinement step of launch slot z (frequency sel.f[z], slot s = sel.s[z]):
 // r <- r - op(M) D, with r read from Bu (the caller's b, user layout: point k
 // of column c at k + c*n) on the first step and from Rg otherwise;  Rg <- r,
-// R <- r in the factor precision (zero padding columns), and the sum of |r|^2
+// R <- r in the factor precision (zero padding columns) unless bit z of `last`
+// is set (then only the norms are wanted), and the sum of |r|^2
 // over the workgroup's points of every column in
 // partial[(z * gridDim.x + block) * nrhs + c].  Rg is in grid order (row
 // k = i + j*nx, stride ld64; each point read and written by its own thread
@@ -2476,12 +2478,19 @@ __global__ void __launch_bounds__(256) k_ir_in(const cx<double> *__restrict__ B,
 // be distinct buffers (other workgroups read a point's d while its own
 // workgroup writes r).  Row k of M has the entries of CSC column k (the
 // pattern is symmetric), all within the 3x3 neighbourhood.  Tiles of kIrTx x
-// kIrTy points (8 consecutive points of four grid rows): per 16-column chunk
-// the d of the (kIrTy + 2) x (kIrTx + 2) neighbourhood points is staged in LDS
-// once (each point's d is used by up to nine rows; an 8 x 4 tile stages 1.9
-// points per output), then one thread per (point, column) applies the stencil
-// from LDS.  grid (blocks, slots), grid-stride over tiles.
-constexpr int kIrTx = 8, kIrTy = 4, kIrCw = 16, kIrPts = kIrTx * kIrTy, kIrStage = (kIrTy + 2) * (kIrTx + 2);
+// kIrTy points: per 16-column chunk the d of the (kIrTy + 2) x (kIrTx + 2)
+// neighbourhood points is staged in LDS once (each point's d is used by up to
+// nine rows), then one thread per (point, column) applies the stencil from LDS.
+// Bound by memory, and on the first step by the caller's layout, whose columns
+// lie n points apart: a 16 x 2 tile stages 2.25 points per output where 8 x 4
+// stages 1.9 but reads 256 bytes of b in a row, and r and the stencil entries in
+// longer runs (1601x401, 8 frequencies x 200 right-hand sides, FP32: first step
+// 13.7 -> 12.0 ms, later ones 11.1 -> 10.5 ms; 32 x 1 is slower on all but the
+// first).  A last step, which writes nothing, takes 6.6 ms of those 11.0; 801x201,
+// 4 x 80, FP64: 0.81 -> 0.55 ms.  Recomputing r from b and all corrections, and
+// writing x from the last step, moves 30 % fewer bytes and was no faster, for the
+// caller's layout again.  grid (blocks, slots), grid-stride over tiles.
+constexpr int kIrTx = 16, kIrTy = 2, kIrCw = 16, kIrPts = kIrTx * kIrTy, kIrStage = (kIrTy + 2) * (kIrTx + 2);
 constexpr int kIrThreads = kIrPts * kIrCw, kIrWaves = kIrThreads / 64;
 constexpr int kIrCoef0 = (kIrStage + 63) / 64 * 64;   // first thread of the stencil-entry gather
 static_assert(kIrStage <= kIrCoef0 && kIrCoef0 + 9 * kIrPts <= kIrThreads,
@@ -2494,7 +2503,8 @@ __global__ void __launch_bounds__(kIrThreads) __attribute__((amdgpu_waves_per_eu
                                                  const int *__restrict__ iperm, int nx, int ny, int nrhs, int ld64,
                                                  int ld, int sys, int64_t nnz, const cx<double> *__restrict__ Bu,
                                                  cx<double> *Rg, const cx<T> *__restrict__ D,
-                                                 cx<T> *__restrict__ R, double *__restrict__ partial, Sel sel) {
+                                                 cx<T> *__restrict__ R, uint64_t last, double *__restrict__ partial,
+                                                 Sel sel) {
     extern __shared__ double wsum[];   // [kIrWaves][nrhs]
     __shared__ cx<T> sx[kIrStage][kIrCw];
     __shared__ cx<double> scoef[kIrPts][9];
@@ -2506,7 +2516,7 @@ __global__ void __launch_bounds__(kIrThreads) __attribute__((amdgpu_waves_per_eu
     vals += sel.f[z] * nnz;
     const int64_t o64 = s * n * ld64, o32 = s * n * ld;
     Rg += o64;
-    const bool first = Bu != nullptr;
+    const bool first = Bu != nullptr, store = !((last >> z) & 1);
     if (first) Bu += s * n * nrhs;
     D += o32;
     R += o32;
@@ -2578,9 +2588,11 @@ __global__ void __launch_bounds__(kIrThreads) __attribute__((amdgpu_waves_per_eu
                     const cx<T> d = sx[sidx[r][t]][cc];
                     acc = cmsub(acc, scoef[r][t], cx<double>{(double)d.x, (double)d.y});
                 }
-                Rg[k * ld64 + c] = acc;
-                R[dst + c] = {(T)acc.x, (T)acc.y};
-            } else if (pin && c < ld) {
+                if (store) {
+                    Rg[k * ld64 + c] = acc;
+                    R[dst + c] = {(T)acc.x, (T)acc.y};
+                }
+            } else if (store && pin && c < ld) {
                 R[dst + c] = {T(0), T(0)};
             }
             // the wave's four points of a column: sum, then one LDS update per column
@@ -3549,6 +3561,7 @@ std::vector<RefineStats> refine_panels(const Factors<T> &F, const std::vector<in
     std::vector<int> act_f = freqs, act_s = slots;
     std::vector<int> base(ns, 0);   // per slot: corrections already folded into acc
     uint64_t folded = 0;            // bit s: slot s has a folded sum in acc
+    std::vector<double> before(ns, 1.0);   // worst relative residual one step before the latest
     cx<double> *acc = nullptr;
     std::vector<int> hmap;          // column maps of a packed correction solve (host side of ws_pmap)
     for (int it = 0;; it++) {
@@ -3570,16 +3583,29 @@ std::vector<RefineStats> refine_panels(const Factors<T> &F, const std::vector<in
                 base[sel.s[z]] = it + 1;
             }
         }
-        {
-            // per slot: r (b on the first step), d and the neighbours' d from
-            // cache, r in FP64 and in the factor precision written; the stencil
-            // values and indices
-            const double panel = (double)n * nr * (16.0 + es + 16.0 + es);
-            ProfScope ps(K_RESIDUAL, st, sel.n * (8.0 * nnz * nr + 2.0 * n * nr), sel.n * (panel + nnz * 28.0));
-            hipLaunchKernelGGL(k_ir_step<T>, dim3(nblk, sel.n), dim3(kIrThreads), kIrWaves * sizeof(double) * nrhs, st,
-                               F.vals, dp.colptr, dp.rowind, dp.tq, dp.iperm, pl.nx, pl.ny, nrhs, ld64, ld, sys,
-                               pl.nnz, it == 0 ? B : nullptr, Rg, dbuf(it % kIrBufs), dbuf(jn), partial, sel);
+        // Launch slots whose last step this should be, from the residual's shrinking
+        // as it did in the step before (the first solve: to 2^16 roundings of the
+        // factor precision); their residual is not written.
+        uint64_t last = 0;
+        for (int z = 0; z < sel.n; z++) {
+            const double w = rs[sel.s[z]].max_rel_residual;
+            const double expect =
+                it == 0 ? std::ldexp((double)std::numeric_limits<T>::epsilon(), 16) : w * (w / before[sel.s[z]]);
+            if (it == max_iter || expect <= tol) last |= uint64_t(1) << z;
+            before[sel.s[z]] = it == 0 ? 1.0 : w;
         }
+        auto step = [&](const Sel &sl, uint64_t lm) {
+            // per slot: r (b on the first step), d and the neighbours' d from cache
+            // read, r in FP64 and in the factor precision written unless the slot is
+            // done with it; the stencil values and indices
+            const int nw = sl.n - __builtin_popcountll(lm);
+            const double panel = (double)n * nr * (16.0 + es);
+            ProfScope ps(K_RESIDUAL, st, sl.n * (8.0 * nnz * nr + 2.0 * n * nr), (sl.n + nw) * panel + sl.n * nnz * 28.0);
+            hipLaunchKernelGGL(k_ir_step<T>, dim3(nblk, sl.n), dim3(kIrThreads), kIrWaves * sizeof(double) * nrhs, st,
+                               F.vals, dp.colptr, dp.rowind, dp.tq, dp.iperm, pl.nx, pl.ny, nrhs, ld64, ld, sys,
+                               pl.nnz, it == 0 ? B : nullptr, Rg, dbuf(it % kIrBufs), dbuf(jn), lm, partial, sl);
+        };
+        step(sel, last);
         {
             ProfScope ps(K_NORM_REDUCE, st, sel.n * (double)nblk * nrhs, sel.n * 8.0 * (nblk + 1.0) * nrhs);
             hipLaunchKernelGGL(k_norm_reduce, dim3(nrhs, sel.n), dim3(256), 0, st, partial, nblk, nrhs, nrm, sel);
@@ -3588,6 +3614,13 @@ std::vector<RefineStats> refine_panels(const Factors<T> &F, const std::vector<in
         GFDFD_HIP(hipStreamSynchronize(st));
         keep_unconverged(h, ns, nrhs, it, tol, max_iter, act_f, act_s, rs);
         if (act_f.empty()) break;
+        std::vector<int> again_f, again_s;   // expected to be done, but not: the residual after all
+        for (int z = 0; z < sel.n; z++)
+            if (((last >> z) & 1) && std::find(act_s.begin(), act_s.end(), sel.s[z]) != act_s.end()) {
+                again_f.push_back(sel.f[z]);
+                again_s.push_back(sel.s[z]);
+            }
+        if (!again_f.empty()) step(make_sel(again_f, again_s), 0);
         // d = op(M)^-1 r in place; when at most half of the columns of every
         // remaining slot are still above the tolerance, only those are solved
         // (packed into ldc columns) and the others get a zero correction

@@ -221,6 +221,76 @@ def test_batched_solves_match_oracle(precision, sysno):
         assert rel(X[z], Xr.T) <= tol, (z, k)
 
 
+# the step expected to be a frequency's last writes no residual: the tolerance is
+# reached, or the step limit; 1e-18 is below what the caller's layout can reach,
+# while the residual carried by r -= op(M) d passes it
+@pytest.mark.parametrize("precision,tol,max_iter", [(G.FP64, 1e-10, 5), (G.FP32, 1e-10, 9), (G.FP32, 1e-10, 0),
+                                                    (G.FP32, 1e-4, 9), (G.FP64, 1e-18, 4), (G.FP32, 1e-18, 6)])
+def test_refinement_last_step(precision, tol, max_iter):
+    """x and the reported residual belong together (the residual of x recomputed
+    apart agrees to FP64 rounding, 1e-12 relative to b), and both agree with the
+    refinement in the caller's layout, which writes every residual."""
+    nx, ny, npml, dh = 45, 37, 6, 10.0
+    m1, m2 = smooth_model(nx, ny, seed=4)
+    freqs = [2.5, 7.0, 13.0]
+    say("refinement last step", precision, tol, max_iter)
+    pl = fdfd.Plan(nx, ny, small_max=16)
+    vals = pl.assemble(G.AC, dh, freqs, dev(m1), dev(m2), npml=npml)
+    F = pl.factor(vals, precision)
+    rng = np.random.default_rng(5)
+    B = dev(rng.standard_normal((3, 21, nx * ny)) + 1j * rng.standard_normal((3, 21, nx * ny)))
+    out = {}
+    try:
+        for layout in (0, 1):
+            fdfd.solve_tuning(refine_layout=layout)
+            X, its, rr = F.solve_refine_batch([0, 1, 2], B, tol=tol, max_iter=max_iter)
+            out[layout] = (X.cpu().numpy(), list(its), list(rr))
+            say("  layout", layout, "iterations", its, rr)
+            for z in range(3):
+                res = pl.residual(vals[z], B[z], X[z])
+                worst = float((res.norm(dim=1) / B[z].norm(dim=1)).max())
+                assert abs(worst - rr[z]) <= 1e-3 * worst + 1e-12, (layout, z, worst, rr[z])
+    finally:
+        fdfd.solve_tuning()
+    if max(out[1][2]) <= tol or max_iter == 0:
+        assert out[0][1] == out[1][1]
+    if max_iter > 0 and tol < 1e-4:
+        assert rel(out[0][0], out[1][0]) <= 1e-9
+
+
+def test_refinement_last_step_expected_wrongly():
+    """A tolerance between what the residual's shrinking promises and what the
+    step delivers: the step runs again for the residual it did not write, and the
+    refinement goes on to the tolerance.  The residual of x, recomputed apart,
+    agrees with the reported one to FP64 rounding, 1e-12 relative to b."""
+    nx, ny, npml, dh = 45, 37, 6, 10.0
+    m1, m2 = smooth_model(nx, ny, seed=4)
+    freqs = [2.5, 7.0, 13.0]
+    say("refinement last step, expected wrongly")
+    pl = fdfd.Plan(nx, ny, small_max=16)
+    vals = pl.assemble(G.AC, dh, freqs, dev(m1), dev(m2), npml=npml)
+    F = pl.factor(vals, G.FP32)
+    rng = np.random.default_rng(6)
+    tried = 0
+    for sysno in (0, 2, 0, 2, 0, 2, 0, 2):
+        B = dev(rng.standard_normal((3, 21, nx * ny)) + 1j * rng.standard_normal((3, 21, nx * ny)))
+        w = [F.solve_refine_batch([0, 1, 2], B, sys=sysno, tol=0.0, max_iter=k)[2] for k in range(3)]
+        for z in range(3):
+            for k in (1, 2):
+                promised = w[k - 1][z] ** 2 / (w[k - 2][z] if k > 1 else 1.0)
+                if w[k][z] <= 1.1 * promised or promised < 1e-14:
+                    continue
+                tried += 1
+                tol = np.sqrt(promised * w[k][z])
+                X, its, rr = F.solve_refine_batch([0, 1, 2], B, sys=sysno, tol=tol, max_iter=9)
+                assert its[z] > k and max(rr) <= tol
+                for y in range(3):
+                    res = pl.residual(vals[y], B[y], X[y], sys=sysno)
+                    worst = float((res.norm(dim=1) / B[y].norm(dim=1)).max())
+                    assert abs(worst - rr[y]) <= 1e-3 * worst + 1e-12, (z, k, y)
+    assert tried
+
+
 @pytest.mark.parametrize("precision", [G.FP32, G.FP64])
 @pytest.mark.parametrize("sysno", [0, 1, 2])
 def test_refinement_layouts_agree(precision, sysno):
