@@ -24,6 +24,7 @@
 #include <cstring>
 #include <limits>
 #include <mutex>
+#include <type_traits>
 
 #include "engine.hpp"
 #include "mfma.hpp"
@@ -223,7 +224,7 @@ __global__ void __launch_bounds__(256) k_fwd_gather(const cx<T> *__restrict__ X,
 // sides, a wave WR x WC of them in 16 x 16 blocks.  A tile's products take one
 // compute unit's matrix cores as long as its RT x CT says (128 x 64 x 64 complex
 // in FP64: 13 us), so a launch with fewer tiles than compute units waits on
-// that; panel_tile (below) picks the small shape there.
+// that; with_tile (below) picks the small shape there.
 template <int RT_, int CT_, int WR_, int WC_>
 struct BlkTile {
     static constexpr int RT = RT_, CT = CT_, WR = WR_, WC = WC_;
@@ -416,7 +417,8 @@ __device__ __forceinline__ void diag_product(const cx<T> *D, T *Yr, T *Yi, T *Zr
 // requested before the first barrier, unconditionally (entries outside read a
 // valid address of the front or panel and are masked when staged); that one is
 // loaded during the first column's products.  A front with a single block left
-// takes the first half alone.  LDS: [second Y | first Y | A tile], the A tile's
+// takes the first half alone.  With yonly only the two blocks are solved (one
+// row tile).  LDS: [second Y | first Y | A tile], the A tile's
 // space holding the diagonal blocks and their coupling in turn.
 // grid: (row tiles, fronts, rhs tiles x slots)
 template <typename T, class C>
@@ -424,9 +426,9 @@ constexpr size_t blk2_smem_bytes() {
     return sizeof(T) * 2 * BK * C::CT + blk_smem_bytes<T, C>();
 }
 template <typename T, class C, bool FWD>
-__global__ void __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && C::NT == 512 ? 4 : 1)))
+__global__ void __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(1)))
 k_blk2(const cx<T> *__restrict__ arena, int64_t fstride, const FrontDev *__restrict__ lvF, cx<T> *__restrict__ X, cx<T> *__restrict__ W, int n, int64_t wstride, int nrhs,
-       int rt, int b0, int trans, int cj, Sel sel) {
+       int rt, int b0, int yonly, int trans, int cj, Sel sel) {
     constexpr int RT = C::RT, CT = C::CT, NT = C::NT, AS = kAStride<T, C>;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     BlkSmem<T, C> s(smem_raw + sizeof(T) * 2 * BK * CT);   // the first block's Y and the A tile
@@ -439,7 +441,7 @@ k_blk2(const cx<T> *__restrict__ arena, int64_t fstride, const FrontDev *__restr
     const int nf = FWD || hi == 0 ? lo : hi, ns = hi == 0 ? 0 : FWD ? hi : lo;
     const int row0 = (FWD ? b0 + lo + hi : 0) + blockIdx.x * RT, rowend = FWD ? m : b0;
     if (blockIdx.x > 0 && row0 >= rowend) return;
-    const bool upd = row0 < rowend;
+    const bool upd = !yonly && row0 < rowend;
     const int z = blockIdx.z / rt, r0 = (blockIdx.z - z * rt) * CT, ncol = min(CT, nrhs - r0);
     const cx<T> *G = arena + sel.f[z] * fstride + F.buf_off;
     X += (int64_t)sel.s[z] * n * nrhs;
@@ -623,6 +625,112 @@ __global__ void __launch_bounds__(C::NT) k_bwd_contrib(const cx<T> *__restrict__
     cx<T> y1[C::NA][C::NB][4];
     load_tile<T, C>(X + (int64_t)F.pos0 * nrhs, nrhs, row0, p, r0, y1);
     sub_tile_from<T, C>(w, nrhs, row0, p, r0, y1, acc);
+}
+
+// The update of a large forward launch as a plain product, after a launch of
+// k_blk2 that only solves the block pair at b0 (y to X):
+//   W[b0 + kd : m] -= L[., b0 : b0 + kd] Y,   kd = min(64, p - b0).
+// A 64 x 64 tile is loaded into the accumulators, A (negated) and Y pass through
+// LDS KB columns at a time with the next chunk in flight, and the tile is stored
+// once; three to four workgroups stay resident per compute unit.  Bound by each
+// tile's load-stage-product chain.  In one launch with the solve (128 x 64 tiles,
+// one to two per compute unit) every row tile repeated the diagonal products and
+// waited on them: 1601x401, 4 frequencies x 200 right-hand sides, forward blocks
+// 5.2 -> 3.8 ms FP64, 2.4 -> 2.2 ms FP32 (17 -> 23 and 37 -> 41 TF).  Grouping a
+// row tile's right-hand-side tiles on one XCD is slower (3.9, 2.3 ms).
+// grid: (row tiles, fronts, rhs tiles x slots)
+template <typename T>
+constexpr int kPanelKB = sizeof(T) == 8 ? 16 : 32;
+template <typename T>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k_fwd_update(
+    const cx<T> *__restrict__ arena, int64_t fstride, const FrontDev *__restrict__ lvF,
+    const cx<T> *__restrict__ X, cx<T> *__restrict__ W, int n, int64_t wstride, int nrhs, int rt, int b0, int trans,
+    int cj, Sel sel) {
+    constexpr int KB = kPanelKB<T>, PER = KB * 64 / 256;
+    __shared__ cx<T> As[KB][64 + 1], Bs[KB][64];
+    const FrontDev F = lvF[blockIdx.y];
+    const int m = F.m, kd = min(2 * BK, F.p - b0);
+    const int row0 = b0 + kd + blockIdx.x * 64;
+    if (kd <= 0 || row0 >= m) return;
+    const int z = blockIdx.z / rt, r0 = (blockIdx.z - z * rt) * 64, ncol = min(64, nrhs - r0), nrow = min(64, m - row0);
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wr = (wv >> 1) * 32, wc = (wv & 1) * 32, lr = lane & 15, lk = lane >> 4;
+    // element (row0 + i, b0 + k) of the operator at Ga[i * sr + k * sk]
+    const int sr = trans ? m : 1, sk = trans ? 1 : m;
+    const cx<T> *Ga = arena + sel.f[z] * fstride + F.buf_off + (int64_t)row0 * sr + (int64_t)b0 * sk;
+    const cx<T> *Y = X + ((int64_t)sel.s[z] * n + F.pos0 + b0) * nrhs + r0;
+    W += sel.s[z] * wstride + (F.fv_off + row0) * nrhs + r0;
+    T ax[PER], ay[PER], bx[PER], by[PER];
+    auto load_chunk = [&](int kc) {
+        const int kb = min(KB, kd - kc);
+#pragma unroll
+        for (int u = 0; u < PER; u++) {
+            const int e = tid + 256 * u, i = trans ? e / KB : e & 63, k = trans ? e % KB : e >> 6;
+            const cx<T> v = Ga[k < kb && i < nrow ? (int64_t)i * sr + (int64_t)(kc + k) * sk : 0];
+            ax[u] = v.x;
+            ay[u] = v.y;
+        }
+#pragma unroll
+        for (int u = 0; u < PER; u++) {
+            const cx<T> v = Y[(int64_t)min(kc + wv + 4 * u, kd - 1) * nrhs + (lane < ncol ? lane : 0)];
+            bx[u] = v.x;
+            by[u] = v.y;
+        }
+    };
+    load_chunk(0);
+    typename mfma_t<T>::acc cr[2][2], ci[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int row = wr + a * 16 + mfma_t<T>::row(lk, v), col = wc + b * 16 + lr;
+                const cx<T> c = W[row < nrow && col < ncol ? (int64_t)row * nrhs + col : 0];
+                cr[a][b][v] = c.x;
+                ci[a][b][v] = c.y;
+            }
+    for (int kc = 0; kc < kd; kc += KB) {
+        const int kb = min(KB, kd - kc);
+        if (kc > 0) __syncthreads();   // every wave is done with the previous chunk
+#pragma unroll
+        for (int u = 0; u < PER; u++) {
+            const int e = tid + 256 * u, i = trans ? e / KB : e & 63, k = trans ? e % KB : e >> 6;
+            const bool in = k < kb && i < nrow;
+            As[k][i] = {in ? -ax[u] : T(0), in ? (cj ? ay[u] : -ay[u]) : T(0)};
+        }
+#pragma unroll
+        for (int u = 0; u < PER; u++) {
+            const bool in = wv + 4 * u < kb && lane < ncol;
+            Bs[wv + 4 * u][lane] = {in ? bx[u] : T(0), in ? by[u] : T(0)};
+        }
+        __syncthreads();
+        if (kc + KB < kd) load_chunk(kc + KB);   // in flight during this chunk's products
+        const int kend = (kb + 3) & ~3;
+#pragma unroll 1
+        for (int kk = 0; kk < kend; kk += 4) {
+            const int k = kk + lk;
+            cx<T> av[2], bv[2];
+#pragma unroll
+            for (int a = 0; a < 2; a++) av[a] = As[k][wr + a * 16 + lr];
+#pragma unroll
+            for (int b = 0; b < 2; b++) bv[b] = Bs[k][wc + b * 16 + lr];
+#pragma unroll
+            for (int b = 0; b < 2; b++)
+                if (wc + b * 16 < ncol)
+#pragma unroll
+                    for (int a = 0; a < 2; a++) cmma<T>(av[a].x, av[a].y, bv[b].x, bv[b].y, cr[a][b], ci[a][b]);
+        }
+    }
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int row = wr + a * 16 + mfma_t<T>::row(lk, v), col = wc + b * 16 + lr;
+                if (row < nrow && col < ncol) W[(int64_t)row * nrhs + col] = {cr[a][b][v], ci[a][b][v]};
+            }
 }
 
 // ---- fused per-front substitutions (fronts whose panel fits in LDS) ---------
@@ -2888,17 +2996,26 @@ inline WaveLaunch small_launch(int nfr, int nrhs, int nslots, size_t lds, int ma
 // right-hand sides, 1.37 ms with big tiles only and 1.01 by the rule; 801x201, 4 x
 // 80, 4.69 and 4.33; at 1601x401, 4 x 200, 16-wide tiles up to 1024 big
 // ones cost 5.51 ms of forward blocks against 5.23.
-using TileFwd = BlkTile<128, 64, 32, 32>;
-using TileBwd = BlkTile<64, 64, 32, 32>;
 using TileMid = BlkTile<64, 32, 16, 32>;
 using TileSmall = BlkTile<64, 16, 16, 16>;
-template <class Big, typename Fn>
+// 64 x 64 tiles of a block launch, on which the choice of its shape rests.  Up
+// to one per compute unit (256) the 16-wide tiles, whose chain is shortest; above
+// that 32-wide ones, to any size: 64-wide tiles were no faster for the backward
+// blocks (1601x401, 4 frequencies x 200: FP64 1.27 against 1.15 ms, FP32 0.70 and
+// 0.66) nor for the contribution products (2.59 and 2.51, 1.27 and 1.21).  A
+// forward launch of more than kSplitTiles solves its block pair apart from the
+// update of the rows below (k_fwd_update): never / > 1024 / > 512 tiles, 801x187,
+// 4 x 100 in FP64: 0.69 / 0.61 / 0.58 ms, 1601x401 6.0 / 3.8 / 3.8; FP32, 801x201,
+// 4 x 80: 0.37 / 0.37 / 0.38, 1601x401 2.6 / 2.2 / 2.25.
+template <typename T>
+constexpr int64_t kSplitTiles = sizeof(T) == 8 ? 512 : 1024;
+int64_t panel_tiles(int rows, int nfr, int nrhs, int ns) {
+    return (int64_t)std::max(1, (rows + 63) / 64) * nfr * ((nrhs + 63) / 64) * ns;
+}
+template <typename Fn>
 void with_tile(int rows, int nfr, int nrhs, int ns, Fn &&launch) {
-    const int64_t wgs =
-        (int64_t)std::max(1, (rows + Big::RT - 1) / Big::RT) * nfr * ((nrhs + Big::CT - 1) / Big::CT) * ns;
-    if (wgs <= 256) launch(TileSmall{});
-    else if (wgs <= 512 * (128 / Big::RT)) launch(TileMid{});
-    else launch(Big{});
+    if (panel_tiles(rows, nfr, nrhs, ns) <= 256) launch(TileSmall{});
+    else launch(TileMid{});
 }
 
 #define FUSED_LAUNCH(kern, T, rw, grid, lds, st, ...)                                                   \
@@ -2920,21 +3037,18 @@ void set_smem_attrs() {
                                   hipFuncAttributeMaxDynamicSharedMemorySize, big));
     GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_bwd_vec<T>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, big));
-    auto blk_attrs = [](auto c, bool big) {
+    auto blk_attrs = [](auto c) {
         using C = decltype(c);
         const int b2 = (int)blk2_smem_bytes<T, C>(), bc = (int)blk_smem_bytes<T, C>() + 4 * kContribRowsMax;
         GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_blk2<T, C, true>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, b2));
         GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_blk2<T, C, false>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, b2));
-        if (!big)
-            GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_bwd_contrib<T, C>),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, bc));
+        GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_bwd_contrib<T, C>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, bc));
     };
-    blk_attrs(TileFwd{}, true);
-    blk_attrs(TileBwd{}, false);
-    blk_attrs(TileSmall{}, false);
-    blk_attrs(TileMid{}, false);
+    blk_attrs(TileSmall{});
+    blk_attrs(TileMid{});
     // the refinement step's per-wave column sums: up to 64 KB at 1024 right-hand sides
     GFDFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_ir_step<T>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, kIrWaves * 8 * 1024));
@@ -3001,6 +3115,15 @@ void sweeps(const Factors<T> &F, const Sel &in, int sys, int nrhs, cx<T> *Xp, cx
     const int64_t wstride = pl.fv_rows * (int64_t)nrhs;
     const double nr = nreal, nz = ns, es = sizeof(cx<T>);
     const bool prof = prof_enabled();
+    // the block pair at b0 of a level's fronts: its solve and, unless yonly, the update of up to `rows` rows by it
+    auto blk2 = [&](auto dir, auto t, int b0, int rows, int l, int nfr, int yonly) {
+        using C = decltype(t);
+        const int rt = (nrhs + C::CT - 1) / C::CT, tiles = yonly ? 1 : std::max(1, (rows + C::RT - 1) / C::RT);
+        const size_t lds = blk2_smem_bytes<T, C>();
+        hipLaunchKernelGGL((k_blk2<T, C, decltype(dir)::value>), dim3(tiles, nfr, rt * ns), dim3(C::NT), lds, st,
+                           F.arena, F.fstride, dp.lv_fr[l], Xp, Wp, n, wstride, nrhs, rt, b0, yonly, (int)trans,
+                           (int)cj, in);
+    };
     for (int l = 0; l < pl.nlevels; l++) {
         if (dp.n_all[l] == 0) continue;
         const DevPlan::LevelCounts &c = dp.counts[l];
@@ -3062,14 +3185,15 @@ void sweeps(const Factors<T> &F, const Sel &in, int sys, int nrhs, cx<T> *Xp, cx
             if (prof)
                 for (int q = 0; q < nbk; q++) fe += c.fwd_blk_elems[b0 / BK + q];
             ProfScope ps(K_FWD_BLK, st, nz * 8.0 * nr * fe, nz * (fe + 2.0 * nr * fe / (nbk * BK)) * es);
-            with_tile<TileFwd>(dp.mmax_all[l] - b0, nfr, nrhs, ns, [&](auto t) {
-                using C = decltype(t);
-                const int tiles = std::max(1, (dp.mmax_all[l] - b0 - 1) / C::RT + 1), rt = (nrhs + C::CT - 1) / C::CT;
-                const size_t lds = blk2_smem_bytes<T, C>();
-                hipLaunchKernelGGL((k_blk2<T, C, true>), dim3(tiles, nfr, rt * ns), dim3(C::NT), lds, st, F.arena,
-                                   F.fstride, dp.lv_fr[l], Xp, Wp, n, wstride, nrhs, rt, b0, (int)trans,
-                                   (int)cj, in);
-            });
+            const int rows = dp.mmax_all[l] - b0;
+            if (panel_tiles(rows, nfr, nrhs, ns) > kSplitTiles<T>) {
+                blk2(std::true_type{}, TileMid{}, b0, rows, l, nfr, 1);
+                const int rt = (nrhs + 63) / 64;
+                hipLaunchKernelGGL(k_fwd_update<T>, dim3((rows + 63) / 64, nfr, rt * ns), dim3(256), 0, st, F.arena,
+                                   F.fstride, dp.lv_fr[l], Xp, Wp, n, wstride, nrhs, rt, b0, (int)trans, (int)cj, in);
+            } else {
+                with_tile(rows, nfr, nrhs, ns, [&](auto t) { blk2(std::true_type{}, t, b0, rows, l, nfr, 0); });
+            }
         }
     }
     for (int l = pl.nlevels - 1; l >= 0; l--) {
@@ -3111,7 +3235,7 @@ void sweeps(const Factors<T> &F, const Sel &in, int sys, int nrhs, cx<T> *Xp, cx
             ProfScope ps(K_BWD_CONTRIB, st, nz * 8.0 * nr * c.contrib_elems,
                          nz * (c.contrib_elems + (c.sum_m + c.sum_p) * nr) * es);
             if (dp.mmax_all[l] > kContribRowsMax) throw std::logic_error("front too large for the contribution kernel");
-            with_tile<TileBwd>(pmax, nfr, nrhs, ns, [&](auto t) {
+            with_tile(pmax, nfr, nrhs, ns, [&](auto t) {
                 using C = decltype(t);
                 const int rt = (nrhs + C::CT - 1) / C::CT;
                 const size_t lds = blk_smem_bytes<T, C>() + 4 * (size_t)dp.mmax_all[l];
@@ -3126,13 +3250,7 @@ void sweeps(const Factors<T> &F, const Sel &in, int sys, int nrhs, cx<T> *Xp, cx
             if (prof)
                 for (int q = 0; q < nbk; q++) be += c.bwd_blk_elems[b0 / BK + q];
             ProfScope ps(K_BWD_BLK, st, nz * 8.0 * nr * be, nz * (be + 2.0 * nr * be / (nbk * BK)) * es);
-            with_tile<TileBwd>(b0, nfr, nrhs, ns, [&](auto t) {
-                using C = decltype(t);
-                const int tiles = std::max(1, (b0 + C::RT - 1) / C::RT), rt = (nrhs + C::CT - 1) / C::CT;
-                const size_t lds = blk2_smem_bytes<T, C>();
-                hipLaunchKernelGGL((k_blk2<T, C, false>), dim3(tiles, nfr, rt * ns), dim3(C::NT), lds, st, F.arena, F.fstride, dp.lv_fr[l], Xp, Wp, n,
-                                   wstride, nrhs, rt, b0, (int)trans, (int)cj, in);
-            });
+            with_tile(b0, nfr, nrhs, ns, [&](auto t) { blk2(std::false_type{}, t, b0, b0, l, nfr, 0); });
         }
         if (trans) {
             ProfScope ps(K_PIV_UNSWAP, st, 0.0, nz * 4.0 * c.sum_p * nr * es);

@@ -111,3 +111,15 @@ def test_block_tiles_match_oracle(nf, nrhs, precision, sys):
     for z, c in enumerate(mats):
         Xr, _ = O.band_solve(*c, B[z][cols].T, sys=sys, perm=O.grid_transpose_perm(nx, ny))
         assert rel(X[z][cols], Xr.T) <= (1e-10 if precision == G.FP64 else 1e-8), z
+
+
+# forward launches large enough that the update of the rows below runs apart from the block pairs' solve; 257
+# right-hand sides leave one column in the last tile
+@pytest.mark.parametrize("sys", [0, 1, 2])
+@pytest.mark.parametrize("nf,nrhs,precision", [(9, 257, G.FP64), (18, 257, G.FP32)])
+def test_split_forward_matches_oracle(nf, nrhs, precision, sys):
+    fr = fdfd.Plan(131, 109).fronts()
+    tiles = [-(-int(fr["m"][s].max()) // 64) * int(s.sum()) * -(-nrhs // 64) * nf
+             for s in (fr["level"] == l for l in np.unique(fr["level"])) if fr["p"][s].max() > 32]
+    assert max(tiles) > (512 if precision == G.FP64 else 1024)
+    test_block_tiles_match_oracle(nf, nrhs, precision, sys)
