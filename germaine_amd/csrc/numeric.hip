@@ -3,16 +3,18 @@
 // Fronts are processed level by level (height above the leaves), all fronts
 // of a level and all frequencies of a batch in the same launches:
 //   1. assemble: every entry of a front is written once, as the sum of the
-//      children's Schur complements (pulled through child->parent index maps);
-//   2. the original matrix entries owned by the level are added (each
-//      destination is unique, so no atomics);
-//   3. partial LU of the first p columns with row pivoting restricted to the
+//      children's Schur complements (pulled through child->parent index maps)
+//      and of the original matrix entries the front owns (each has one
+//      destination, so no atomics);
+//   2. partial LU of the first p columns with row pivoting restricted to the
 //      p fully summed rows (the front's structure never changes):
-//      - fronts with m <= small_max: one workgroup, front held in LDS;
+//      - fronts with m <= small_max: one workgroup each, which does step 1 too
+//        and keeps the front in LDS throughout;
 //      - larger fronts: blocked right-looking LU, per panel step a panel
-//        kernel (pivot search, row swaps over the whole front, scaling),
-//        a TRSM of the U row block, and an MFMA trailing update of the
-//        remaining front (which leaves the Schur complement in F22).
+//        kernel (pivot search, scaling, the swaps within the panel), a kernel
+//        that replays the swaps on the other columns and solves the U rows,
+//        and an MFMA trailing update of the remaining front (which leaves the
+//        Schur complement in F22).
 // Factors stay in place in the front arena (L11\U11 and L21 in the first p
 // columns, U12 in the first p rows); the pivot swaps go to piv[pos0 + j].
 #include <algorithm>
