@@ -69,6 +69,13 @@ inline void dev_free(void *p) {
     }
 }
 
+// Workgroup `id` of `total` runs on XCD id % 8, each with an L2 of its own: the
+// item it takes so that every XCD works through one contiguous range of them.
+__device__ __forceinline__ int xcd_range_item(int id, int total) {
+    const int x = id % 8, q = total / 8, r = total % 8;
+    return x * q + min(x, r) + id / 8;
+}
+
 // ---- device complex arithmetic --------------------------------------------
 template <typename T>
 __device__ __forceinline__ cx<T> cmul(cx<T> a, cx<T> b) {

@@ -1379,6 +1379,9 @@ constexpr size_t trsm_lds() {
 // four workgroups per CU: 1601x401, four frequencies, 10.2 ms a factorisation with C
 // and both chunks' operands in registers and LDS (FP64, two per CU), now 9.3; FP32
 // 7.1 and 6.6.
+// Each XCD takes one contiguous range of the tiles (of all frequencies), whose
+// operands it reads into its own L2 once: 403x207, two frequencies 555 -> 530 us
+// FP64, 421 -> 395 FP32; 1601x401, four, 9.27 -> 9.21 ms and 6.55 -> 6.40.
 // 4 waves in 2x2, each wave 32x32 = 2x2 blocks of 16x16.
 // MFMA 16x16x4 operand layout: A lane l -> (row l%16, k l/16), B lane l ->
 // (k l/16, col l%16).  Accumulator register v of lane l holds column l%16 and
@@ -1392,12 +1395,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
                                                      const TileDev *__restrict__ tiles, int k0, int depth, int ccap) {
     constexpr int KB = kGemmKB<T>, PER = KB * 64 / 256;
     __shared__ cx<T> As[KB][64], Bs[64][KB + 1];
-    const TileDev tl = tiles[blockIdx.x];
+    const int item = xcd_range_item(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
+    const int freq = item / gridDim.x;
+    const TileDev tl = tiles[item - freq * gridDim.x];
     const FrontDev F = lvF[tl.front];
     const int m = F.m, kd = min(depth, F.p - k0);
     const int base = k0 + kd, cend = ccap > 0 ? min(k0 + ccap, F.p) : m;
     const int r0 = base + tl.ti * 64, c0 = base + tl.tj * 64;
-    cx<T> *G = arena + blockIdx.y * fstride + F.buf_off;
+    cx<T> *G = arena + freq * fstride + F.buf_off;
     const int tid = threadIdx.x;
     const int lane = tid & 63, w = tid >> 6, wr = (w >> 1) * 32, wc = (w & 1) * 32;
     const int lr = lane & 15, lk = lane >> 4;

@@ -636,23 +636,27 @@ __global__ void __launch_bounds__(C::NT) k_bwd_contrib(const cx<T> *__restrict__
 // tile's load-stage-product chain.  In one launch with the solve (128 x 64 tiles,
 // one to two per compute unit) every row tile repeated the diagonal products and
 // waited on them: 1601x401, 4 frequencies x 200 right-hand sides, forward blocks
-// 5.2 -> 3.8 ms FP64, 2.4 -> 2.2 ms FP32 (17 -> 23 and 37 -> 41 TF).  Grouping a
-// row tile's right-hand-side tiles on one XCD is slower (3.9, 2.3 ms).
-// grid: (row tiles, fronts, rhs tiles x slots)
+// 5.2 -> 3.7 ms FP64, 2.4 -> 2.25 ms FP32.  Its large launches move 4.6 TB/s in
+// FP64; a row tile's right-hand-side tiles stand side by side in one XCD's range,
+// so the operator comes from that L2 after the first: 3.7 -> 3.55 and 2.25 -> 2.18
+// ms.  (Spread with padding, one row tile per XCD, they were slower: 3.9, 2.3.)
+// grid: (rhs tiles x row tiles x fronts x slots), rhs tiles fastest
 template <typename T>
 constexpr int kPanelKB = sizeof(T) == 8 ? 16 : 32;
 template <typename T>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k_fwd_update(
     const cx<T> *__restrict__ arena, int64_t fstride, const FrontDev *__restrict__ lvF,
-    const cx<T> *__restrict__ X, cx<T> *__restrict__ W, int n, int64_t wstride, int nrhs, int rt, int b0, int trans,
-    int cj, Sel sel) {
+    const cx<T> *__restrict__ X, cx<T> *__restrict__ W, int n, int64_t wstride, int nrhs, int tiles, int rt, int nfr,
+    int b0, int trans, int cj, Sel sel) {
     constexpr int KB = kPanelKB<T>, PER = KB * 64 / 256;
     __shared__ cx<T> As[KB][64 + 1], Bs[KB][64];
-    const FrontDev F = lvF[blockIdx.y];
+    const int ncl = rt * tiles, item = xcd_range_item(blockIdx.x, gridDim.x);
+    const int fz = item / ncl, e0 = item - fz * ncl, rowt = e0 / rt, z = fz / nfr;
+    const FrontDev F = lvF[fz - z * nfr];
     const int m = F.m, kd = min(2 * BK, F.p - b0);
-    const int row0 = b0 + kd + blockIdx.x * 64;
+    const int row0 = b0 + kd + rowt * 64;
     if (kd <= 0 || row0 >= m) return;
-    const int z = blockIdx.z / rt, r0 = (blockIdx.z - z * rt) * 64, ncol = min(64, nrhs - r0), nrow = min(64, m - row0);
+    const int r0 = (e0 - rowt * rt) * 64, ncol = min(64, nrhs - r0), nrow = min(64, m - row0);
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = (wv >> 1) * 32, wc = (wv & 1) * 32, lr = lane & 15, lk = lane >> 4;
     // element (row0 + i, b0 + k) of the operator at Ga[i * sr + k * sk]
@@ -3189,8 +3193,9 @@ void sweeps(const Factors<T> &F, const Sel &in, int sys, int nrhs, cx<T> *Xp, cx
             if (panel_tiles(rows, nfr, nrhs, ns) > kSplitTiles<T>) {
                 blk2(std::true_type{}, TileMid{}, b0, rows, l, nfr, 1);
                 const int rt = (nrhs + 63) / 64;
-                hipLaunchKernelGGL(k_fwd_update<T>, dim3((rows + 63) / 64, nfr, rt * ns), dim3(256), 0, st, F.arena,
-                                   F.fstride, dp.lv_fr[l], Xp, Wp, n, wstride, nrhs, rt, b0, (int)trans, (int)cj, in);
+                const int tiles = (rows + 63) / 64;
+                hipLaunchKernelGGL(k_fwd_update<T>, dim3(tiles * nfr * rt * ns), dim3(256), 0, st, F.arena, F.fstride,
+                                   dp.lv_fr[l], Xp, Wp, n, wstride, nrhs, tiles, rt, nfr, b0, (int)trans, (int)cj, in);
             } else {
                 with_tile(rows, nfr, nrhs, ns, [&](auto t) { blk2(std::true_type{}, t, b0, rows, l, nfr, 0); });
             }
