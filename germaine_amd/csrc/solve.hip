@@ -6,10 +6,10 @@
 // move whole rows.  The forward sweep walks the levels upwards: a front's work
 // rows W[f] (m x nrhs) are its own pivot rows of X (row-permuted by the
 // front's pivoting) plus the children's contribution rows, pulled through the
-// child->parent maps.  The pivot rows are then solved in 32-row blocks: each
-// block kernel solves its 32x32 diagonal triangle in LDS and applies the
-// block's columns to every later row of the front as an MFMA product
-// (64 rows x 64 right-hand sides per workgroup); the contribution rows left in
+// child->parent maps.  The pivot rows are then solved in pairs of 32-row
+// blocks: a block kernel solves the pair's inverted diagonal triangles in LDS
+// and applies its columns to every later row of the front as an MFMA product
+// (large launches by a kernel of its own); the contribution rows left in
 // W feed the parent.  The backward sweep walks the levels downwards:
 // z = y1 - U12 x2 as one MFMA product over the ancestors' rows of X, then
 // 32-row blocks from the bottom.  Transposed solves (M^T, M^H) use U^T in the

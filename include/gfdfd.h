@@ -357,10 +357,11 @@ int gfdfd_grad_te_taper(int n, int nshots, const float *omega, const float *omeg
 /* ---- measurement ------------------------------------------------------------
  * Per-kernel-class timing with HIP events on the launch stream, plus the
  * algorithmic flops and HBM bytes of each launch derived from the plan.
- * Classes (one kernel symbol per precision each; piv_unswap two, fwd_front
- * and bwd_front one per tile width): assemble, front_assemble,
- * scatter_orig, small_lu, panel, panel_apply, trsm_u, gemm_update, diag_inv,
- * fwd_gather, fwd_leaf, fwd_small1, fwd_front1, fwd_front, fwd_blk,
+ * Classes (one kernel symbol per precision each; piv_unswap two, panel, the
+ * block and the fused front classes one per tile shape, fwd_blk also its
+ * separate update; scatter_orig is part of the assembly and stays empty):
+ * assemble, front_assemble, scatter_orig, small_lu, panel, panel_apply,
+ * trsm_u, gemm_update, diag_inv, fwd_gather, fwd_leaf, fwd_small1, fwd_front1, fwd_front, fwd_blk,
  * bwd_small1, bwd_front1, bwd_front, bwd_contrib, bwd_blk, piv_unswap,
  * fwd_vec, bwd_vec, permute_in, permute_out, residual, norm_reduce, axpy,
  * subtree.
