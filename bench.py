@@ -108,11 +108,11 @@ def main():
                          "(0: none, -1: as far as LDS allows)")
     ap.add_argument("--refine-layout", type=int, default=0,
                     help="panel refinement layout: 0 elimination order (default), 1 caller's layout")
-    ap.add_argument("--persistent", type=int, default=1,
+    ap.add_argument("--persistent", type=int, default=0,
                     help="small subtrees factored in one persistent launch (1) or level by level (0)")
-    ap.add_argument("--deep-min-m", type=int, default=0,
+    ap.add_argument("--deep-min-m", type=int, default=-1,
                     help="blocked levels with a front of order >= this update the trailing block once per 64 "
-                         "pivots (0: every level; 1073741824: none)")
+                         "pivots (0: every level; 1073741824: none; -1: by the level's size and precision)")
     ap.add_argument("--no-graph", action="store_true",
                     help="refactor with eager launches instead of replaying the captured hipGraph")
     ap.add_argument("--copy-probe", type=int, default=0, metavar="MIB",

@@ -15,7 +15,8 @@ and, in a second stage with the solve switches fixed, the factorisation's schedu
 * ``persistent``: the small subtrees in one persistent launch (1) or level by level (0);
 * ``deep_min_m``: the front-size bucket boundary of the blocked path -- levels whose largest
   blocked front has at least this order factor two 32-column panels per step and update the
-  trailing block once per 64 pivots (product depth 64), smaller ones once per panel (depth 32).
+  trailing block once per 64 pivots (product depth 64), smaller ones once per panel (depth 32);
+  -1 chooses by each level's size and precision.
 
 ``tune`` times a caller-supplied measurement (seconds per step of the real workload for one
 configuration) over the candidates, keeps the fastest and records it in a JSON cache keyed by the
@@ -29,7 +30,7 @@ CACHE = os.environ.get("GFDFD_TUNE_CACHE",
 
 DEFAULT = dict(small_max=64, rw_cap=64, fused_mmax=0, refine_layout=0)
 NO_DEEP = 1 << 30
-FACTOR_DEFAULT = dict(persistent=1, deep_min_m=0)
+FACTOR_DEFAULT = dict(persistent=0, deep_min_m=-1)   # what the library starts with
 
 
 def candidates():
@@ -45,9 +46,11 @@ def candidates():
 
 
 def factor_candidates():
-    """The factorisation schedules (8 configurations): product depth 64 on every blocked level,
-    on levels with fronts of order >= 384 or >= 1024 only, or on none; subtrees persistent or not."""
-    return [dict(persistent=p, deep_min_m=d) for p in (1, 0) for d in (0, 384, 1024, NO_DEEP)]
+    """The factorisation schedules (9 configurations): the library's default, then product depth
+    64 on every blocked level, on levels with fronts of order >= 384 or >= 1024 only, or on none;
+    subtrees persistent or not."""
+    return [dict(FACTOR_DEFAULT)] + [dict(persistent=p, deep_min_m=d) for p in (1, 0)
+                                     for d in (0, 384, 1024, NO_DEEP)]
 
 
 def key(nx, ny, nfreq, nrhs, precision, device):

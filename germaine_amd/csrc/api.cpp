@@ -320,7 +320,7 @@ int gfdfd_release_workspace(void) {
 
 int gfdfd_factor_tuning(int panel_lds_cap, int persistent, int deep_min_m) {
     if (panel_lds_cap < 0) return report(GFDFD_ERR_ARG, "gfdfd_factor_tuning: negative panel LDS cap");
-    if (deep_min_m < 0) return report(GFDFD_ERR_ARG, "gfdfd_factor_tuning: negative deep_min_m");
+    if (deep_min_m < -1) return report(GFDFD_ERR_ARG, "gfdfd_factor_tuning: deep_min_m below -1");
     set_factor_tuning(panel_lds_cap, persistent, deep_min_m);
     return GFDFD_OK;
 }

@@ -153,7 +153,8 @@ void set_solve_tuning(int rw_cap, int fused_mmax, int refine_layout);
 // (0: no cap) take the global-memory panel kernel, as those too tall for
 // registers always do; persistent: the small subtrees in one launch, else level
 // by level; deep_min_m: levels whose largest blocked front has order >=
-// deep_min_m take the two-panel (depth-64) schedule, the others one panel at a time
+// deep_min_m take the two-panel (depth-64) schedule, the others one panel at a
+// time (-1: by the level's size and precision); (0, 0, -1) until it is called
 void set_factor_tuning(int panel_lds_cap, int persistent, int deep_min_m);
 // frees the calling thread's cached solve work buffers
 void release_solve_workspaces();

@@ -1786,16 +1786,18 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
 // ---------------------------------------------------------------------------
 namespace {
 size_t g_panel_lds_cap = 0;   // 0: none
-// Until a caller selects otherwise (g_deep_min_m < 0): the small fronts level by
-// level, and two panels per step only where the trailing update is bound by
-// its passes over memory.  The persistent subtree launch is a serial chain of
-// fronts per workgroup: 61x41, one FP64 frequency, 0.91 ms per factorisation
-// against 0.52 level by level; 1601x401, four frequencies, 43.0 against 42.3.
-// Two panels per step trade a pass over the trailing block for three more
-// launches and a 64-row triangular solve: 270x145 2.46 ms against 2.30, 1601x401
-// (four frequencies) 42.3 against 38.6 in FP64 and 24.7 against 24.4 in FP32;
-// they pay in FP32 from fronts of order 384 once the level's tiles fill the
-// device several times over (1601x401, eight frequencies: 43.2 against 43.9).
+// The default: the small fronts level by level, and (g_deep_min_m < 0) two panels
+// per step only where the trailing update is bound by its passes over memory.
+// The persistent subtree launch is a serial chain of fronts per workgroup:
+// 61x41, one FP64 frequency, 0.91 ms per factorisation against 0.52 level by
+// level; 1601x401, four frequencies, 43.0 against 42.3.  Two panels per step
+// trade a pass over the trailing block for three more launches and a 64-row
+// triangular solve.  Two panels on every level / one / by the rule, ms: FP64
+// 270x145 2.46 / 2.30, 1601x401 with four frequencies 28.6 / 25.2, 2001x2001
+// 145.0 / 141.0; FP32 1601x401 with four 17.6 / 17.4 / 17.1, with eight 30.8 /
+// 31.1 / 30.2, 801x801 with four 20.1 / 20.1 / 19.7, 2401x801 with four 61.5 /
+// 65.6 / 61.6, 2001x2001 72.4 / 75.7 / 71.5: FP32 gains from fronts of order 384
+// once the level's tiles fill the device several times over.
 int g_persistent = 0;    // small subtrees in one persistent launch
 int g_deep_min_m = -1;   // blocked levels with a front of order >= this take the two-panel schedule
 constexpr int kDeepFp32M = 384, kDeepFp32Tiles = 6 * 256;

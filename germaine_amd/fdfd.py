@@ -98,16 +98,18 @@ def solve_tuning(rw_cap=64, fused_mmax=0, refine_layout=0):
 
 
 NO_DEEP = 1 << 30   # deep_min_m that keeps every level on one panel per step
+AUTO_DEEP = -1      # deep_min_m that chooses by the level's size and precision
 
 
-def factor_tuning(panel_lds_cap=0, persistent=1, deep_min_m=0):
+def factor_tuning(panel_lds_cap=0, persistent=0, deep_min_m=AUTO_DEEP):
     """Factorisation kernel selection (process-wide): panels of more than
     panel_lds_cap bytes take the global-memory panel kernel (0: no cap beyond
     what fits in registers); persistent selects the one-launch factorisation of the
     small subtrees (else level by level); levels whose largest blocked front
     has order >= deep_min_m take the two-panel schedule (trailing update once
-    per 64 pivots), the others one panel at a time (NO_DEEP: none).  Until the
-    first call: level by level, and a schedule by the level's size and precision."""
+    per 64 pivots), the others one panel at a time (0: every level, NO_DEEP: none,
+    AUTO_DEEP: by the level's size and precision).  The defaults are what the
+    library starts with; factor_tuning() returns to them."""
     check(lib().gfdfd_factor_tuning(int(panel_lds_cap), int(persistent), int(deep_min_m)), "gfdfd_factor_tuning")
 
 

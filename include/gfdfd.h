@@ -189,9 +189,9 @@ int gfdfd_solve_tuning(int rw_cap, int fused_mmax, int refine_layout);
  * which a workgroup factors one whole subtree of one frequency per task, 0
  * level by level; levels whose largest blocked front has order >= deep_min_m
  * factor two 32-column panels per step and update the trailing block once
- * per 64 pivots (0: every level), the others once per panel.  Until the first
- * call the small fronts go level by level and the schedule follows the
- * level's size and precision.                                               */
+ * per 64 pivots (0: every level), the others once per panel; with deep_min_m
+ * -1 the choice follows the level's size and precision.  The library starts
+ * with (0, 0, -1); a call with these values returns to it.                  */
 int gfdfd_factor_tuning(int panel_lds_cap, int persistent, int deep_min_m);
 
 /* ---- shot kernels --------------------------------------------------------------

@@ -11,3 +11,12 @@ if ROOT not in sys.path:
 def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an MI355X (gfx950) GPU")
     config.addinivalue_line("markers", "slow: takes more than a few seconds on the CPU")
+
+
+@pytest.fixture(autouse=True)
+def default_factor_schedule(request):
+    """GPU tests start from the library's default factorisation schedule, whatever ran before."""
+    if request.node.get_closest_marker("gpu") is not None:
+        from germaine_amd import fdfd
+        fdfd.factor_tuning()
+    yield

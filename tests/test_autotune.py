@@ -35,3 +35,14 @@ def test_all_candidates_failing_falls_back_to_default(tmp_path):
     best, how, table = autotune.tune("k", measure, path=path)
     assert how == "default" and best == autotune.DEFAULT and table == []
     assert autotune.lookup("k", path) is None
+
+
+def test_factor_candidates_start_with_the_library_default():
+    """tune() falls back to the first candidate, and fdfd.factor_tuning's defaults are the same schedule."""
+    import inspect
+
+    from germaine_amd import fdfd
+    cands = autotune.factor_candidates()
+    assert cands[0] == autotune.FACTOR_DEFAULT and cands.count(autotune.FACTOR_DEFAULT) == 1
+    d = inspect.signature(fdfd.factor_tuning).parameters
+    assert dict(persistent=d["persistent"].default, deep_min_m=d["deep_min_m"].default) == autotune.FACTOR_DEFAULT

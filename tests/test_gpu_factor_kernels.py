@@ -123,3 +123,54 @@ def test_split_forward_matches_oracle(nf, nrhs, precision, sys):
              for s in (fr["level"] == l for l in np.unique(fr["level"])) if fr["p"][s].max() > 32]
     assert max(tiles) > (512 if precision == G.FP64 else 1024)
     test_block_tiles_match_oracle(nf, nrhs, precision, sys)
+
+
+# a threshold between the blocked levels' orders: two-panel and one-panel levels in one factorisation
+@pytest.mark.parametrize("precision", [G.FP64, G.FP32])
+def test_mixed_schedule_matches_oracle(precision):
+    nx, ny, deep = 97, 81, 110
+    say("mixed schedule", precision)
+    pl = fdfd.Plan(nx, ny, small_max=16)
+    fr = pl.fronts()
+    top = [fr["m"][fr["level"] == l].max() for l in np.unique(fr["level"]) if fr["p"][fr["level"] == l].max() > 32]
+    assert min(top) < deep <= max(top)
+    m1, m2 = smooth_model(nx, ny, seed=6)
+    fdfd.factor_tuning(0, 0, deep)
+    solve_and_check(pl, nx, ny, [oracle_system(G.AC, nx, ny, 8, 10.0, 6.0, m1, m2)[1], random_grid_csc(nx, ny, 2)],
+                    precision, 1e-8, sys=2)
+
+
+def test_default_schedule_after_other_calls():
+    """factor_tuning() returns to the schedule the library starts with: FP64 levels and FP32 levels of few
+    tiles one panel per step, FP32 levels of at least 1536 tiles with fronts of order >= 384 two.  On 300 x 300
+    a level of order 450 has 221 depth-64 tiles per frequency and the next one 183 at order 451, so eight
+    frequencies lie between the two."""
+    nx, ny = 300, 300
+    say("default schedule")
+    pl = fdfd.Plan(nx, ny)
+    fr = pl.fronts()
+    tiles = []
+    for l in np.unique(fr["level"]):
+        s = fr["level"] == l
+        if fr["m"][s].max() >= 384:
+            tiles.append(int((((fr["m"][s] - np.minimum(64, fr["p"][s]) + 63) // 64) ** 2).sum()))
+    assert min(tiles) * 8 < 1536 < max(tiles) * 8
+    m1, m2 = smooth_model(nx, ny, seed=1)
+    vals = pl.assemble(G.AC, 10.0, [2.0 + 0.7 * k for k in range(8)], dev(m1), dev(m2), npml=10)
+    rng = np.random.default_rng(3)
+    B = dev(rng.standard_normal((5, pl.n)) + 1j * rng.standard_normal((5, pl.n)))
+
+    def solution(v, precision, *tuning):
+        fdfd.factor_tuning(0, 1, 0)
+        fdfd.factor_tuning(*tuning)
+        F = pl.factor(v, precision)
+        rr = F.solve_refine(0, B, tol=1e-12, max_iter=30)[2]
+        assert rr <= 1e-12
+        return F.solve(0, B).cpu().numpy()
+
+    none = (0, 0, fdfd.NO_DEEP)
+    assert np.array_equal(solution(vals[:1], G.FP64), solution(vals[:1], G.FP64, *none))
+    assert np.array_equal(solution(vals[:1], G.FP32), solution(vals[:1], G.FP32, *none))
+    some = solution(vals, G.FP32)
+    assert not np.array_equal(some, solution(vals, G.FP32, *none))
+    assert not np.array_equal(some, solution(vals, G.FP32, 0, 0, 384))
