@@ -530,6 +530,26 @@ template <int N, typename Fn>
 __device__ __forceinline__ void static_for(Fn &&fn) {
     static_for_seq(fn, std::make_integer_sequence<int, N>{});
 }
+// acc += a*b.  The panel kernels sum an entry's terms from zero and subtract the
+// sum once: subtracted one by one every term rounds at the size of the entry,
+// which the terms are far below (with the panels' eliminations done so, FP32
+// factors' solutions 1.2 to 1.3 times further off: 201x101, 3.8e-6 against
+// 2.9e-6, the geometric mean of 12 matrices).
+template <typename T>
+__device__ __forceinline__ void cmadd_to(T &sx, T &sy, cx<T> a, cx<T> b) {
+    sx = fma(-a.y, b.y, fma(a.x, b.x, sx));
+    sy = fma(a.y, b.x, fma(a.x, b.y, sy));
+}
+// c - a*b where a sum cannot be kept, for each step needs the entry: in FP64 the
+// product first, so that only the subtraction rounds at the size of c (61x41,
+// error 2.26e-15 against 2.37e-15, at no cost); in FP32 fused (61x41, error 1.68e-6
+// against 1.53e-6, 201x101, 2.9e-6 and 2.8e-6; the contribution rows alone take
+// 0.4 % of a factorisation of 1601x401 more with the product apart)
+template <typename T>
+__device__ __forceinline__ cx<T> cmsub_step(cx<T> c, cx<T> a, cx<T> b) {
+    if constexpr (sizeof(T) == 8) return csub(c, cmul_f(a, b));
+    else return cmsub_f(c, a, b);
+}
 // wave-wide maximum and minimum by DPP (row shifts, then row broadcasts): six
 // register steps where xor-shuffles take six LDS-crossbar round trips
 template <int CTRL, int ROWS>
@@ -1077,7 +1097,7 @@ __global__ void __launch_bounds__(64 * NW) k_panel_reg(cx<T> *__restrict__ arena
                     ai[jj] = l.y;
                     static_for<8>([&](auto c) {
                         if (c > jj) {
-                            const cx<T> a = cmsub_f(cx<T>{ar[c], ai[c]}, l, s.row[c]);
+                            const cx<T> a = cmsub_step(cx<T>{ar[c], ai[c]}, l, s.row[c]);
                             ar[c] = a.x;
                             ai[c] = a.y;
                         }
@@ -1104,13 +1124,17 @@ __global__ void __launch_bounds__(64 * NW) k_panel_reg(cx<T> *__restrict__ arena
                     ur[t] = Ub[t][tid].x;
                     ui[t] = Ub[t][tid].y;
                 });
-                static_for<7>([&](auto s) {
+                T sr[8], si[8];
+                static_for<8>([&](auto t) { sr[t] = si[t] = T(0); });
+                if constexpr (NW == 16) __builtin_amdgcn_sched_barrier(0);   // (128 registers a thread there)
+                static_for<8>([&](auto s) {
+                    ur[s] -= sr[s];
+                    ui[s] -= si[s];
                     static_for<7 - s>([&](auto d) {
                         constexpr int t = s + 1 + d;
-                        const cx<T> u = cmsub_f(cx<T>{ur[t], ui[t]}, Lb[t][s], cx<T>{ur[s], ui[s]});
-                        ur[t] = u.x;
-                        ui[t] = u.y;
+                        cmadd_to(sr[t], si[t], Lb[t][s], cx<T>{ur[s], ui[s]});
                     });
+                    if constexpr (NW == 16) __builtin_amdgcn_sched_barrier(0);
                 });
                 static_for<8>([&](auto t) { Ub[t][tid] = {ur[t], ui[t]}; });
             }
@@ -1123,13 +1147,12 @@ __global__ void __launch_bounds__(64 * NW) k_panel_reg(cx<T> *__restrict__ arena
                             ai[8 * g + 8 + c] = Ub[t0][8 * g + c].y;
                         });
                     else if (in && t0 >= 8)
-                        static_for<8>([&](auto t) {
-                            static_for<8>([&](auto cc) {
-                                constexpr int c = 8 * g + 8 + cc;
-                                const cx<T> a = cmsub_f(cx<T>{ar[c], ai[c]}, cx<T>{ar[t], ai[t]}, Ub[t][8 * g + cc]);
-                                ar[c] = a.x;
-                                ai[c] = a.y;
-                            });
+                        static_for<8>([&](auto cc) {
+                            constexpr int c = 8 * g + 8 + cc;
+                            T sr = T(0), si = T(0);
+                            static_for<8>([&](auto t) { cmadd_to(sr, si, cx<T>{ar[t], ai[t]}, Ub[t][8 * g + cc]); });
+                            ar[c] -= sr;
+                            ai[c] -= si;
                         });
                 }
             });
@@ -1256,15 +1279,25 @@ __global__ void __launch_bounds__(64) k_panel_finish(cx<T> *__restrict__ arena, 
             });
         }
         if (TRSM && beyond)
-            static_for<31>([&](auto t) {
-                static_for<31 - t>([&](auto d) {
-                    constexpr int i = t + 1 + d;
-                    const cx<T> v = cmsub_f(cx<T>{xr[i], xi[i]}, U[i][t], cx<T>{xr[t], xi[t]});
-                    xr[i] = v.x;
-                    xi[i] = v.y;
+            // eight rows at a time: the terms of the rows above them, then their own
+            static_for<4>([&](auto b) {
+                T sr[8], si[8];
+                static_for<8>([&](auto i) { sr[i] = si[i] = T(0); });
+                static_for<8 * b>([&](auto t) {
+                    static_for<8>([&](auto i) { cmadd_to(sr[i], si[i], U[8 * b + i][t], cx<T>{xr[t], xi[t]}); });
+                    // (keeps the scheduler from hoisting the whole block's LDS reads into registers)
+                    if constexpr (sizeof(T) == 8 ? t % 2 == 1 : t % 4 == 3) __builtin_amdgcn_sched_barrier(0);
                 });
-                // (keeps the scheduler from hoisting the whole block's LDS reads into registers)
-                if constexpr (sizeof(T) == 8 || t % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+                static_for<8>([&](auto i) {
+                    constexpr int t = 8 * b + i;
+                    xr[t] -= sr[i];
+                    xi[t] -= si[i];
+                    static_for<7 - i>([&](auto d) {
+                        constexpr int q = i + 1 + d;
+                        cmadd_to(sr[q], si[q], U[8 * b + q][t], cx<T>{xr[t], xi[t]});
+                    });
+                });
+                __builtin_amdgcn_sched_barrier(0);
             });
         static_for<32>([&](auto t) {
             if (t < kb) col[k0 + t] = {xr[t], xi[t]};
@@ -1281,7 +1314,7 @@ __global__ void __launch_bounds__(64) k_panel_finish(cx<T> *__restrict__ arena, 
             xi[t] = x.y;
             static_for<31 - t>([&](auto d) {
                 constexpr int s = t + 1 + d;
-                const cx<T> v = cmsub_f(cx<T>{xr[s], xi[s]}, x, U[t][s]);
+                const cx<T> v = cmsub_step(cx<T>{xr[s], xi[s]}, x, U[t][s]);
                 xr[s] = v.x;
                 xi[s] = v.y;
             });
@@ -1368,17 +1401,20 @@ constexpr size_t trsm_lds() {
 // 64x64 tiles.  The product's depth is the front's next min(depth, p - k0)
 // pivot columns (depth 32: one panel; 64: two panels), taken KB at a time
 // through the same LDS with the next chunk's loads in flight during a chunk's
-// products, so C is read and written once per `depth` pivots.  C is loaded into
-// the accumulators themselves and A staged negated, which leaves the registers
-// for a tile of C beside them to more waves; the operands are staged as complex
+// products, so C is read and written once per `depth` pivots.  The product is
+// summed from zero and subtracted from C once: accumulated onto C every step
+// rounds at the size of C, which the terms are far below (FP32 factors'
+// solutions 1.2 to 1.5 times further off: 201x101, 3.8e-6 against 5.5e-6, the
+// geometric mean of 12 matrices).  C is loaded under the last chunk's products,
+// when the prefetch registers are free.  The operands are staged as complex
 // entries, A by columns and B by its rows, each with the lanes that write it
 // along the contiguous direction (staging B by columns put 32 lanes on one bank).
 // The updated block starts at row and column k0 + that depth; ccap > 0 ends
 // its columns at min(k0 + ccap, p) (the thin update of the second panel's
-// columns), else at m.  Bound by each tile's load-stage-product chain at three to
-// four workgroups per CU: 1601x401, four frequencies, 10.2 ms a factorisation with C
-// and both chunks' operands in registers and LDS (FP64, two per CU), now 9.3; FP32
-// 7.1 and 6.6.
+// columns), else at m.  Bound by each tile's load-stage-product chain at three
+// workgroups per CU.  A factorisation of 1601x401, four frequencies: 25.3 ms in
+// FP64 and 17.2 in FP32, 25.2 and 17.1 with C in the accumulators; chunks of 32
+// columns in FP32 17.4.
 // Each XCD takes one contiguous range of the tiles (of all frequencies), whose
 // operands it reads into its own L2 once: 403x207, two frequencies 555 -> 530 us
 // FP64, 421 -> 395 FP32; 1601x401, four, 9.27 -> 9.21 ms and 6.55 -> 6.40.
@@ -1388,12 +1424,10 @@ constexpr size_t trsm_lds() {
 // row 4*(l/16)+v for f32, but row 4*v+l/16 for f64.
 // ---------------------------------------------------------------------------
 template <typename T>
-constexpr int kGemmKB = sizeof(T) == 8 ? 16 : 32;
-template <typename T>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k_gemm_update(cx<T> *__restrict__ arena, int64_t fstride,
-                                                     const FrontDev *__restrict__ lvF,
-                                                     const TileDev *__restrict__ tiles, int k0, int depth, int ccap) {
-    constexpr int KB = kGemmKB<T>, PER = KB * 64 / 256;
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+k_gemm_update(cx<T> *__restrict__ arena, int64_t fstride, const FrontDev *__restrict__ lvF,
+              const TileDev *__restrict__ tiles, int k0, int depth, int ccap) {
+    constexpr int KB = 16, PER = KB * 64 / 256;
     __shared__ cx<T> As[KB][64], Bs[64][KB + 1];
     const int item = xcd_range_item(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
     const int freq = item / gridDim.x;
@@ -1433,28 +1467,19 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
         static_for<PER>([&](auto u) {
             const int e = tid + 256 * u, i = e & 63, ka = e >> 6, kb2 = e % KB, j = e / KB;
             const bool ina = ka < kb && r0 + i < m, inb = kb2 < kb && c0 + j < cend;
-            As[ka][i] = {ina ? -ax[u] : T(0), ina ? -ay[u] : T(0)};
+            As[ka][i] = {ina ? ax[u] : T(0), ina ? ay[u] : T(0)};
             Bs[j][kb2] = {inb ? bx[u] : T(0), inb ? by[u] : T(0)};
         });
     };
-    load_chunk(0);
     typename mfma_t<T>::acc cr[2][2], ci[2][2];
 #pragma unroll
     for (int a = 0; a < 2; a++)
 #pragma unroll
-        for (int b = 0; b < 2; b++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int row = r0 + wr + a * 16 + mfma_t<T>::row(lk, v), j = wc + b * 16 + lr;
-                const cx<T> c = at(Gc, row < m && c0 + j < cend ? row + j * m : 0);
-                cr[a][b][v] = c.x;
-                ci[a][b][v] = c.y;
-            }
-    for (int kc = 0; kc < kd; kc += KB) {
-        if (kc > 0) __syncthreads();   // every wave is done with the previous chunk
-        stage_chunk(kc);
-        __syncthreads();
-        if (kc + KB < kd) load_chunk(kc + KB);   // in flight during this chunk's products
+        for (int b = 0; b < 2; b++) {
+            cr[a][b] = typename mfma_t<T>::acc{0, 0, 0, 0};
+            ci[a][b] = cr[a][b];
+        }
+    auto products = [&](int kc) {
         const int kend = (min(KB, kd - kc) + 3) & ~3;
 #pragma unroll 1
         for (int kk = 0; kk < kend; kk += 4) {
@@ -1469,7 +1494,32 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
 #pragma unroll
                 for (int a = 0; a < 2; a++) cmma<T>(av[a].x, av[a].y, bv[b].x, bv[b].y, cr[a][b], ci[a][b]);
         }
+    };
+    load_chunk(0);
+    int kc = 0;
+    for (; kc + KB < kd; kc += KB) {
+        stage_chunk(kc);
+        __syncthreads();
+        load_chunk(kc + KB);   // in flight during this chunk's products
+        products(kc);
+        __syncthreads();   // every wave is done with this chunk
     }
+    stage_chunk(kc);
+    __syncthreads();
+    // the tile of C, in flight during the last chunk's products
+    T gx[2][2][4], gy[2][2][4];
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int row = r0 + wr + a * 16 + mfma_t<T>::row(lk, v), j = wc + b * 16 + lr;
+                const cx<T> c = at(Gc, row < m && c0 + j < cend ? row + j * m : 0);
+                gx[a][b][v] = c.x;
+                gy[a][b][v] = c.y;
+            }
+    products(kc);
     int ms = m;
     asm("" : "+s"(ms));   // (the stores' offsets computed anew rather than kept through the products)
 #pragma unroll
@@ -1480,8 +1530,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
             for (int v = 0; v < 4; v++) {
                 const int row = r0 + wr + a * 16 + mfma_t<T>::row(lk, v), j = wc + b * 16 + lr;
                 if (row < ms && c0 + j < cend)
-                    *reinterpret_cast<cx<T> *>(Gc + (unsigned)(row + j * ms) * (unsigned)sizeof(cx<T>)) = {cr[a][b][v],
-                                                                                                        ci[a][b][v]};
+                    *reinterpret_cast<cx<T> *>(Gc + (unsigned)(row + j * ms) * (unsigned)sizeof(cx<T>)) = {
+                        gx[a][b][v] - cr[a][b][v], gy[a][b][v] - ci[a][b][v]};
             }
 }
 

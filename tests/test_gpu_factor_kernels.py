@@ -174,3 +174,63 @@ def test_default_schedule_after_other_calls():
     some = solution(vals, G.FP32)
     assert not np.array_equal(some, solution(vals, G.FP32, *none))
     assert not np.array_equal(some, solution(vals, G.FP32, 0, 0, 384))
+
+
+def small_terms_system(nx, per_ulp, precision):
+    """(values, c) of a 64 x 2 grid's matrix [[T, a I], [-b I, I]], T the tridiagonal
+    (-1, 2, -1) with a first entry of 1, whose factors are all +-1: the Schur
+    complement is I + c K, K[i, j] = nx - max(i, j), and every entry of it the sum of
+    that many equal terms c = a b of per_ulp units in the last place of 1."""
+    ulp = 2.0 ** (-52 if precision == G.FP64 else -23)
+    a, b = ulp, per_ulp
+    pl = fdfd.Plan(nx, 2, leaf_area=2 * nx, small_max=8)
+    cp, ri = pl.pattern()
+    col = np.repeat(np.arange(pl.n), np.diff(cp))
+    top_r, top_c = ri < nx, col < nx
+    v = np.zeros(pl.nnz, np.complex128)
+    v[top_r & top_c & (ri == col)] = 2.0
+    v[(ri == 0) & (col == 0)] = 1.0
+    v[top_r & top_c & (abs(ri - col) == 1)] = -1.0
+    v[top_r & ~top_c & (col - ri == nx)] = a
+    v[~top_r & top_c & (ri - col == nx)] = -b
+    v[~top_r & ~top_c & (ri == col)] = 1.0
+    return pl, v, a * b
+
+
+
+def small_terms_error(pl, v, c, precision):
+    """Largest error, in units of the last place of 1, of solutions with right-hand
+    sides in the second grid row, where the Schur complement I + c K stands."""
+    F = pl.factor(dev(v[None]), precision)
+    assert F.singular()[0] == 0
+    nx = pl.n // 2
+    rows = [0, 1, 2, 5, 9]
+    B = np.zeros((5, 2 * nx), np.complex128)
+    B[np.arange(5), nx + np.array(rows)] = 1.0
+    X = F.solve(0, dev(B)).cpu().numpy()
+    # (I + c K)^-1 e to second order in c K, whose norm is below 3e-5
+    K = c * (nx - np.maximum(*np.mgrid[0:nx, 0:nx])).astype(np.longdouble)
+    E = B[:, nx:].real.T.astype(np.longdouble)
+    ref = E - K @ E + K @ (K @ E)
+    err = float(np.abs(X[:, nx:] - ref.T).max() * 2.0 ** (52 if precision == G.FP64 else 23))
+    say("  error in units of the last place of 1:", err)
+    return err
+
+
+# the trailing update's terms are summed before they meet the entry they update: 64 terms of 0.12 units in the
+# last place each are lost when they are added to it one by one (or four by four), 7.7 units in all.  Summed
+# first, the entry is rounded once or twice and its inverse once: 3 units at most.  One panel and two per step.
+@pytest.mark.parametrize("deep", [0, fdfd.NO_DEEP])
+@pytest.mark.parametrize("precision", [G.FP64, G.FP32])
+def test_trailing_update_keeps_small_terms(precision, deep):
+    say("trailing update, small terms", precision, deep)
+    fdfd.factor_tuning(0, 0, deep)
+    assert small_terms_error(*small_terms_system(64, 0.12, precision), precision) <= 3.0
+
+
+# the same inside a panel, whose columns are eliminated eight at a time: 16 terms of 0.3 units, lost one by one
+# (4.8 units); summed over the eight columns the entry is rounded twice and its inverse once
+@pytest.mark.parametrize("precision", [G.FP64, G.FP32])
+def test_panel_keeps_small_terms(precision):
+    say("panel, small terms", precision)
+    assert small_terms_error(*small_terms_system(16, 0.3, precision), precision) <= 2.0
