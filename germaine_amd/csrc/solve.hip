@@ -630,12 +630,13 @@ __global__ void __launch_bounds__(C::NT) k_bwd_contrib(const cx<T> *__restrict__
 // The update of a large forward launch as a plain product, after a launch of
 // k_blk2 that only solves the block pair at b0 (y to X):
 //   W[b0 + kd : m] -= L[., b0 : b0 + kd] Y,   kd = min(64, p - b0).
-// A 64 x 64 tile is loaded into the accumulators, A (negated) and Y pass through
-// LDS KB columns at a time with the next chunk in flight, and the tile is stored
-// once; three to four workgroups stay resident per compute unit.  Bound by each
-// tile's load-stage-product chain.  In one launch with the solve (128 x 64 tiles,
-// one to two per compute unit) every row tile repeated the diagonal products and
-// waited on them: 1601x401, 4 frequencies x 200 right-hand sides, forward blocks
+// A and Y pass through LDS KB columns at a time with the next chunk in flight, the
+// product is summed from zero (accumulated onto W every step would round at the
+// size of W's entries) and subtracted once from the 64 x 64 tile of W, which is
+// loaded under the last chunk's products; three to four workgroups stay resident
+// per compute unit.  Bound by each tile's load-stage-product chain.  In one launch
+// with the solve (128 x 64 tiles, one to two per compute unit) every row tile
+// repeated the diagonal products and waited on them: 1601x401, 4 frequencies x 200 right-hand sides, forward blocks
 // 5.2 -> 3.7 ms FP64, 2.4 -> 2.25 ms FP32.  Its large launches move 4.6 TB/s in
 // FP64; a row tile's right-hand-side tiles stand side by side in one XCD's range,
 // so the operator comes from that L2 after the first: 3.7 -> 3.55 and 2.25 -> 2.18
@@ -681,36 +682,30 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
             by[u] = v.y;
         }
     };
-    load_chunk(0);
     typename mfma_t<T>::acc cr[2][2], ci[2][2];
 #pragma unroll
     for (int a = 0; a < 2; a++)
 #pragma unroll
-        for (int b = 0; b < 2; b++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int row = wr + a * 16 + mfma_t<T>::row(lk, v), col = wc + b * 16 + lr;
-                const cx<T> c = W[row < nrow && col < ncol ? (int64_t)row * nrhs + col : 0];
-                cr[a][b][v] = c.x;
-                ci[a][b][v] = c.y;
-            }
-    for (int kc = 0; kc < kd; kc += KB) {
+        for (int b = 0; b < 2; b++) {
+            cr[a][b] = typename mfma_t<T>::acc{0, 0, 0, 0};
+            ci[a][b] = cr[a][b];
+        }
+    auto stage_chunk = [&](int kc) {
         const int kb = min(KB, kd - kc);
-        if (kc > 0) __syncthreads();   // every wave is done with the previous chunk
 #pragma unroll
         for (int u = 0; u < PER; u++) {
             const int e = tid + 256 * u, i = trans ? e / KB : e & 63, k = trans ? e % KB : e >> 6;
             const bool in = k < kb && i < nrow;
-            As[k][i] = {in ? -ax[u] : T(0), in ? (cj ? ay[u] : -ay[u]) : T(0)};
+            As[k][i] = {in ? ax[u] : T(0), in ? (cj ? -ay[u] : ay[u]) : T(0)};
         }
 #pragma unroll
         for (int u = 0; u < PER; u++) {
             const bool in = wv + 4 * u < kb && lane < ncol;
             Bs[wv + 4 * u][lane] = {in ? bx[u] : T(0), in ? by[u] : T(0)};
         }
-        __syncthreads();
-        if (kc + KB < kd) load_chunk(kc + KB);   // in flight during this chunk's products
-        const int kend = (kb + 3) & ~3;
+    };
+    auto products = [&](int kc) {
+        const int kend = (min(KB, kd - kc) + 3) & ~3;
 #pragma unroll 1
         for (int kk = 0; kk < kend; kk += 4) {
             const int k = kk + lk;
@@ -725,7 +720,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
 #pragma unroll
                     for (int a = 0; a < 2; a++) cmma<T>(av[a].x, av[a].y, bv[b].x, bv[b].y, cr[a][b], ci[a][b]);
         }
+    };
+    load_chunk(0);
+    int kc = 0;
+    for (; kc + KB < kd; kc += KB) {
+        stage_chunk(kc);
+        __syncthreads();
+        load_chunk(kc + KB);   // in flight during this chunk's products
+        products(kc);
+        __syncthreads();   // every wave is done with this chunk
     }
+    stage_chunk(kc);
+    __syncthreads();
+    // the tile of W, in flight during the last chunk's products
+    T gx[2][2][4], gy[2][2][4];
 #pragma unroll
     for (int a = 0; a < 2; a++)
 #pragma unroll
@@ -733,7 +741,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const int row = wr + a * 16 + mfma_t<T>::row(lk, v), col = wc + b * 16 + lr;
-                if (row < nrow && col < ncol) W[(int64_t)row * nrhs + col] = {cr[a][b][v], ci[a][b][v]};
+                const cx<T> c = W[row < nrow && col < ncol ? (int64_t)row * nrhs + col : 0];
+                gx[a][b][v] = c.x;
+                gy[a][b][v] = c.y;
+            }
+    products(kc);
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int row = wr + a * 16 + mfma_t<T>::row(lk, v), col = wc + b * 16 + lr;
+                if (row < nrow && col < ncol)
+                    W[(int64_t)row * nrhs + col] = {gx[a][b][v] - cr[a][b][v], gy[a][b][v] - ci[a][b][v]};
             }
 }
 

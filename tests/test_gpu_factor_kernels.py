@@ -234,3 +234,24 @@ def test_trailing_update_keeps_small_terms(precision, deep):
 def test_panel_keeps_small_terms(precision):
     say("panel, small terms", precision)
     assert small_terms_error(*small_terms_system(16, 0.3, precision), precision) <= 2.0
+
+
+# the forward update of the rows below, where it runs apart from the block pairs' solve: 64 terms of 0.12 units in
+# the last place of the entry, lost one by one (7.7 units); summed first the entry is rounded once
+@pytest.mark.parametrize("precision,nrhs", [(G.FP64, 257 * 64 - 3), (G.FP32, 513 * 64 - 3)])
+def test_split_forward_keeps_small_terms(precision, nrhs):
+    nx, bits = 64, 52 if precision == G.FP64 else 23
+    say("split forward, small terms", precision)
+    assert -(-2 * nx // 64) * -(-nrhs // 64) > (512 if precision == G.FP64 else 1024)
+    # [[T, 0], [-I / 4, I]]: L21 is -1/4 on and above the diagonal, y of the first rows 0.48 units throughout
+    pl, v, _ = small_terms_system(nx, 0.25, precision)
+    v[v == 2.0 ** -bits] = 0.0
+    F = pl.factor(dev(v[None]), precision)
+    t = float(np.float32(0.48)) * 2.0 ** -bits
+    B = np.zeros((1, 2 * nx), np.complex128)
+    B[0, 0], B[0, nx:] = t, 1.0
+    X = F.solve(0, dev(B).expand(nrhs, -1).contiguous()).cpu().numpy()
+    ref = 1.0 + 0.25 * np.longdouble(t) * (nx - np.arange(nx))
+    err = float(np.abs(X[:, nx:] - ref).max() * 2.0 ** bits)
+    say("  error in units of the last place of 1:", err)
+    assert err <= 1.0
