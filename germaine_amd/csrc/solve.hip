@@ -420,15 +420,16 @@ __device__ __forceinline__ void diag_product(const cx<T> *D, T *Yr, T *Yi, T *Zr
 // takes the first half alone.  With yonly only the two blocks are solved (one
 // row tile).  LDS: [second Y | first Y | A tile], the A tile's
 // space holding the diagonal blocks and their coupling in turn.
-// grid: (row tiles, fronts, rhs tiles x slots)
+// grid: (row tiles, fronts, rhs tiles x slots from t0 on)
 template <typename T, class C>
 constexpr size_t blk2_smem_bytes() {
     return sizeof(T) * 2 * BK * C::CT + blk_smem_bytes<T, C>();
 }
 template <typename T, class C, bool FWD>
 __global__ void __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(1)))
-k_blk2(const cx<T> *__restrict__ arena, int64_t fstride, const FrontDev *__restrict__ lvF, cx<T> *__restrict__ X, cx<T> *__restrict__ W, int n, int64_t wstride, int nrhs,
-       int rt, int b0, int yonly, int trans, int cj, Sel sel) {
+k_blk2(const cx<T> *__restrict__ arena, int64_t fstride, const FrontDev *__restrict__ lvF, cx<T> *__restrict__ X,
+       cx<T> *__restrict__ W, int n, int64_t wstride, int nrhs, int rt, int t0, int b0, int yonly, int trans, int cj,
+       Sel sel) {
     constexpr int RT = C::RT, CT = C::CT, NT = C::NT, AS = kAStride<T, C>;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     BlkSmem<T, C> s(smem_raw + sizeof(T) * 2 * BK * CT);   // the first block's Y and the A tile
@@ -442,7 +443,7 @@ k_blk2(const cx<T> *__restrict__ arena, int64_t fstride, const FrontDev *__restr
     const int row0 = (FWD ? b0 + lo + hi : 0) + blockIdx.x * RT, rowend = FWD ? m : b0;
     if (blockIdx.x > 0 && row0 >= rowend) return;
     const bool upd = !yonly && row0 < rowend;
-    const int z = blockIdx.z / rt, r0 = (blockIdx.z - z * rt) * CT, ncol = min(CT, nrhs - r0);
+    const int zt = t0 + blockIdx.z, z = zt / rt, r0 = (zt - z * rt) * CT, ncol = min(CT, nrhs - r0);
     const cx<T> *G = arena + sel.f[z] * fstride + F.buf_off;
     X += (int64_t)sel.s[z] * n * nrhs;
     cx<T> *w = W + sel.s[z] * wstride + F.fv_off * nrhs;
@@ -550,13 +551,14 @@ k_blk2(const cx<T> *__restrict__ arena, int64_t fstride, const FrontDev *__restr
 // contribution positions.  The positions are staged in LDS first (after the
 // block tiles, m - p ints), so each 32-column chunk of Uop12 and x2 is one
 // memory round trip, loaded into registers while the previous chunk's products
-// run.  grid: (row tiles over p, fronts, rhs tiles x slots)
+// run.  grid: (row tiles over p, fronts, rhs tiles x slots from t0 on)
 constexpr int kContribRowsMax = 16384;   // m - p of any front on this path
 template <typename T, class C>
 __global__ void __launch_bounds__(C::NT) k_bwd_contrib(const cx<T> *__restrict__ arena, int64_t fstride,
                                                        const FrontDev *__restrict__ lvF, const int *__restrict__ idx,
                                                        const cx<T> *__restrict__ X, cx<T> *__restrict__ W, int n,
-                                                       int64_t wstride, int nrhs, int rt, int trans, int cj, Sel sel) {
+                                                       int64_t wstride, int nrhs, int rt, int t0, int trans, int cj,
+                                                       Sel sel) {
     constexpr int RT = C::RT, CT = C::CT, NT = C::NT, AS = kAStride<T, C>;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     BlkSmem<T, C> s(smem_raw);
@@ -567,7 +569,7 @@ __global__ void __launch_bounds__(C::NT) k_bwd_contrib(const cx<T> *__restrict__
     if (row0 >= p) return;
     for (int e = tid; e < m - p; e += NT) srow[e] = idx[F.idx_off + p + e];
     __syncthreads();
-    const int z = blockIdx.z / rt, r0 = (blockIdx.z - z * rt) * CT, ncol = min(CT, nrhs - r0);
+    const int zt = t0 + blockIdx.z, z = zt / rt, r0 = (zt - z * rt) * CT, ncol = min(CT, nrhs - r0);
     const cx<T> *G = arena + sel.f[z] * fstride + F.buf_off;
     X += (int64_t)sel.s[z] * n * nrhs;
     cx<T> *w = W + sel.s[z] * wstride + F.fv_off * nrhs;
@@ -3037,6 +3039,14 @@ constexpr int64_t kSplitTiles = sizeof(T) == 8 ? 512 : 1024;
 int64_t panel_tiles(int rows, int nfr, int nrhs, int ns) {
     return (int64_t)std::max(1, (rows + 63) / 64) * nfr * ((nrhs + 63) / 64) * ns;
 }
+// fn(t0, count) for the right-hand-side tiles of all slots, at most 65535 per
+// launch (the grid's limit in z, which 32-wide tiles reach at 2.1 million
+// right-hand sides)
+template <typename Fn>
+void for_tiles(int tiles, Fn &&fn) {
+    constexpr int most = 65535;
+    for (int t0 = 0; t0 < tiles; t0 += most) fn(t0, std::min(most, tiles - t0));
+}
 template <typename Fn>
 void with_tile(int rows, int nfr, int nrhs, int ns, Fn &&launch) {
     if (panel_tiles(rows, nfr, nrhs, ns) <= 256) launch(TileSmall{});
@@ -3145,9 +3155,11 @@ void sweeps(const Factors<T> &F, const Sel &in, int sys, int nrhs, cx<T> *Xp, cx
         using C = decltype(t);
         const int rt = (nrhs + C::CT - 1) / C::CT, tiles = yonly ? 1 : std::max(1, (rows + C::RT - 1) / C::RT);
         const size_t lds = blk2_smem_bytes<T, C>();
-        hipLaunchKernelGGL((k_blk2<T, C, decltype(dir)::value>), dim3(tiles, nfr, rt * ns), dim3(C::NT), lds, st,
-                           F.arena, F.fstride, dp.lv_fr[l], Xp, Wp, n, wstride, nrhs, rt, b0, yonly, (int)trans,
-                           (int)cj, in);
+        for_tiles(rt * ns, [&](int t0, int nt) {
+            hipLaunchKernelGGL((k_blk2<T, C, decltype(dir)::value>), dim3(tiles, nfr, nt), dim3(C::NT), lds, st,
+                               F.arena, F.fstride, dp.lv_fr[l], Xp, Wp, n, wstride, nrhs, rt, t0, b0, yonly,
+                               (int)trans, (int)cj, in);
+        });
     };
     for (int l = 0; l < pl.nlevels; l++) {
         if (dp.n_all[l] == 0) continue;
@@ -3265,9 +3277,11 @@ void sweeps(const Factors<T> &F, const Sel &in, int sys, int nrhs, cx<T> *Xp, cx
                 using C = decltype(t);
                 const int rt = (nrhs + C::CT - 1) / C::CT;
                 const size_t lds = blk_smem_bytes<T, C>() + 4 * (size_t)dp.mmax_all[l];
-                hipLaunchKernelGGL((k_bwd_contrib<T, C>), dim3((pmax + C::RT - 1) / C::RT, nfr, rt * ns), dim3(C::NT),
-                                   lds, st, F.arena, F.fstride, dp.lv_fr[l], dp.idx, Xp, Wp, n, wstride, nrhs, rt, (int)trans, (int)cj,
-                                   in);
+                for_tiles(rt * ns, [&](int t0, int nt) {
+                    hipLaunchKernelGGL((k_bwd_contrib<T, C>), dim3((pmax + C::RT - 1) / C::RT, nfr, nt), dim3(C::NT),
+                                       lds, st, F.arena, F.fstride, dp.lv_fr[l], dp.idx, Xp, Wp, n, wstride, nrhs, rt,
+                                       t0, (int)trans, (int)cj, in);
+                });
             });
         }
         for (int b0 = (pmax - 1) / (2 * BK) * (2 * BK); b0 >= 0; b0 -= 2 * BK) {

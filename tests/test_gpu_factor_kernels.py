@@ -255,3 +255,23 @@ def test_split_forward_keeps_small_terms(precision, nrhs):
     err = float(np.abs(X[:, nx:] - ref).max() * 2.0 ** bits)
     say("  error in units of the last place of 1:", err)
     assert err <= 1.0
+
+
+# more right-hand-side tiles than a launch's grid holds in z: 2 x 32769 of 32 columns
+@pytest.mark.parametrize("sys", [0, 2])
+def test_more_tiles_than_one_launch(sys):
+    torch = pytest.importorskip("torch")
+    nx, ny, nrhs = 13, 6, 32 * 32768 + 17
+    say("tiles beyond one launch", sys)
+    pl = fdfd.Plan(nx, ny, leaf_area=36)
+    assert pl.info.max_pivots > 32
+    mats = [random_grid_csc(nx, ny, s) for s in (3, 4)]
+    F = pl.factor(dev(np.stack([c[2] + 1j * c[3] for c in mats])), G.FP64)
+    rng = np.random.default_rng(0)
+    B = rng.standard_normal((2, 7, nx * ny)) + 1j * rng.standard_normal((2, 7, nx * ny))
+    pick = torch.arange(nrhs, device="cuda") % 7
+    X = F.solve_batch([0, 1], dev(B)[:, pick].contiguous(), sys=sys)
+    for z, c in enumerate(mats):
+        Xr, _ = O.band_solve(*c, B[z].T, sys=sys, perm=O.grid_transpose_perm(nx, ny))
+        ref = dev(np.ascontiguousarray(Xr.T))
+        assert float((X[z] - ref[pick]).abs().max()) <= 1e-10 * float(ref.abs().max())
