@@ -17,6 +17,8 @@ def pytest_configure(config):
 def default_factor_schedule(request):
     """GPU tests start from the library's default factorisation schedule, whatever ran before."""
     if request.node.get_closest_marker("gpu") is not None:
+        import torch  # noqa: F401  (its HIP runtime is the process's: loaded before the library)
+
         from germaine_amd import fdfd
         fdfd.factor_tuning()
     yield
