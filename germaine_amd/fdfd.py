@@ -419,8 +419,8 @@ def forward_shots(plan, physics, dh, freqs, m1, m2, ksrc, krec=None, npml=0, a0_
         res += rr
         if krec is not None:
             data += [_sample(X[i], kr) for i in range(len(sel))]
-        if keep_fields:
-            fields += [X[i] for i in range(len(sel))]
+        if keep_fields:          # each frequency's field in storage of its own
+            fields += [X[0]] if len(sel) == 1 else [x.clone() for x in X]
     return dict(data=None if krec is None else data, fields=fields, iters=its, relres=res, factors=F, vals=vals)
 
 

@@ -51,3 +51,16 @@ def test_grouped_frequencies_equal_one_at_a_time(phys, precision, nshots, monkey
     # FP32 factors stop at a 1e-12 residual along different corrections; receiver samples round to float
     for a, b in zip(together, results()):
         assert np.linalg.norm(a - b) <= (2e-7 if a.dtype == np.complex64 else 1e-7) * np.linalg.norm(b)
+
+
+@pytest.mark.gpu
+def test_kept_fields_own_their_storage():
+    """A field kept, dropped or saved by itself is one frequency's panel, not its group's."""
+    torch = pytest.importorskip("torch")
+    nx, ny, npml = 41, 37, 6
+    m1, m2 = (torch.as_tensor(m, device="cuda") for m in smooth_model(nx, ny, seed=4))
+    pl = fdfd.Plan(nx, ny)
+    src = models.acquisition_row(nx, npml, 10.0, 2, 5)
+    fields = fdfd.forward_shots(pl, G.AC, 10.0, [4.0, 7.0, 9.0], m1, m2, src, npml=npml, keep_fields=True)["fields"]
+    assert [tuple(x.shape) for x in fields] == [(5, pl.n)] * 3
+    assert all(x.untyped_storage().nbytes() == 5 * pl.n * 16 for x in fields)
