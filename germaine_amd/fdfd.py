@@ -438,6 +438,7 @@ def hessian_shin(plan, physics, dh, freqs, m1, m2, ksrc, npml=0, a0_pml=90.0, s=
     n = plan.n
     F, _ = _factors(plan, ws, physics, dh, freqs, m1, m2, precision, s=s, npml=npml, a0_pml=a0_pml,
                     free_surf=free_surf)
+    freqs = list(freqs)
     h1 = torch.zeros(n, dtype=torch.float64, device="cuda")
     h2 = torch.zeros(n, dtype=torch.float64, device="cuda")
     amps = [source_amp(physics, fr, s, dh, wavelet) for fr in freqs]
@@ -471,6 +472,7 @@ def hessian_gn(plan, physics, dh, freqs, m1, m2, ksrc, krec, npml=0, a0_pml=90.0
     n = plan.n
     F, _ = _factors(plan, ws, physics, dh, freqs, m1, m2, precision, s=s, npml=npml, a0_pml=a0_pml,
                     free_surf=free_surf)
+    freqs = list(freqs)
     hess = torch.zeros(n, dtype=torch.float64, device="cuda")
     h2 = torch.zeros(n, dtype=torch.float64, device="cuda")
     amps = [source_amp(physics, fr, s, dh, wavelet) for fr in freqs]
@@ -836,6 +838,7 @@ def grad_obj(plan, physics, dh, freqs, m1, m2, ksrc, krec, pobs, npml=0, a0_pml=
     n = plan.n
     F, _ = _factors(plan, ws, physics, dh, freqs, m1, m2, precision, s=s, npml=npml, a0_pml=a0_pml,
                     free_surf=free_surf)
+    freqs = list(freqs)
     tp = None if taper is None else taper.device_struct(len(ksrc))
     g1 = torch.zeros(n, dtype=torch.float64, device="cuda")
     g2 = torch.zeros(n, dtype=torch.float64, device="cuda")

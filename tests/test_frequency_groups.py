@@ -64,3 +64,23 @@ def test_kept_fields_own_their_storage():
     fields = fdfd.forward_shots(pl, G.AC, 10.0, [4.0, 7.0, 9.0], m1, m2, src, npml=npml, keep_fields=True)["fields"]
     assert [tuple(x.shape) for x in fields] == [(5, pl.n)] * 3
     assert all(x.untyped_storage().nbytes() == 5 * pl.n * 16 for x in fields)
+
+
+@pytest.mark.gpu
+def test_frequencies_of_any_sized_iterable():
+    """Frequencies need a length and an order, not an index: a dict's keys, as a list of them."""
+    torch = pytest.importorskip("torch")
+    nx, ny, npml = 41, 37, 6
+    m1, m2 = (torch.as_tensor(m, device="cuda") for m in smooth_model(nx, ny, seed=4))
+    src, rec = models.acquisition_row(nx, npml, 10.0, 2, 5), models.acquisition_row(nx, npml, 10.0, 5, 7)
+    args = (fdfd.Plan(nx, ny), G.AC, 10.0)
+    pobs = [torch.ones((5, 7), dtype=torch.complex64, device="cuda")] * 2
+
+    def results(freqs):
+        fwd = fdfd.forward_shots(*args, freqs, m1, m2, src, rec, npml=npml)["data"]
+        return fwd + [fdfd.hessian_shin(*args, freqs, m1, m2, src, npml=npml),
+                      fdfd.hessian_gn(*args, freqs, m1, m2, src, rec, npml=npml),
+                      fdfd.grad_obj(*args, freqs, m1, m2, src, rec, pobs, npml=npml)[1]]
+
+    for a, b in zip(results([4.0, 7.0]), results({4.0: "a", 7.0: "b"}.keys())):
+        assert torch.equal(a, b)
