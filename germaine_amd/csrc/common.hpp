@@ -50,7 +50,11 @@ template <typename T>
 T *dev_alloc(size_t count) {
     void *p = nullptr;
     if (count == 0) count = 1;
-    GFDFD_HIP(hipMalloc(&p, count * sizeof(T)));
+    const hipError_t e = hipMalloc(&p, count * sizeof(T));
+    if (e != hipSuccess) {
+        (void)hipGetLastError();   // reported here, not by the next call's check of its launches
+        throw hip_error("hipMalloc of " + std::to_string(count * sizeof(T)) + " bytes: " + hipGetErrorString(e), e);
+    }
     mem_track_alloc(p, count * sizeof(T));
     return static_cast<T *>(p);
 }

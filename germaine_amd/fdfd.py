@@ -23,7 +23,7 @@ import ctypes as C
 
 import numpy as np
 
-from . import AC, FP32, FP64, SH, TE, FreqParams, PlanInfo, ShotTaperC, check, lib
+from . import AC, FP32, FP64, SH, TE, FreqParams, GfdfdError, PlanInfo, ShotTaperC, check, lib
 
 
 def _ptr(t):
@@ -349,9 +349,32 @@ _GROUP_ENTRIES = 1 << 27
 
 
 def _groups(nfreq, nrhs, n):
-    """Index lists of the frequencies solved together (at most 64, the library's batch limit)."""
-    g = max(1, min(64, _GROUP_ENTRIES // max(1, nrhs * n)))
-    return [list(range(f, min(f + g, nfreq))) for f in range(0, nfreq, g)]
+    """Index lists of the frequencies solved together (at most 64, the library's batch limit), in
+    as few groups as the limits allow and of even size: four frequencies at a limit of three go 2 + 2."""
+    most = max(1, min(64, _GROUP_ENTRIES // max(1, nrhs * n)))
+    g = -(-nfreq // max(1, -(-nfreq // most)))
+    return [list(range(f, min(f + g, nfreq))) for f in range(0, nfreq, max(1, g))]
+
+
+def _grouped(nfreq, nrhs, n, solve):
+    """(sel, solve(sel)) for the groups of nfreq frequencies in order.  A group that does not fit in
+    device memory (its panels and work buffers take up to some 30 GiB) is solved one frequency at a
+    time; solve returns everything it computes and changes nothing else."""
+    import torch
+    for sel in _groups(nfreq, nrhs, n):
+        try:
+            done = solve(sel)
+        except (GfdfdError, torch.OutOfMemoryError) as e:
+            if len(sel) == 1 or "out of memory" not in str(e):
+                raise
+            done = None
+        if done is not None:
+            yield sel, done
+            continue
+        check(lib().gfdfd_release_workspace(), "gfdfd_release_workspace")
+        torch.cuda.empty_cache()
+        for f in sel:
+            yield [f], solve([f])
 
 
 def _solve_group(F, sel, B, precision, tol, max_iter, sys=0):
@@ -413,8 +436,11 @@ def forward_shots(plan, physics, dh, freqs, m1, m2, ksrc, krec=None, npml=0, a0_
     data, fields, its, res = [], [], [], []
     amps = [source_amp(physics, fr, s, dh, wavelet) for fr in freqs]
     k, kr = _rows(ksrc), None if krec is None else _rows(krec)
-    for sel in _groups(len(freqs), len(k), plan.n):
-        X, it, rr = _solve_group(F, sel, _source_panels(sel, plan.n, k, amps), precision, tol, max_iter)
+
+    def solve(sel):
+        return _solve_group(F, sel, _source_panels(sel, plan.n, k, amps), precision, tol, max_iter)
+
+    for sel, (X, it, rr) in _grouped(len(freqs), len(k), plan.n, solve):
         its += it
         res += rr
         if krec is not None:
@@ -443,8 +469,11 @@ def hessian_shin(plan, physics, dh, freqs, m1, m2, ksrc, npml=0, a0_pml=90.0, s=
     h2 = torch.zeros(n, dtype=torch.float64, device="cuda")
     amps = [source_amp(physics, fr, s, dh, wavelet) for fr in freqs]
     k = _rows(ksrc)
-    for sel in _groups(len(freqs), len(k), n):
-        Us, _, _ = _solve_group(F, sel, _source_panels(sel, n, k, amps), precision, tol, max_iter)
+
+    def solve(sel):
+        return _solve_group(F, sel, _source_panels(sel, n, k, amps), precision, tol, max_iter)[0]
+
+    for sel, Us in _grouped(len(freqs), len(k), n, solve):
         for U, f in zip(Us, sel):
             if physics == AC:
                 o2 = omega2_grad_ac(freqs[f], s)
@@ -478,9 +507,12 @@ def hessian_gn(plan, physics, dh, freqs, m1, m2, ksrc, krec, npml=0, a0_pml=90.0
     amps = [source_amp(physics, fr, s, dh, wavelet) for fr in freqs]
     green = [complex(np.float32(1.0) / np.float32(np.float32(dh) * np.float32(dh)))] * len(freqs)
     k, kr = _rows(ksrc), _rows(krec)
-    for sel in _groups(len(freqs), max(len(k), len(kr)), n):
-        Us, _, _ = _solve_group(F, sel, _source_panels(sel, n, k, amps), precision, tol, max_iter)
-        GRs, _, _ = _solve_group(F, sel, _source_panels(sel, n, kr, green), precision, tol, max_iter)
+
+    def solve(sel):
+        return [_solve_group(F, sel, _source_panels(sel, n, rows, a), precision, tol, max_iter)[0]
+                for rows, a in ((k, amps), (kr, green))]
+
+    for sel, (Us, GRs) in _grouped(len(freqs), max(len(k), len(kr)), n, solve):
         for U, GR, f in zip(Us, GRs, sel):
             if physics == AC:
                 o2 = omega2_grad_ac(freqs[f], s)
@@ -545,12 +577,15 @@ def objective(plan, physics, dh, freqs, m1, m2, ksrc, krec, pobs, npml=0, a0_pml
     l2 = []
     amps = [source_amp(physics, fr, s, dh, wavelet) for fr in freqs]
     k, kr = _rows(ksrc), _rows(krec)
-    for sel in _groups(len(freqs), len(k), n):
+
+    def solve(sel):
         B = _source_panels(sel, n, k, amps)
         Us, _, _ = _solve_group(F, sel, B, precision, tol, max_iter)
-        for i, f in enumerate(sel):
-            l2s, _ = _residual_sources(kr, _sample(Us[i], kr), pobs[f], dh, misfit, stf_inv, False, B[i])
-            l2.append(l2s.sum())
+        return [_residual_sources(kr, _sample(Us[i], kr), pobs[f], dh, misfit, stf_inv, False, B[i])[0].sum()
+                for i, f in enumerate(sel)]
+
+    for _, l2s in _grouped(len(freqs), len(k), n, solve):
+        l2 += l2s
     return 0.5 * sum(float(v) for v in l2)
 
 
@@ -850,15 +885,19 @@ def grad_obj(plan, physics, dh, freqs, m1, m2, ksrc, krec, pobs, npml=0, a0_pml=
     k, kr = _rows(ksrc), _rows(krec)
     nshots = len(k)
     tpp = None if tp is None else C.byref(tp)
-    for sel in _groups(len(freqs), nshots, n):
+
+    def solve(sel):
         B = _source_panels(sel, n, k, amps)
         Us, _, _ = _solve_group(F, sel, B, precision, tol, max_iter)
-        stfs = []
+        l2s, stfs = [], []
         for i, f in enumerate(sel):              # the adjoint panels take the sources' place
-            l2s, stf = _residual_sources(kr, _sample(Us[i], kr), pobs[f], dh, misfit, stf_inv, rtm, B[i])
-            l2.append(l2s.sum())
+            v, stf = _residual_sources(kr, _sample(Us[i], kr), pobs[f], dh, misfit, stf_inv, rtm, B[i])
+            l2s.append(v.sum())
             stfs.append(stf)
-        LAMs, _, _ = _solve_group(F, sel, B, precision, tol, max_iter, sys=adj_sys)
+        return Us, _solve_group(F, sel, B, precision, tol, max_iter, sys=adj_sys)[0], l2s, stfs
+
+    for sel, (Us, LAMs, l2s, stfs) in _grouped(len(freqs), nshots, n, solve):
+        l2 += l2s
         for i, f in enumerate(sel):
             U, LAM, stf = Us[i], LAMs[i], stfs[i]
             if physics == AC:

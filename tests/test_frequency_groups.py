@@ -84,3 +84,55 @@ def test_frequencies_of_any_sized_iterable():
 
     for a, b in zip(results([4.0, 7.0]), results({4.0: "a", 7.0: "b"}.keys())):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["library", "torch"])
+def test_group_beyond_memory_goes_one_at_a_time(kind, monkeypatch):
+    """A group whose second panel solve runs out of memory gives what its frequencies give one by one; other
+    errors, and one frequency's own, are the caller's."""
+    torch = pytest.importorskip("torch")
+    nx, ny, npml = 41, 37, 6
+    m1, m2 = (torch.as_tensor(m, device="cuda") for m in smooth_model(nx, ny, seed=4))
+    src, rec = models.acquisition_row(nx, npml, 10.0, 2, 5), models.acquisition_row(nx, npml, 10.0, 5, 7)
+    args = (fdfd.Plan(nx, ny), G.AC, 10.0, [4.0, 7.0, 9.0], m1, m2, src, rec)
+    pobs = [torch.ones((5, 7), dtype=torch.complex64, device="cuda")] * 3
+
+    def results():
+        fwd = fdfd.forward_shots(*args, npml=npml)
+        l2, grad = fdfd.grad_obj(*args, pobs, npml=npml)
+        return fwd["data"] + [fdfd.hessian_gn(*args, npml=npml), grad], [l2, fdfd.objective(*args, pobs, npml=npml)]
+
+    monkeypatch.setattr(fdfd, "_GROUP_ENTRIES", 1)
+    ref = results()
+    monkeypatch.undo()
+    solve, calls = fdfd.Factors.solve_refine_batch, []
+
+    def limited(self, freqs, *a, **kw):
+        calls.append(len(freqs))
+        if len(freqs) > 1 and len(calls) % 2 == 0:
+            raise (G.GfdfdError("hipMalloc of 1 bytes: out of memory") if kind == "library" else
+                   torch.OutOfMemoryError("HIP out of memory."))
+        return solve(self, freqs, *a, **kw)
+
+    monkeypatch.setattr(fdfd.Factors, "solve_refine_batch", limited)
+    got = results()
+    assert max(calls) == 3 and 1 in calls
+    assert got[1] == ref[1] and all(torch.equal(a, b) for a, b in zip(got[0], ref[0]))
+
+    def failing(self, freqs, *a, **kw):
+        raise G.GfdfdError("out of memory" if len(freqs) == 1 else "singular")
+
+    monkeypatch.setattr(fdfd.Factors, "solve_refine_batch", failing)
+    with pytest.raises(G.GfdfdError, match="singular"):
+        fdfd.forward_shots(*args, npml=npml)
+    monkeypatch.setattr(fdfd, "_GROUP_ENTRIES", 1)
+    with pytest.raises(G.GfdfdError, match="out of memory"):
+        fdfd.forward_shots(*args, npml=npml)
+
+
+def test_groups_are_even():
+    n = fdfd._GROUP_ENTRIES // 3
+    assert [len(g) for g in fdfd._groups(4, 1, n)] == [2, 2]
+    assert [len(g) for g in fdfd._groups(7, 1, n)] == [3, 3, 1]
+    assert fdfd._groups(0, 1, n) == []
