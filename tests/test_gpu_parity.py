@@ -258,6 +258,28 @@ def test_refinement_last_step(precision, tol, max_iter):
         assert rel(out[0][0], out[1][0]) <= 1e-9
 
 
+# at the step limit with residuals well above FP64 rounding: after the first solve about 1e-6 of b and after one
+# correction about 1e-11, where recomputing it leaves 1e-15, 1e-4 of it
+@pytest.mark.parametrize("max_iter", [0, 1])
+@pytest.mark.parametrize("sysno", [0, 1, 2])
+def test_refinement_step_limit_reports_its_residual(sysno, max_iter):
+    nx, ny, npml, dh = 45, 37, 6, 10.0
+    m1, m2 = smooth_model(nx, ny, seed=4)
+    say("refinement at the step limit", sysno, max_iter)
+    pl = fdfd.Plan(nx, ny, small_max=16)
+    vals = pl.assemble(G.AC, dh, [2.5, 7.0, 13.0], dev(m1), dev(m2), npml=npml)
+    F = pl.factor(vals, G.FP32)
+    rng = np.random.default_rng(8)
+    B = dev(rng.standard_normal((3, 21, nx * ny)) + 1j * rng.standard_normal((3, 21, nx * ny)))
+    X, its, rr = F.solve_refine_batch([0, 1, 2], B, sys=sysno, tol=1e-18, max_iter=max_iter)
+    assert its == [max_iter] * 3
+    for z in range(3):
+        res = pl.residual(vals[z], B[z], X[z], sys=sysno)
+        worst = float((res.norm(dim=1) / B[z].norm(dim=1)).max())
+        say("  ", z, worst, rr[z])
+        assert worst > 1e-13 and abs(worst - rr[z]) <= 1e-2 * worst
+
+
 def test_refinement_last_step_expected_wrongly():
     """A tolerance between what the residual's shrinking promises and what the
     step delivers: the step runs again for the residual it did not write, and the
