@@ -120,7 +120,8 @@ void DevPlan::build_small(const Plan &pl, std::vector<FrontDev> &fd) {
     large_cptr = dev_upload(cptr);
     large_oq = dev_upload(lq);
     large_ooff = dev_upload(loff);
-    bytes += (2 * first.size() + ooff.size() + cptr.size() + loff.size()) * 4 + (optr.size() + oq.size() + lq.size()) * 8;
+    bytes += (2 * first.size() + ooff.size() + cptr.size() + loff.size()) * 4 +
+             (optr.size() + oq.size() + lq.size()) * 8;
     for (int l = 0; l < pl.nlevels; l++) {
         const LevelPlan &L = pl.levels[l];
         // the level's small fronts outside the subtrees
@@ -1009,7 +1010,7 @@ __global__ void __launch_bounds__(256) k_panel(cx<T> *__restrict__ arena, int64_
 // by eight registers, so the code stays short enough for the instruction
 // cache.  k_panel_finish applies the panel's permutation to the front's other
 // columns.  Bound by the 32-step chain: a panel in LDS with three barriers per
-// column took 48 us (270x145, one FP64 frequency, event-timed), this 28; the 69
+// column took 48 us (270x145, one FP64 frequency, event-timed), this 27; the 69
 // panels of 1601x401, four frequencies, 8.5 ms (those above 318 rows in global
 // memory) and 2.9.
 // ---------------------------------------------------------------------------
@@ -1194,9 +1195,9 @@ constexpr int kPanelRows = sizeof(T) == 8 ? 512 : 1024;
 // once every lane holds its sources.  The other chunks: 64 contribution rows,
 // x U_kk = a.  Replaces 32 dependent swaps in memory and a triangular
 // solve with a shuffle reduction per row in a launch of its own: 345 + 325 us
-// against 511 per factorisation of 270x145 (FP64, 22 panels), 1.48 + 1.70 ms
-// against 2.41 in FP32 at 1601x401, four frequencies.  Bound by the dependent
-// rows at two to three waves per SIMD (registers).
+// against 343 per factorisation of 270x145 (FP64, 22 panels; 386 with the U12 rows'
+// terms subtracted one by one).  Bound by the dependent rows at two waves per SIMD
+// in FP64 and four in FP32 (registers).
 template <typename T, bool TRSM>
 __global__ void __launch_bounds__(64) k_panel_finish(cx<T> *__restrict__ arena, int64_t fstride,
                                                      const FrontDev *__restrict__ lvF, const int *__restrict__ piv,
@@ -1412,9 +1413,9 @@ constexpr size_t trsm_lds() {
 // The updated block starts at row and column k0 + that depth; ccap > 0 ends
 // its columns at min(k0 + ccap, p) (the thin update of the second panel's
 // columns), else at m.  Bound by each tile's load-stage-product chain at three
-// workgroups per CU.  A factorisation of 1601x401, four frequencies: 25.3 ms in
-// FP64 and 17.2 in FP32, 25.2 and 17.1 with C in the accumulators; chunks of 32
-// columns in FP32 17.4.
+// workgroups per CU.  Its share of a factorisation of 1601x401, four frequencies:
+// 9.35 ms in FP64 (31 TF/s) and 5.35 in FP32, 9.21 and 5.21 with C in the
+// accumulators.  Chunks of 32 columns in FP32: 17.4 ms a factorisation against 17.2.
 // Each XCD takes one contiguous range of the tiles (of all frequencies), whose
 // operands it reads into its own L2 once: 403x207, two frequencies 555 -> 530 us
 // FP64, 421 -> 395 FP32; 1601x401, four, 9.27 -> 9.21 ms and 6.55 -> 6.40.
@@ -1443,7 +1444,9 @@ k_gemm_update(cx<T> *__restrict__ arena, int64_t fstride, const FrontDev *__rest
     // addresses: a uniform base per operand and 32-bit byte offsets within 64 columns of it
     const char *Ga = reinterpret_cast<const char *>(G + (int64_t)k0 * m + r0);   // column k of A at k m
     char *Gc = reinterpret_cast<char *>(G + (int64_t)c0 * m);                    // column j of B and C at j m
-    auto at = [](const char *base, int e) { return *reinterpret_cast<const cx<T> *>(base + (unsigned)e * (unsigned)sizeof(cx<T>)); };
+    auto at = [](const char *base, int e) {
+        return *reinterpret_cast<const cx<T> *>(base + (unsigned)e * (unsigned)sizeof(cx<T>));
+    };
     // a chunk's operands, loaded unconditionally (entries outside read the
     // operand's first and are zeroed when staged) so that they stay in flight
     T ax[PER], ay[PER], bx[PER], by[PER];
@@ -1745,9 +1748,9 @@ __device__ __forceinline__ void u12_mfma(const cx<T> (*V)[33], const cx<double> 
 }
 
 template <typename T>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k_diag_inv(cx<T> *__restrict__ arena, int64_t fstride,
-                                                  const FrontDev *__restrict__ fronts,
-                                                  const int *__restrict__ lv_single) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+k_diag_inv(cx<T> *__restrict__ arena, int64_t fstride, const FrontDev *__restrict__ fronts,
+           const int *__restrict__ lv_single) {
     __shared__ cx<T> D[32][33];   // the block being inverted, then the rectangles' chunks
     __shared__ cx<double> LI[32][33], UI[32][33];
     const FrontDev F = fronts[blockIdx.x];
@@ -1948,9 +1951,9 @@ void factor_numeric(const DevPlan &dp, Factors<T> &F, const cx<double> *vals, in
                     {
                         ProfScope ps(K_PANEL, st, flops * nf, 0.0);
                         const dim3 g(dp.n_large[l], nf);
-#define PANEL(NW) \
-    hipLaunchKernelGGL((k_panel_reg<T, NW>), g, dim3(64 * NW), 0, st, F.arena, F.fstride, lvL, F.piv, F.rowperm, pl.n, k0, \
-                       pl.nb, F.sing)
+#define PANEL(NW)                                                                                                   \
+    hipLaunchKernelGGL((k_panel_reg<T, NW>), g, dim3(64 * NW), 0, st, F.arena, F.fstride, lvL, F.piv, F.rowperm,     \
+                       pl.n, k0, pl.nb, F.sing)
                         if (rows <= 64) PANEL(1);
                         else if (rows <= 128) PANEL(2);
                         else if (rows <= 256) PANEL(4);

@@ -222,8 +222,8 @@ __global__ void __launch_bounds__(256) k_fwd_gather(const cx<T> *__restrict__ X,
 // ---- panel substitutions on MFMA -------------------------------------------
 // Tile shapes of the block kernels: a workgroup covers RT rows x CT right-hand
 // sides, a wave WR x WC of them in 16 x 16 blocks.  A tile's products take one
-// compute unit's matrix cores as long as its RT x CT says (128 x 64 x 64 complex
-// in FP64: 13 us), so a launch with fewer tiles than compute units waits on
+// compute unit's matrix cores as long as its RT x CT says (64 x 32 x 64 complex
+// in FP64: 3 us), so a launch with fewer tiles than compute units waits on
 // that; with_tile (below) picks the small shape there.
 template <int RT_, int CT_, int WR_, int WC_>
 struct BlkTile {
@@ -638,11 +638,13 @@ __global__ void __launch_bounds__(C::NT) k_bwd_contrib(const cx<T> *__restrict__
 // loaded under the last chunk's products; three to four workgroups stay resident
 // per compute unit.  Bound by each tile's load-stage-product chain.  In one launch
 // with the solve (128 x 64 tiles, one to two per compute unit) every row tile
-// repeated the diagonal products and waited on them: 1601x401, 4 frequencies x 200 right-hand sides, forward blocks
-// 5.2 -> 3.7 ms FP64, 2.4 -> 2.25 ms FP32.  Its large launches move 4.6 TB/s in
-// FP64; a row tile's right-hand-side tiles stand side by side in one XCD's range,
-// so the operator comes from that L2 after the first: 3.7 -> 3.55 and 2.25 -> 2.18
-// ms.  (Spread with padding, one row tile per XCD, they were slower: 3.9, 2.3.)
+// repeated the diagonal products and waited on them: 1601x401, 4 frequencies x 200
+// right-hand sides, forward blocks 5.2 -> 3.7 ms FP64, 2.4 -> 2.25 ms FP32.  A row
+// tile's right-hand-side tiles stand side by side in one XCD's range, so the
+// operator comes from that L2 after the first (119 -> 63 GB fetched by the launches
+// of seven FP64 passes at 8 frequencies): 3.7 -> 3.55 and 2.25 -> 2.18 ms, 3.55 and
+// 2.10 with the terms summed first.  (Spread with padding, one row tile per XCD,
+// they were slower: 3.9, 2.3.)
 // grid: (rhs tiles x row tiles x fronts x slots), rhs tiles fastest
 template <typename T>
 constexpr int kPanelKB = sizeof(T) == 8 ? 16 : 32;
@@ -2633,13 +2635,11 @@ static_assert(kIrStage <= kIrCoef0 && kIrCoef0 + 9 * kIrPts <= kIrThreads,
 constexpr int kIrPer = (kIrStage * kIrCw + kIrThreads - 1) / kIrThreads;   // staging entries per thread
 
 template <typename T>
-__global__ void __launch_bounds__(kIrThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 4))) k_ir_step(const cx<double> *__restrict__ vals, const int *__restrict__ colptr,
-                                                 const int *__restrict__ rowind, const int64_t *__restrict__ tq,
-                                                 const int *__restrict__ iperm, int nx, int ny, int nrhs, int ld64,
-                                                 int ld, int sys, int64_t nnz, const cx<double> *__restrict__ Bu,
-                                                 cx<double> *Rg, const cx<T> *__restrict__ D,
-                                                 cx<T> *__restrict__ R, uint64_t last, double *__restrict__ partial,
-                                                 Sel sel) {
+__global__ void __launch_bounds__(kIrThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 4)))
+k_ir_step(const cx<double> *__restrict__ vals, const int *__restrict__ colptr, const int *__restrict__ rowind,
+          const int64_t *__restrict__ tq, const int *__restrict__ iperm, int nx, int ny, int nrhs, int ld64, int ld,
+          int sys, int64_t nnz, const cx<double> *__restrict__ Bu, cx<double> *Rg, const cx<T> *__restrict__ D,
+          cx<T> *__restrict__ R, uint64_t last, double *__restrict__ partial, Sel sel) {
     extern __shared__ double wsum[];   // [kIrWaves][nrhs]
     __shared__ cx<T> sx[kIrStage][kIrCw];
     __shared__ cx<double> scoef[kIrPts][9];
@@ -3014,20 +3014,17 @@ inline WaveLaunch small_launch(int nfr, int nrhs, int nslots, size_t lds, int ma
     return {dim3(((nfr + 7) / 8) * 8 * rtg, nslots), dim3(64 * wpg), (lds + 15) & ~size_t(15), rtg, 0};
 }
 
-// Tile shapes of the block kernels and the rule between them.  A big tile reads
-// each operator entry once per 64 right-hand sides but holds one compute unit
-// for its whole product; when the big tiles would not fill the 256 compute
-// units the launch lasts as long as one of them, so the work goes out in tiles
-// of 16 right-hand sides, and of 32 while they would fill the units less than
-// twice (128-row tiles).  One FP64 solve pass: 403x207, 2 frequencies x 31
-// right-hand sides, 1.37 ms with big tiles only and 1.01 by the rule; 801x201, 4 x
-// 80, 4.69 and 4.33; at 1601x401, 4 x 200, 16-wide tiles up to 1024 big
-// ones cost 5.51 ms of forward blocks against 5.23.
+// Tile shapes of the block kernels: a wider tile reads each operator entry once
+// for more right-hand sides but holds one compute unit for its whole product.
 using TileMid = BlkTile<64, 32, 16, 32>;
 using TileSmall = BlkTile<64, 16, 16, 16>;
 // 64 x 64 tiles of a block launch, on which the choice of its shape rests.  Up
 // to one per compute unit (256) the 16-wide tiles, whose chain is shortest; above
-// that 32-wide ones, to any size: 64-wide tiles were no faster for the backward
+// that 32-wide ones.  A solve pass with 16-wide tiles only / 32-wide only / by the
+// rule, M in FP64: 403x207, 2 frequencies x 31 right-hand sides, 1.00 / 1.09 / 1.00
+// ms, 801x201, 4 x 80, 4.28 / 4.30 / 4.25, 1601x401, 4 x 200, 36.2 / 35.7 / 35.7;
+// FP32 0.71 / 0.77 / 0.71, 2.54 / 2.56 / 2.52 and 21.6 / 21.4 / 21.3.  32-wide
+// tiles serve launches of any size: 64-wide ones were no faster for the backward
 // blocks (1601x401, 4 frequencies x 200: FP64 1.27 against 1.15 ms, FP32 0.70 and
 // 0.66) nor for the contribution products (2.59 and 2.51, 1.27 and 1.21).  A
 // forward launch of more than kSplitTiles solves its block pair apart from the
@@ -3758,7 +3755,8 @@ std::vector<RefineStats> refine_panels(const Factors<T> &F, const std::vector<in
             // done with it; the stencil values and indices
             const int nw = sl.n - __builtin_popcountll(lm);
             const double panel = (double)n * nr * (16.0 + es);
-            ProfScope ps(K_RESIDUAL, st, sl.n * (8.0 * nnz * nr + 2.0 * n * nr), (sl.n + nw) * panel + sl.n * nnz * 28.0);
+            ProfScope ps(K_RESIDUAL, st, sl.n * (8.0 * nnz * nr + 2.0 * n * nr),
+                         (sl.n + nw) * panel + sl.n * nnz * 28.0);
             hipLaunchKernelGGL(k_ir_step<T>, dim3(nblk, sl.n), dim3(kIrThreads), kIrWaves * sizeof(double) * nrhs, st,
                                F.vals, dp.colptr, dp.rowind, dp.tq, dp.iperm, pl.nx, pl.ny, nrhs, ld64, ld, sys,
                                pl.nnz, it == 0 ? B : nullptr, Rg, dbuf(it % kIrBufs), dbuf(jn), lm, partial, sl);

@@ -90,8 +90,8 @@ def test_wide_register_panels_residual(nx, ny, precision):
     assert np.max(np.linalg.norm(R, axis=1) / np.linalg.norm(B.cpu().numpy(), axis=1)) <= 1e-11
 
 
-# panel sweeps of the multi-block levels at each tile width (16, 32 and 64 right-hand sides per workgroup, by
-# how many tiles a launch has): one column past a tile, several frequencies, single last blocks
+# panel sweeps of the multi-block levels at each tile width (16 and 32 right-hand sides per workgroup, by how
+# many tiles a launch has): one column past a tile, several frequencies, single last blocks
 @pytest.mark.parametrize("sys", [0, 1, 2])
 @pytest.mark.parametrize("nf,nrhs,precision", [(1, 17, G.FP64), (3, 33, G.FP64), (8, 129, G.FP64), (3, 65, G.FP32)])
 def test_block_tiles_match_oracle(nf, nrhs, precision, sys):

@@ -471,8 +471,8 @@ def test_two_panel_schedule_matches_oracle(precision, matrix):
 @pytest.mark.parametrize("precision", [G.FP64, G.FP32])
 def test_global_memory_panel_path_matches_oracle(precision, matrix):
     """The blocked path's global-memory panel kernel, which factors panels too
-    large for LDS (separators above 318 rows in FP64, 637 in FP32): forced on
-    every blocked panel of a small grid by a one-byte LDS cap, against the
+    tall for registers (above 512 rows in FP64, 1024 in FP32): forced on every
+    blocked panel of a small grid by a one-byte cap, against the
     banded oracle for M and M^T -- on the assembled Helmholtz matrix and on
     random values whose partial pivoting swaps rows."""
     nx, ny = 45, 33
