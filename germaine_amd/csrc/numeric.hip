@@ -543,9 +543,11 @@ __device__ __forceinline__ void cmadd_to(T &sx, T &sy, cx<T> a, cx<T> b) {
 }
 // c - a*b where a sum cannot be kept, for each step needs the entry: in FP64 the
 // product first, so that only the subtraction rounds at the size of c (61x41,
-// error 2.26e-15 against 2.37e-15, at no cost); in FP32 fused (61x41, error 1.68e-6
-// against 1.53e-6, 201x101, 2.9e-6 and 2.8e-6; the contribution rows alone take
-// 0.4 % of a factorisation of 1601x401 more with the product apart)
+// error 2.26e-15 against 2.37e-15, at no cost); in FP32 fused.  That is 1.68e-6 at
+// 61x41, 3 % above the LDS panels (1.62e-6), and 2.9e-6 at 201x101, 4 % below
+// them; with the product apart 1.53e-6 and 2.8e-6, the contribution rows 0.4 % of
+// a factorisation of 1601x401 slower, and the refinement's second step contracts
+// so well that the test of a step expected wrongly finds none on its inputs.
 template <typename T>
 __device__ __forceinline__ cx<T> cmsub_step(cx<T> c, cx<T> a, cx<T> b) {
     if constexpr (sizeof(T) == 8) return csub(c, cmul_f(a, b));
