@@ -1848,11 +1848,12 @@ size_t g_panel_lds_cap = 0;   // 0: none
 // level; 1601x401, four frequencies, 43.0 against 42.3.  Two panels per step
 // trade a pass over the trailing block for three more launches and a 64-row
 // triangular solve.  Two panels on every level / one / by the rule, ms: FP64
-// 270x145 2.46 / 2.30, 1601x401 with four frequencies 28.6 / 25.2, 2001x2001
-// 145.0 / 141.0; FP32 1601x401 with four 17.6 / 17.4 / 17.1, with eight 30.8 /
-// 31.1 / 30.2, 801x801 with four 20.1 / 20.1 / 19.7, 2401x801 with four 61.5 /
-// 65.6 / 61.6, 2001x2001 72.4 / 75.7 / 71.5: FP32 gains from fronts of order 384
-// once the level's tiles fill the device several times over.
+// 270x145 1.67 / 1.32 / 1.31, 1601x401 with four frequencies 28.5 / 25.1 / 25.1,
+// 2001x2001 143.5 / 144.2 / 144.2, 3001x3001 407 / 423 / 423; FP32 1601x401 with
+// four 17.8 / 17.3 / 17.1, with eight 31.2 / 31.4 / 30.5, 801x801 with four 20.2 /
+// 20.0 / 19.7, 2401x801 with four 62.1 / 66.3 / 62.4, 2001x2001 72.9 / 75.7 / 71.9.
+// FP32 gains from fronts of order 384 once the level's tiles fill the device
+// several times over; FP64 only on grids of millions of points.
 int g_persistent = 0;    // small subtrees in one persistent launch
 int g_deep_min_m = -1;   // blocked levels with a front of order >= this take the two-panel schedule
 constexpr int kDeepFp32M = 384, kDeepFp32Tiles = 6 * 256;
